@@ -163,7 +163,6 @@ Launch make_launch(const mxopt_ctx* ctx, const mxopt_table* t, const Group& g, b
   L.stream = ctx->stream;
   L.nontemporal = ctx->nontemporal;
   L.pipelined_norm = ctx->pipelined_norm;
-  L.any_unaligned = g.any_unaligned;
   L.partial_chunks = g.elems * 10 < (uint64_t)g.nchunks * kChunkElems * 9;
   return L;
 }
@@ -254,11 +253,9 @@ static int run_update(mxopt_ctx* ctx, const mxopt_table* t, const char* op, F&& 
   return MXOPT_OK;
 }
 
-void fill_dev_tensor(const mxopt_tensor& s, DevTensor& d) {
-  d.p = s.p; d.p_out = s.p_out; d.g = s.g; d.g_out = s.g_out; d.m = s.m; d.v = s.v;
-  d.n = s.n; d.bc1 = s.bc1; d.bc2 = s.bc2;
-  d.flags = s.flags & ~kTfUnaligned;
-  // Smallest number of leading elements after which every stream is 16-byte aligned.
+// Smallest number of leading elements after which every stream of the tensor is 16-byte aligned; kMaxHead + 1 when
+// there is none.
+static uint32_t common_head(const mxopt_tensor& s) {
   const void* ptrs[6] = {s.p, s.p_out, s.g, s.g_out, s.m, s.v};
   const int sizes[6] = {dtype_size(s.p_dtype), dtype_size(s.p_out_dtype), dtype_size(s.g_dtype),
                         dtype_size(s.g_out_dtype), 4, 4};
@@ -269,11 +266,20 @@ void fill_dev_tensor(const mxopt_tensor& s, DevTensor& d) {
       if (ptrs[k] && ((reinterpret_cast<uintptr_t>(ptrs[k]) + (uintptr_t)head * sizes[k]) & 15u)) ok = false;
     if (ok) break;
   }
-  if (head > kMaxHead) {  // the streams disagree: per-element path for the whole tensor
+  return head;
+}
+
+void fill_dev_tensor(const mxopt_tensor& s, DevTensor& d) {
+  d.p = s.p; d.p_out = s.p_out; d.g = s.g; d.g_out = s.g_out; d.m = s.m; d.v = s.v;
+  d.n = s.n; d.bc1 = s.bc1; d.bc2 = s.bc2;
+  d.flags = s.flags & ~kTfUnaligned;
+  const uint32_t head = common_head(s);
+  if (head > kMaxHead) {  // the streams disagree: 16-byte accesses at whatever phase each stream has
     d.flags |= kTfUnaligned;
-    head = 0;
+    d.head = 0;
+  } else {
+    d.head = (uint32_t)std::min<uint64_t>(head, s.n);
   }
-  d.head = head;
 }
 
 uint64_t chunks_of(const DevTensor& d) {
@@ -291,7 +297,6 @@ Launch make_single_launch(const mxopt_ctx* ctx, const mxopt_tensor& t, bool pers
   L.stream = ctx->stream;
   L.nontemporal = ctx->nontemporal;
   L.pipelined_norm = ctx->pipelined_norm;
-  L.any_unaligned = (L.one.flags & kTfUnaligned) != 0;
   L.partial_chunks = L.one.n * 10 < (uint64_t)L.nchunks * kChunkElems * 9;
   return L;
 }
@@ -491,7 +496,6 @@ int mxopt_table_build(mxopt_ctx* ctx, const mxopt_tensor* tensors, size_t n, mxo
     g.pd = (kv.first >> 24) & 0xff; g.gd = (kv.first >> 16) & 0xff; g.pod = (kv.first >> 8) & 0xff; g.god = kv.first & 0xff;
     g.chunk_begin = (uint32_t)chunks.size();
     for (uint32_t ti : kv.second) {
-      g.any_unaligned = g.any_unaligned || (t->dev[ti].flags & kTfUnaligned) != 0;
       g.elems += t->dev[ti].n;
       const uint64_t nc = chunks_of(t->dev[ti]);
       for (uint64_t c = 0; c < nc; ++c) chunks.push_back(DevChunk{ti, (uint32_t)c});
@@ -624,7 +628,7 @@ int mxopt_table_set_pending(mxopt_table* t, int k, const void* const* streams, i
       const DevTensor& d = t->dev[i];
       if (d.flags & kTfUnaligned) {
         if (reinterpret_cast<uintptr_t>(ptr) % esize) return fail(ctx, MXOPT_ERR_INVALID_ARG, where + " is not element-aligned");
-      } else if ((reinterpret_cast<uintptr_t>(ptr) + (uintptr_t)d.head * esize) & 15u) {
+      } else if ((reinterpret_cast<uintptr_t>(ptr) + (uintptr_t)common_head(t->host[i]) * esize) & 15u) {
         return fail(ctx, MXOPT_ERR_INVALID_ARG, where + " does not share the 16-byte phase of the tensor's other buffers");
       }
     }
@@ -678,8 +682,9 @@ int mxopt_tensor_layout(const mxopt_tensor* t, uint32_t* head, int* vector_path,
   if (!t) return fail(nullptr, MXOPT_ERR_INVALID_ARG, "mxopt_tensor_layout: null tensor");
   DevTensor d;
   fill_dev_tensor(*t, d);
-  if (head) *head = d.head;
-  if (vector_path) *vector_path = (d.flags & kTfUnaligned) ? 0 : 1;
+  const uint32_t h = common_head(*t);
+  if (head) *head = h > kMaxHead ? 0 : h;
+  if (vector_path) *vector_path = h > kMaxHead ? 0 : 1;
   if (num_chunks) *num_chunks = chunks_of(d);
   return MXOPT_OK;
 }

@@ -15,7 +15,7 @@ namespace mxopt {
 
 constexpr int kChunkElems = MXOPT_CHUNK_ELEMS;
 constexpr uint32_t kTfFirst = MXOPT_TF_FIRST;
-constexpr uint32_t kTfUnaligned = 0x80000000u;  // set by the table builder: element-wise path
+constexpr uint32_t kTfUnaligned = 0x80000000u;  // set by the table builder: no head aligns every stream
 constexpr uint32_t kMaxHead = 7;                // a shifted tensor peels at most this many elements
 
 // One per tensor, in device memory.
@@ -69,7 +69,6 @@ struct StreamScales {
 struct Group {
   int pd, gd, pod, god;
   uint32_t chunk_begin, nchunks;
-  bool any_unaligned = false;  // some tensor of the group takes the element-wise path
   uint64_t elems = 0;          // elements of the group's tensors (chunks * kChunkElems when every chunk is full)
 };
 

@@ -92,8 +92,8 @@ __global__ __launch_bounds__(kThreads) void update_kernel(const DevTensor* __res
         if (use_v) store_group<MXOPT_F32, E, NT>(V, off, v[j]);
       }
     } else {
-      // Last chunk of a tensor, or a tensor whose buffers are not 16-byte aligned.
-      const uint32_t ngroups = (flags & kTfUnaligned) ? 0u : len / E;
+      // Last chunk of a tensor.
+      const uint32_t ngroups = len / E;
       for (uint32_t q = tid; q < ngroups; q += kThreads) {
         const uint64_t off = start + (uint64_t)q * E;
         float p[E], g[E], g2[E], m[E], v[E];
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(kThreads) void transform_kernel(const DevTensor* __
         store_group<OD, E, NT && ADD>(GO, start + (uint64_t)(j * kThreads + tid) * E, g[j]);  // streaming only where the line was read
       }
     } else {
-      const uint32_t ngroups = (cv.t.flags & kTfUnaligned) ? 0u : cv.len / E;
+      const uint32_t ngroups = cv.len / E;
       for (uint32_t q = tid; q < ngroups; q += kThreads) {
         float g[E], a[E];
         load_group<GD, E, false>(G, start + (uint64_t)q * E, g);

@@ -137,7 +137,7 @@ struct ChunkView {
   uint32_t len;    // elements in this chunk (kChunk except for the last one)
   uint32_t head;   // chunk 0 of a shifted tensor: elements [0, head) are this workgroup's too
   uint32_t tensor; // row of the table (0 for a single tensor passed by value)
-  bool fast;       // full chunk of a 16-byte aligned (after the head) tensor: 128-bit path, fully unrolled
+  bool fast;       // full chunk: fully unrolled
 };
 
 __device__ __forceinline__ ChunkView locate(const DevTensor* __restrict__ T, const DevChunk* __restrict__ C,
@@ -154,11 +154,16 @@ __device__ __forceinline__ ChunkView locate(const DevTensor* __restrict__ T, con
     cv.tensor = 0;
     index = c;
   }
+  // The same for the whole workgroup, so it stays in scalar registers: the builder has cut `head` to n, and the number
+  // of full chunks fits 32 bits (its limit on n), which leaves no 64-bit compare (there is no scalar one).  Chunks of
+  // 10,000 tensors of 2,461 elements: AdamW over four micro-batches 161 -> 143 us, its norm 62 -> 53.
+  static_assert(kChunk == 4096, "shift and mask below");
+  const uint64_t body = cv.t.n - cv.t.head;
+  const uint32_t full = (uint32_t)(body >> 12);
   cv.start = (uint64_t)cv.t.head + (uint64_t)index * kChunk;
-  const uint64_t left = cv.t.n > cv.start ? cv.t.n - cv.start : 0;
-  cv.len = left < (uint64_t)kChunk ? (uint32_t)left : (uint32_t)kChunk;
-  cv.head = index == 0 ? (cv.t.n < (uint64_t)cv.t.head ? (uint32_t)cv.t.n : cv.t.head) : 0u;
-  cv.fast = !(cv.t.flags & kTfUnaligned) && cv.len == (uint32_t)kChunk;
+  cv.fast = index < full;
+  cv.len = cv.fast ? (uint32_t)kChunk : index == full ? (uint32_t)body & (uint32_t)(kChunk - 1) : 0u;
+  cv.head = index == 0 ? cv.t.head : 0u;
   return cv;
 }
 

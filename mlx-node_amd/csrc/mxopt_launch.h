@@ -21,7 +21,6 @@ struct Launch {
   hipStream_t stream = nullptr;
   int nontemporal = 1;               // non-zero: streaming-hint loads and stores
   int pipelined_norm = 2;            // plain 16-bit norms take the software-pipelined kernel
-  bool any_unaligned = false;        // some tensor of the launch takes the element-wise path
   bool partial_chunks = false;       // the chunks are under 90 % full on average (many small tensors)
   // Deferred accumulation (the *_list launchers): stream j of table row r is pending[j * ntensors + r].
   const void* const* pending = nullptr;

@@ -177,7 +177,7 @@ __global__ __launch_bounds__(kThreads) void update_list_kernel(const DevTensor* 
         if (use_v) store_group<MXOPT_F32, E, kListNT>(V, off, v[j]);
       }
     } else {
-      const uint32_t ngroups = (flags & kTfUnaligned) ? 0u : len / E;
+      const uint32_t ngroups = len / E;
       for (uint32_t q = tid; q < ngroups; q += kThreads) {
         const uint64_t off = start + (uint64_t)q * E;
         float p[E], g[E], x[KMAX][E], m[E], v[E];

@@ -77,7 +77,7 @@ __global__ __launch_bounds__(kThreads) void sumsq_list_kernel(const DevTensor* _
         }
       }
     } else {
-      const uint32_t ngroups = (cv.t.flags & kTfUnaligned) ? 0u : cv.len / E;
+      const uint32_t ngroups = cv.len / E;
       for (uint32_t q = tid; q < ngroups; q += kThreads) {
         const uint64_t off = cv.start + (uint64_t)q * E;
         float g[E], x[E];

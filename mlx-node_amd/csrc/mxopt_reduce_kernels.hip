@@ -135,7 +135,7 @@ struct SumsqChunk {
     }
   }
 
-  // Partial or unaligned chunk.
+  // Partial chunk.
   static __device__ __forceinline__ float slow(const ChunkView& cv, const PrepRegs& pr, uint32_t tid, bool first) {
     const void* X = squared_stream(cv);
     const void* G = cv.t.g;
@@ -143,7 +143,7 @@ struct SumsqChunk {
     float s32 = 0.0f;
     const bool clamped = (pr.flags & kPrepClampPre) != 0;
     bool bad = false;
-    const uint32_t ngroups = (cv.t.flags & kTfUnaligned) ? 0u : cv.len / E;
+    const uint32_t ngroups = cv.len / E;
     for (uint32_t q = tid; q < ngroups; q += kThreads) {
       const uint64_t off = cv.start + (uint64_t)q * E;
       float x[E], g[E];
@@ -218,9 +218,9 @@ __global__ __launch_bounds__(kThreads) void sumsq_kernel(const DevTensor* __rest
       // instead of two widenings and two multiply-adds; with twice the elements per byte the widening path
       // is bound by instruction issue (6.3 against 6.8 TB/s).  The norm is held to 1e-5, not bitwise; NaN
       // and Inf propagate into the partial sum as before.
-      const MXOPT_GLOBAL u32x4* q =
-          global_ptr<u32x4>((const void*)((const uint16_t*)Chunk::squared_stream(cv) + cv.start)) + tid;
-      u32x4 r[2];
+      const MXOPT_GLOBAL u32x4_mem* q =
+          global_ptr<u32x4_mem>((const void*)((const uint16_t*)Chunk::squared_stream(cv) + cv.start)) + tid;
+      u32x4_mem r[2];
 #pragma unroll
       for (int j = 0; j < 2; ++j) r[j] = NT ? __builtin_nontemporal_load(q + j * kThreads) : q[j * kThreads];
       s = 0.0f;
@@ -278,8 +278,7 @@ __global__ __launch_bounds__(kThreads) void sumsq_kernel(const DevTensor* __rest
 // compiler waits for all of them at the top of every trip.)
 //   per lane and chunk: two 16-byte pieces of the chunk's full 8-element groups and one single element (lanes
 //   0-6: the up to 7 elements behind the last full group; lanes 8-14: the up to 7 elements in front of a
-//   shifted tensor's first chunk).  A table with a tensor whose streams disagree about alignment (element-wise
-//   path) is not launched here.
+//   shifted tensor's first chunk).
 // WHICH: 0 squares tensor.g, 1 tensor.g_out.
 // ------------------------------------------------------------------------------------
 template <int AD, int WHICH, bool NT, int NCH>
@@ -297,7 +296,7 @@ __global__ __launch_bounds__(kThreads) void sumsq16_multi_kernel(const DevTensor
   double acc_sum = 0.0;
 
   struct InFlight {
-    u32x4 r[2];
+    u32x4_mem r[2];
     uint32_t single;  // one 16-bit element, or 0
   };
   // Starts the loads of one chunk.  `live` false: every lane reads the safe address.
@@ -311,7 +310,7 @@ __global__ __launch_bounds__(kThreads) void sumsq16_multi_kernel(const DevTensor
     for (int j = 0; j < 2; ++j) {
       const uint32_t q = tid + (uint32_t)j * kThreads;
       const void* a = q < ng ? (const void*)(X + cv.start + (uint64_t)q * 8u) : safe;
-      const MXOPT_GLOBAL u32x4* gp = global_ptr<u32x4>(a);
+      const MXOPT_GLOBAL u32x4_mem* gp = global_ptr<u32x4_mem>(a);
       f.r[j] = NT ? __builtin_nontemporal_load(gp) : *gp;
     }
     const bool tail_lane = tid < rem, head_lane = tid >= 8u && tid - 8u < head;
@@ -356,9 +355,8 @@ __global__ __launch_bounds__(kThreads) void sumsq16_multi_kernel(const DevTensor
   auto fetch = [&](uint32_t c0, ChunkView (&v)[NCH], bool (&l)[NCH]) {
 #pragma unroll
     for (int k = 0; k < NCH; ++k) {
-      const uint64_t ck = (uint64_t)c0 + (uint64_t)k * stride;
-      l[k] = ck < nchunks;
-      v[k] = locate(T, C, one, l[k] ? (uint32_t)ck : blockIdx.x);  // a dead slot re-reads the first descriptor
+      l[k] = (uint32_t)k * stride < nchunks - c0;  // c0 < nchunks; a 32-bit compare stays scalar
+      v[k] = locate(T, C, one, l[k] ? c0 + (uint32_t)k * stride : blockIdx.x);  // a dead slot re-reads the first descriptor
     }
   };
   uint32_t c = blockIdx.x;
@@ -369,12 +367,12 @@ __global__ __launch_bounds__(kThreads) void sumsq16_multi_kernel(const DevTensor
     InFlight f[NCH];
 #pragma unroll
     for (int k = 0; k < NCH; ++k) f[k] = issue(cv[k], live[k]);
-    const uint64_t next = (uint64_t)c + (uint64_t)NCH * stride;
-    if (next < nchunks) fetch((uint32_t)next, ahead, live_ahead);  // scalar loads: they do not wait for the data
+    const bool more = (uint32_t)NCH * stride < nchunks - c;
+    if (more) fetch(c + (uint32_t)NCH * stride, ahead, live_ahead);  // scalar loads: they do not wait for the data
 #pragma unroll
     for (int k = 0; k < NCH; ++k) acc_sum += (double)consume(cv[k], live[k], f[k]);
-    if (next >= nchunks) break;
-    c = (uint32_t)next;
+    if (!more) break;
+    c += (uint32_t)NCH * stride;
   }
   unsigned long long unused = 0;
   block_sum(acc_sum, unused);
@@ -481,7 +479,7 @@ bool launch_sumsq(int mode, int ad, int gd, const Launch& L, const DevPrep& prep
   // 10,000 tensors of 64 ... 65,536 elements: 45.9 against 53.1 us; on the Qwen3-1.7B list, whose chunks are
   // full, the general kernel is the leaner one (0.581 against 0.593 ms).
   const bool wanted = L.pipelined_norm == 1 || (L.pipelined_norm > 1 && L.partial_chunks);
-  if (mode < 2 && partial_sum != nullptr && prep.flags == 0 && wanted && !L.any_unaligned) {
+  if (mode < 2 && partial_sum != nullptr && prep.flags == 0 && wanted) {
     if (ad == MXOPT_BF16) {
       if (L.pipelined_norm >= 4) launch_sumsq16_multi<MXOPT_BF16, 4>(mode, L, prep, partial_sum);
       else launch_sumsq16_multi<MXOPT_BF16, 2>(mode, L, prep, partial_sum);

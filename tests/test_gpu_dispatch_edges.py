@@ -1,0 +1,73 @@
+"""GPU: sizes and layouts at the edges of the kernels' variants, against the oracle."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+import mxopt_oracle as O
+from gpu_util import assert_bit_equal, to_dev, to_host
+
+F = np.float32
+CHUNK = 4096
+
+
+@pytest.fixture(scope="module")
+def mx():
+    import torch
+    import mxopt
+    assert torch.cuda.is_available()
+    return mxopt
+
+
+@pytest.fixture(scope="module")
+def ctx(mx):
+    c = mx.Context()
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("chunks", [1, 2, 255, 256, 257, 2047, 2048, 2049, 4096, 4097, 8 * 4096 + 8, 8 * 16384 + 3])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_norm_second_pass_at_the_edges_of_its_variants(mx, ctx, chunks, dtype):
+    """One partial sum per workgroup: 1 to 16,384 of them, at and beside the counts where the second pass changes
+    shape.  Every element is 2^-6, so the sum of squares is exact whatever the order of the additions."""
+    import torch
+    n = (chunks - 1) * CHUNK + 5
+    g = torch.full((n,), 2.0 ** -6, dtype=torch.float32 if dtype == "f32" else torch.bfloat16, device="cuda")
+    res = ctx.norm_result()
+    ctx.global_norm(ctx.table([mx.TensorSpec(g=g)]), res, max_norm=1.0)
+    r = ctx.read_norm_result(res)
+    assert r.sumsq == n * 2.0 ** -12 and r.nonfinite == 0
+    _, scale = O.norm_scale_c1(n * 2.0 ** -12, 1.0)
+    assert O.ulp_diff_f32(np.array([r.scale], F), np.array([scale], F))[0] <= 1
+
+
+@pytest.mark.parametrize("g_off,out_off", [(1, 0), (0, 1), (3, 2), (7, 4)])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_streams_of_different_16_byte_phases(mx, ctx, g_off, out_off, dtype):
+    """Gradient and output (float32) start g_off / out_off elements into their allocations: norm, transform and
+    accumulation over every remainder of a group and of a chunk, and nothing outside the views is written."""
+    import torch
+    sizes = [1, 3, 4, 7, 8, 9, 255 * 8 + 1, CHUNK - 1, CHUNK, CHUNK + 1, 2 * CHUNK + 17]
+    rng = np.random.default_rng(7)
+    gs = [rng.normal(0, 1e-2, n).astype(F) for n in sizes]
+    if dtype == "bf16":
+        gs = [O.f32_to_bf16(g) for g in gs]
+    dg = [to_dev(g, g_off) for g in gs]
+    slabs = [torch.full((n + 40,), 9.0, device="cuda") for n in sizes]
+    outs = [s[16 + out_off:16 + out_off + n] for s, n in zip(slabs, sizes)]
+    table = ctx.table([mx.TensorSpec(g=g, g_out=o) for g, o in zip(dg, outs)])
+    res = ctx.norm_result()
+    ctx.global_norm(table, res, max_norm=0.5)
+    r = ctx.read_norm_result(res)
+    exact = O.exact_sumsq(gs)
+    assert abs(r.sumsq - exact) <= 1e-6 * exact
+    ctx.grad_transform(table, mx.make_prep(scale=res))
+    want = [O.as_f32(g) * F(r.scale) for g in gs]
+    for i, w in enumerate(want):
+        assert_bit_equal(to_host(outs[i]), w, f"transform {i}")
+    ctx.accumulate(table, first=False)
+    for i, w in enumerate(want):
+        assert_bit_equal(to_host(outs[i]), w + O.as_f32(gs[i]), f"accumulate {i}")
+    for s, n in zip(slabs, sizes):
+        assert (s[:16 + out_off] == 9.0).all() and (s[16 + out_off + n:] == 9.0).all()
