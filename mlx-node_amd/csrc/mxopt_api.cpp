@@ -795,6 +795,13 @@ int mxopt_sgd_plain(mxopt_ctx* ctx, const mxopt_table* t, double learning_rate, 
 
 int mxopt_sgd_plain_with_pending(mxopt_ctx* ctx, const mxopt_table* t, double learning_rate, double weight_decay,
                                  const mxopt_grad_prep* prep, int prep_covers_sum) {
+  return sgd_plain_with_pending(ctx, t, learning_rate, weight_decay, prep, prep_covers_sum, false);
+}
+
+}  // extern "C"
+
+int mxopt::sgd_plain_with_pending(mxopt_ctx* ctx, const mxopt_table* t, double learning_rate, double weight_decay,
+                                  const mxopt_grad_prep* prep, int prep_covers_sum, bool sum_16) {
   int rc = require(ctx, t, kNeedP | kNeedPOut | kNeedG | kNeedGOut, "mxopt_sgd_plain_with_pending");
   if (rc) return rc;
   DevPrep dp = make_prep(prep);
@@ -803,9 +810,12 @@ int mxopt_sgd_plain_with_pending(mxopt_ctx* ctx, const mxopt_table* t, double le
   const float wd32 = (float)weight_decay;
   const int has_wd = weight_decay > 0.0;  // sft/engine.rs:345
   return run_update(ctx, t, "mxopt_sgd_plain_with_pending", [&](const Group& g, const Launch& L) {
+    if (g.gd != MXOPT_F32 && !sum_16) return false;
     return launch_sgd_plain_pending(g.pd, g.gd, g.pod, g.god, L, round_to_dtype(lr32, g.pd), wd32, has_wd, dp);
   });
 }
+
+extern "C" {
 
 static void attach_pending(const mxopt_table* t, Launch& L) {
   L.pending = t->d_pending;

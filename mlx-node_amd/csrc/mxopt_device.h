@@ -167,6 +167,19 @@ __device__ __forceinline__ void load_group(const void* base, uint64_t off, float
   }
 }
 
+// x rounded to DT and widened again, two elements per conversion (Elem::round takes three instructions for each).
+template <int DT, int E>
+__device__ __forceinline__ void round_group(float (&x)[E]) {
+  if constexpr (DT != MXOPT_F32) {
+#pragma unroll
+    for (int e = 0; e < E; e += 2) {
+      const uint32_t w = Elem<DT>::pack2(x[e], x[e + 1]);
+      x[e] = Elem<DT>::unpack(w & 0xffffu);
+      x[e + 1] = Elem<DT>::unpack(w >> 16);
+    }
+  }
+}
+
 template <int DT, int E, bool NT>
 __device__ __forceinline__ void store_group(void* base, uint64_t off, const float (&x)[E]) {
   if constexpr (DT == MXOPT_F32) {

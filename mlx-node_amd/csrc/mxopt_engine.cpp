@@ -738,9 +738,17 @@ int sft_micro_batch(mxopt_engine* e, const std::vector<size_t>& idx, const mxopt
   // Last micro-batch of the cycle, every held tensor has a gradient in it: the sum acc + g is formed
   // in registers by the norm pass and again by the update, instead of being written back and read
   // twice.  With no accumulator yet (N = 1) the gradient is applied straight from where it lies.
-  bool all_f32 = true;
+  // A 16-bit accumulator takes the same way (both passes round the sum to its dtype): r(acc, g) + r(p, acc, g) w(p) is
+  // as many bytes as r(acc, g) w(acc) + r(p, acc) w(p), but half the writes.  bf16, 596 M elements: 705 + 667 us of
+  // accumulation with norm and update -> 411 + 835 us, the step of four micro-batches 3.18 -> 3.05 ms.
+  bool all_f32 = true, twice = false;
+  std::vector<char> seen(e->slots.size(), 0);
   for (const mxopt_tensor& r : rows) all_f32 = all_f32 && r.g_out_dtype == MXOPT_F32;
-  const bool pending = boundary && !first_cycle_step && e->cfg.apply == MXOPT_ENGINE_APPLY_SGD && all_f32 &&
+  for (size_t i = 0; i < n; ++i) {  // a name given twice: the buffer holds one of the sums
+    twice = twice || seen[idx[i]];
+    seen[idx[i]] = 1;
+  }
+  const bool pending = boundary && !first_cycle_step && e->cfg.apply == MXOPT_ENGINE_APPLY_SGD && (all_f32 || !twice) &&
                        rows.size() == held;
   if ((direct || pending) && !rows.empty()) {
     mxopt_grad_prep prep = no_prep();
@@ -780,7 +788,7 @@ int sft_micro_batch(mxopt_engine* e, const std::vector<size_t>& idx, const mxopt
       if (direct) {
         r.g = grads[i].data; r.g_dtype = (uint8_t)grads[i].dtype;
       } else {
-        r.g = s.acc; r.g_dtype = MXOPT_F32;
+        r.g = s.acc; r.g_dtype = (uint8_t)s.acc_dtype;
         r.g_out = grads[i].data; r.g_out_dtype = (uint8_t)grads[i].dtype;
       }
       urows.push_back(r);
@@ -795,7 +803,7 @@ int sft_micro_batch(mxopt_engine* e, const std::vector<size_t>& idx, const mxopt
     } else {
       if ((rc = cached_table(ctx, urows, &t))) return rc;
       rc = direct ? mxopt_sgd_plain(ctx, t, e->cfg.learning_rate, e->cfg.weight_decay, &prep)
-                  : mxopt_sgd_plain_with_pending(ctx, t, e->cfg.learning_rate, e->cfg.weight_decay, &prep, 1);
+                  : sgd_plain_with_pending(ctx, t, e->cfg.learning_rate, e->cfg.weight_decay, &prep, 1, true);
     }
     if (rc) return rc;
     end_cycle(e);

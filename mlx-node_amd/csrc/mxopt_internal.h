@@ -77,6 +77,10 @@ int check_array(mxopt_ctx* ctx, const mxopt_array* a, const char* what, bool all
 // keeps the most recently used few.
 int cached_table(mxopt_ctx* ctx, std::vector<mxopt_tensor>& rows, mxopt_table** out);
 int norm_scratch(mxopt_ctx* ctx, mxopt_norm_result** out);
+// mxopt_sgd_plain_with_pending; sum_16 also takes 16-bit accumulation buffers whose pending gradient has their dtype
+// (prep_covers_sum only): the sum is rounded to that dtype in registers, as the buffer would have stored it.
+int sgd_plain_with_pending(mxopt_ctx* ctx, const mxopt_table* t, double learning_rate, double weight_decay,
+                           const mxopt_grad_prep* prep, int prep_covers_sum, bool sum_16);
 // Puts an optimizer's call counter (mxopt_optimizer_step_count) back: for a caller whose conditional
 // update turned out to have been skipped on the device.
 void optimizer_set_step_count(mxopt_optimizer* opt, int64_t calls);

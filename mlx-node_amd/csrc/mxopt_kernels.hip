@@ -8,8 +8,8 @@ namespace mxopt {
 
 // ------------------------------------------------------------------------------------
 // Update kernel.  G2 >= 0: a second gradient stream of that dtype in tensor.g_out is added to g
-// first (one float32 add: the last micro-batch folded into the update instead of being written
-// back to the accumulation buffer).
+// first (one float32 add, rounded to the buffer's dtype GD: the last micro-batch folded into the
+// update instead of being written back to the accumulation buffer).
 // ------------------------------------------------------------------------------------
 
 template <int PD, int GD, int OD, int G2, class Math, bool NT>
@@ -18,6 +18,7 @@ __global__ __launch_bounds__(kThreads) void update_kernel(const DevTensor* __res
                                                           uint32_t nchunks, Math math, DevPrep prep) {
   constexpr bool kHasG2 = G2 >= 0;
   constexpr int G2D = kHasG2 ? G2 : MXOPT_F32;
+  constexpr bool kSum16 = kHasG2 && GD != MXOPT_F32;  // the sum is what a 16-bit buffer would have held
   // Elements per lane and group.  With a 16-bit stream in the mix, 8 (one 16-byte access of the 16-bit stream,
   // two of every float32 stream) when a second gradient stream is folded in, 4 (8-byte accesses of the 16-bit
   // streams, one 16-byte access of the float32 ones) without: then every access covers whole sectors and can
@@ -38,6 +39,7 @@ __global__ __launch_bounds__(kThreads) void update_kernel(const DevTensor* __res
   const bool pending_only = kHasG2 && (pr.flags & kPrepPendingOnly);
   auto combine = [&](float g, float g2) {
     if (!kHasG2) return prep_all(pr, g);
+    if (kSum16) return prep_all(pr, Elem<GD>::round(g + g2));
     return pending_only ? g + prep_all(pr, g2) : prep_all(pr, g + g2);
   };
 
@@ -78,9 +80,15 @@ __global__ __launch_bounds__(kThreads) void update_kernel(const DevTensor* __res
       }
 #pragma unroll
       for (int j = 0; j < U; ++j) {
+        if (kSum16) {
+#pragma unroll
+          for (int e = 0; e < E; ++e) g[j][e] = g[j][e] + g2[j][e];
+          round_group<GD, E>(g[j]);
+        }
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-          math(p[j][e], combine(g[j][e], g2[j][e]), m[j][e], v[j][e], bc1, bc2, flags);
+          const float ge = kSum16 ? prep_all(pr, g[j][e]) : combine(g[j][e], g2[j][e]);
+          math(p[j][e], ge, m[j][e], v[j][e], bc1, bc2, flags);
         }
       }
 #pragma unroll
@@ -289,10 +297,13 @@ static bool plain_for_pd(int gd, int od, const Launch& L, float lr_p, float wd, 
   return dispatch_gd<PD>(gd, od, L, m, prep);
 }
 
-// Plain SGD on (float32 accumulation buffer + prep(pending gradient)); output in the parameter's dtype.
+// Plain SGD on (float32 accumulation buffer + prep(pending gradient)), or on prep(16-bit buffer + pending gradient of
+// the same dtype); output in the parameter's dtype.
 template <int PD>
-static bool plain_pending_for_pd(int g2d, const Launch& L, float lr_p, float wd, int has_wd, const DevPrep& prep) {
+static bool plain_pending_for_pd(int gd, int g2d, const Launch& L, float lr_p, float wd, int has_wd, const DevPrep& prep) {
   PlainSgdMath<PD, false> m{lr_p, wd, has_wd};
+  if (gd == MXOPT_BF16) { launch_update_t<PD, MXOPT_BF16, PD, MXOPT_BF16>(L, m, prep); return true; }
+  if (gd == MXOPT_F16) { launch_update_t<PD, MXOPT_F16, PD, MXOPT_F16>(L, m, prep); return true; }
   switch (g2d) {
     case MXOPT_F32: launch_update_t<PD, MXOPT_F32, PD, MXOPT_F32>(L, m, prep); return true;
     case MXOPT_BF16: launch_update_t<PD, MXOPT_F32, PD, MXOPT_BF16>(L, m, prep); return true;
@@ -303,11 +314,12 @@ static bool plain_pending_for_pd(int g2d, const Launch& L, float lr_p, float wd,
 
 bool launch_sgd_plain_pending(int pd, int gd, int od, int g2d, const Launch& L, float lr_p, float wd, int has_wd,
                               const DevPrep& prep) {
-  if (gd != MXOPT_F32 || od != pd) return false;
+  if (od != pd) return false;
+  if (gd != MXOPT_F32 && (gd != g2d || (prep.flags & kPrepPendingOnly))) return false;
   switch (pd) {
-    case MXOPT_F32: return plain_pending_for_pd<MXOPT_F32>(g2d, L, lr_p, wd, has_wd, prep);
-    case MXOPT_BF16: return plain_pending_for_pd<MXOPT_BF16>(g2d, L, lr_p, wd, has_wd, prep);
-    case MXOPT_F16: return plain_pending_for_pd<MXOPT_F16>(g2d, L, lr_p, wd, has_wd, prep);
+    case MXOPT_F32: return plain_pending_for_pd<MXOPT_F32>(gd, g2d, L, lr_p, wd, has_wd, prep);
+    case MXOPT_BF16: return plain_pending_for_pd<MXOPT_BF16>(gd, g2d, L, lr_p, wd, has_wd, prep);
+    case MXOPT_F16: return plain_pending_for_pd<MXOPT_F16>(gd, g2d, L, lr_p, wd, has_wd, prep);
   }
   return false;
 }

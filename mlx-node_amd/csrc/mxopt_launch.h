@@ -39,7 +39,8 @@ bool launch_sgd_plain(int pd, int gd, int od, const Launch& L, float lr_p, float
                       const DevPrep& prep);
 // add != 0: g_out = g_out + prep(g) instead of g_out = prep(g).
 // g: float32 accumulation buffer, tensor.g_out: pending gradient of dtype g2d; prep's kPrepPendingOnly
-// flag says whether prep covers the pending gradient alone or the sum.
+// flag says whether prep covers the pending gradient alone or the sum.  A 16-bit g goes with a pending gradient of its
+// own dtype and a prep that covers the sum.
 bool launch_sgd_plain_pending(int pd, int gd, int od, int g2d, const Launch& L, float lr_p, float wd, int has_wd,
                               const DevPrep& prep);
 bool launch_transform(int gd, int od, const Launch& L, const DevPrep& prep, int add);

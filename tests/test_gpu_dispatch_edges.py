@@ -71,3 +71,35 @@ def test_streams_of_different_16_byte_phases(mx, ctx, g_off, out_off, dtype):
         assert_bit_equal(to_host(outs[i]), w + O.as_f32(gs[i]), f"accumulate {i}")
     for s, n in zip(slabs, sizes):
         assert (s[:16 + out_off] == 9.0).all() and (s[16 + out_off + n:] == 9.0).all()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("micro", [2, 3])
+def test_sft_last_micro_batch_folded_into_a_16_bit_sum(mx, ctx, dtype, micro):
+    """The sum the update forms in registers is the 16-bit sum an accumulation pass would have stored: every operation
+    redone on the host, one rounding at a time, over every remainder of a group and of a chunk.  Bit for bit."""
+    import torch
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float16
+    sizes = [1, 2, 7, 8, 9, 255 * 8 + 1, CHUNK - 1, CHUNK, CHUNK + 1, 3 * CHUNK + 13]
+    gen = torch.Generator().manual_seed(11)
+    ps = {str(i): torch.randn(n, generator=gen).mul_(0.02).to(dt) for i, n in enumerate(sizes)}
+    gs = [{k: torch.randn(p.numel(), generator=gen).mul_(0.1).to(dt) for k, p in ps.items()} for _ in range(micro)]
+    dev = {k: p.cuda() for k, p in ps.items()}
+    engine = mx.SFTEngineOptimizerSide(dev, learning_rate=0.5, gradient_accumulation_steps=micro, weight_decay=0.01, ctx=ctx)
+    for cycle in range(2):                       # the second one overwrites what the first left in the buffers
+        for g in gs:
+            m = engine.micro_batch({k: x.cuda() for k, x in g.items()})
+        assert m.gradients_applied and m.norm_measured
+        total = 0.0
+        for k in ps:
+            s = gs[0][k]
+            for g in gs[1:]:
+                s = (s.float() + g[k].float()).to(dt)
+            ge = s.float() * torch.tensor(1.0 / micro, dtype=torch.float32)
+            total += float((ge.double() ** 2).sum())
+            ge = ge * torch.tensor(m.clip_scale, dtype=torch.float32)
+            ge = ge + ps[k].float() * torch.tensor(0.01, dtype=torch.float32)
+            lr = torch.tensor(0.5).to(dt).float()
+            ps[k] = (ps[k].float() - lr * ge).to(dt)
+            assert torch.equal(dev[k].cpu().view(torch.int16), ps[k].view(torch.int16)), (cycle, k)
+        assert abs(m.grad_sumsq - total) <= 1e-6 * total  # float32 squares, 16 of them added in float32
