@@ -39,7 +39,7 @@ def _run(cmd, verbose):
     err = "\n".join(l for l in proc.stderr.splitlines() if "packed-fp32-ops" not in l)
     if proc.returncode != 0:
         sys.stderr.write(err + "\n")
-        raise RuntimeError("hipcc failed: " + os.path.basename(cmd[-1]))
+        raise RuntimeError(os.path.basename(cmd[0]) + " failed: " + os.path.basename(cmd[-1]))
     if verbose and err.strip():
         print(err)
 
@@ -74,6 +74,10 @@ def build(verbose: bool = False, incremental: bool = False) -> str:
     from concurrent.futures import ThreadPoolExecutor
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     os.makedirs(OBJ_DIR, exist_ok=True)
+    arrays, arrays_pool = None, ThreadPoolExecutor(max_workers=1)
+    source = os.path.join(CSRC, "mxopt_torch_arrays.cpp")
+    if not (incremental and os.path.exists(ARRAYS) and os.path.getmtime(ARRAYS) > max(os.path.getmtime(source), _headers_mtime())):
+        arrays = arrays_pool.submit(build_arrays, verbose)
     jobs, objs = [], []
     newest_header = _headers_mtime() if incremental else 0.0
     for s in SOURCES:
@@ -88,9 +92,33 @@ def build(verbose: bool = False, incremental: bool = False) -> str:
     jobs = [(None, o) for o in objs]
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC"] + [obj for _, obj in jobs] + ["-o", LIB + ".tmp"], verbose)
     os.replace(LIB + ".tmp", LIB)
+    if arrays is not None:
+        arrays.result()
+    arrays_pool.shutdown()
     build_demo(verbose)
     build_napi(verbose)
     return LIB
+
+
+ARRAYS = os.path.join(HERE, "mxopt", "_arrays.so")
+
+
+def build_arrays(verbose: bool = False) -> str:
+    """csrc/mxopt_torch_arrays.cpp -> mxopt/_arrays.so, the part of the Python package that reads torch's tensors in
+    C++.  Tied to the torch it is compiled against, whose libraries the importing process has loaded."""
+    import importlib.util
+    import sysconfig
+    torch_dir = importlib.util.find_spec("torch").submodule_search_locations[0]
+    inc, lib = os.path.join(torch_dir, "include"), os.path.join(torch_dir, "lib")
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(ROOT, "include"),
+           "-isystem", inc, "-isystem", os.path.join(inc, "torch", "csrc", "api", "include"),
+           "-isystem", os.path.join(rocm, "include"), "-I", sysconfig.get_paths()["include"],
+           os.path.join(CSRC, "mxopt_torch_arrays.cpp"), "-o", ARRAYS + ".tmp",
+           "-L", lib, "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    _run(cmd, verbose)
+    os.replace(ARRAYS + ".tmp", ARRAYS)
+    return ARRAYS
 
 
 DEMO = os.path.join(HERE, "bin", "cabi_demo")

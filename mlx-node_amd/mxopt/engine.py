@@ -17,7 +17,7 @@ import torch
 
 from . import _lib as L
 from .core import Context
-from .optimizers import _arr, default_context
+from .optimizers import _arrs, _names, default_context
 
 
 class TrainingStopped(L.MxoptError):
@@ -34,10 +34,8 @@ class _EngineOptimizerSide:
         self._held = []
         self.params = dict(params)
         names = list(self.params)
-        cnames = (C.c_char_p * max(len(names), 1))(*[s.encode() for s in names])
-        arrs = (L.Array * max(len(names), 1))()
-        for i, nm in enumerate(names):
-            arrs[i] = _arr(self.params[nm])
+        cnames = _names(names)
+        arrs = _arrs([self.params[nm] for nm in names])
         self.handle = C.c_void_p()
         L.check(self.lib.mxopt_engine_new(self.ctx.handle, C.byref(cfg), len(names), cnames, arrs,
                                           C.byref(self.handle)), self.ctx.handle)
@@ -69,10 +67,8 @@ class _EngineOptimizerSide:
     def micro_batch(self, gradients: Dict[str, torch.Tensor]) -> L.EngineMetrics:
         """The part of train_step after the backward pass, for one micro-batch of gradients."""
         names = list(gradients)
-        cnames = (C.c_char_p * max(len(names), 1))(*[s.encode() for s in names])
-        arrs = (L.Array * max(len(names), 1))()
-        for i, nm in enumerate(names):
-            arrs[i] = _arr(gradients[nm])
+        cnames = _names(names)
+        arrs = _arrs([gradients[nm] for nm in names])
         m = L.EngineMetrics()
         if self.defers:   # deferred accumulation reads the cycle's gradients when it is applied: keep them alive
             self._held.append(list(gradients.values()))
@@ -85,10 +81,8 @@ class _EngineOptimizerSide:
         """micro_batch without the host synchronisation (GRPO, plain-SGD apply): the validity flag stays on the
         device; settle() -- or the next call of any kind -- books a skipped micro-batch afterwards."""
         names = list(gradients)
-        cnames = (C.c_char_p * max(len(names), 1))(*[s.encode() for s in names])
-        arrs = (L.Array * max(len(names), 1))()
-        for i, nm in enumerate(names):
-            arrs[i] = _arr(gradients[nm])
+        cnames = _names(names)
+        arrs = _arrs([gradients[nm] for nm in names])
         # the kernels read the gradients after this returns: they stay alive until the call after next has settled them
         self._async_keep = [getattr(self, "_async_keep", [None, None])[1], list(gradients.values())]
         if self.defers:

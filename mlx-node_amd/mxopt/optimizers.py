@@ -18,7 +18,7 @@ from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
 
-from . import _lib as L
+from . import _arrays, _lib as L
 from .core import Context, dtype_code
 
 _default_ctx: Optional[Context] = None
@@ -42,9 +42,22 @@ def _arr(t: Optional[torch.Tensor]) -> L.Array:
 
 
 def _arrs(ts: Sequence[Optional[torch.Tensor]]):
-    a = (L.Array * max(len(ts), 1))()
-    for i, t in enumerate(ts):
-        a[i] = _arr(t)
+    if not isinstance(ts, (list, tuple)):
+        ts = list(ts)
+    n = len(ts)
+    a = (L.Array * max(n, 1))()
+    at = _arrays.fill(ts, C.addressof(a), 0, n)
+    while at < n:   # not plainly a dense device tensor: described, or refused, here
+        a[at] = _arr(ts[at])
+        at = _arrays.fill(ts, C.addressof(a), at + 1, n)
+    return a
+
+
+def _names(names: Sequence[str]):
+    held = tuple(names)
+    a = (C.c_char_p * max(len(held), 1))()
+    _arrays.names(held, C.addressof(a))
+    a.held = held   # the strings the pointers point into
     return a
 
 
@@ -66,6 +79,7 @@ class _Optimizer:
     def __init__(self, ctx: Optional[Context]):
         self.ctx = ctx or default_context()
         self.lib = self.ctx.lib
+        self._update_single = C.cast(self.lib.mxopt_optimizer_update_single, C.c_void_p).value
         self.handle = C.c_void_p()
 
     def __del__(self):
@@ -79,8 +93,12 @@ class _Optimizer:
         itself for an in-place update."""
         if out is None:
             out = _out_like(param, out_dtype)
-        L.check(self.lib.mxopt_optimizer_update_single(self.handle, param_name.encode(), C.byref(_arr(param)),
-                                                       C.byref(_arr(grad)), C.byref(_arr(out))), self.ctx.handle)
+        rc = _arrays.update_single(self._update_single, self.handle.value, param_name, param, grad, out)
+        if rc is None:
+            rc = self.lib.mxopt_optimizer_update_single(self.handle, param_name.encode(), C.byref(_arr(param)),
+                                                        C.byref(_arr(grad)), C.byref(_arr(out)))
+        if rc != L.OK:
+            L.check(rc, self.ctx.handle)
         return out
 
     def update_many(self, names: Sequence[str], params: Sequence[torch.Tensor], grads: Sequence[torch.Tensor],
@@ -90,7 +108,7 @@ class _Optimizer:
         if outs is None:
             outs = [_out_like(p, out_dtype) for p in params]
         n = len(names)
-        cnames = (C.c_char_p * max(n, 1))(*[s.encode() for s in names])
+        cnames = _names(names)
         L.check(self.lib.mxopt_optimizer_update_many(self.handle, n, cnames, _arrs(params), _arrs(grads), _arrs(outs),
                                                      C.byref(prep) if prep else None), self.ctx.handle)
         return list(outs)
@@ -107,7 +125,7 @@ class _Optimizer:
         n, k = len(names), len(micro_batches)
         if any(len(mb) != n for mb in micro_batches):
             raise L.InvalidArg(L.ERR_INVALID_ARG, "every micro-batch needs one gradient per name")
-        cnames = (C.c_char_p * max(n, 1))(*[s.encode() for s in names])
+        cnames = _names(names)
         flat = [g for mb in micro_batches for g in mb]
         L.check(self.lib.mxopt_optimizer_update_many_accumulated(
             self.handle, n, cnames, _arrs(params), k, _arrs(flat), _arrs(outs), C.byref(prep) if prep else None,

@@ -103,3 +103,24 @@ def test_sft_last_micro_batch_folded_into_a_16_bit_sum(mx, ctx, dtype, micro):
             ps[k] = (ps[k].float() - lr * ge).to(dt)
             assert torch.equal(dev[k].cpu().view(torch.int16), ps[k].view(torch.int16)), (cycle, k)
         assert abs(m.grad_sumsq - total) <= 1e-6 * total  # float32 squares, 16 of them added in float32
+
+
+def test_descriptors_made_in_c_equal_the_ones_made_in_python(mx):
+    import torch
+    from mxopt import optimizers as M
+
+    class Sub(torch.Tensor):
+        pass
+
+    base = torch.arange(64, dtype=torch.float32, device="cuda")
+    ts = [None, base, base[3:7], base[:0], base.to(torch.bfloat16)[1:], base.half(), torch.nn.Parameter(base.clone()),
+          base.as_subclass(Sub), base.view(8, 8), base.view(8, 8)[:, :1].reshape(-1)]
+    got = M._arrs(ts)
+    for t, a in zip(ts, got):
+        want = M._arr(t)
+        assert (a.data, a.n, a.dtype) == (want.data, want.n, want.dtype)
+    for bad in (base.view(8, 8).t(), base[::2], base.double(), base.cpu()):
+        with pytest.raises(mx.InvalidArg):
+            M._arrs([base, bad])
+        with pytest.raises(mx.InvalidArg):
+            mx.Adam().update_single("p", base.clone(), bad)
