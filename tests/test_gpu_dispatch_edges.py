@@ -114,7 +114,7 @@ def test_descriptors_made_in_c_equal_the_ones_made_in_python(mx):
 
     base = torch.arange(64, dtype=torch.float32, device="cuda")
     ts = [None, base, base[3:7], base[:0], base.to(torch.bfloat16)[1:], base.half(), torch.nn.Parameter(base.clone()),
-          base.as_subclass(Sub), base.view(8, 8), base.view(8, 8)[:, :1].reshape(-1)]
+          base.as_subclass(Sub), base.view(8, 8), base.view(8, 8)[2]]
     got = M._arrs(ts)
     for t, a in zip(ts, got):
         want = M._arr(t)
@@ -124,3 +124,15 @@ def test_descriptors_made_in_c_equal_the_ones_made_in_python(mx):
             M._arrs([base, bad])
         with pytest.raises(mx.InvalidArg):
             mx.Adam().update_single("p", base.clone(), bad)
+
+
+@pytest.mark.parametrize("n", [1, 7, CHUNK + 3, 32768 * CHUNK, 32768 * CHUNK + 1])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_widening_transform_on_both_sides_of_its_line(mx, ctx, n, dtype):
+    """A power of two times the gradient: exact, so the reference is the same product in torch."""
+    import torch
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float16
+    g = torch.empty(n, dtype=dt, device="cuda").normal_()
+    out = torch.full((n + 4,), 7.0, dtype=torch.float32, device="cuda")
+    ctx.grad_transform(ctx.table([mx.TensorSpec(g=g, g_out=out[:n])]), mx.make_prep(pre_mul=0.5))
+    assert torch.equal(out[:n], g.float() * 0.5) and bool((out[n:] == 7.0).all())
