@@ -74,10 +74,6 @@ def build(verbose: bool = False, incremental: bool = False) -> str:
     from concurrent.futures import ThreadPoolExecutor
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     os.makedirs(OBJ_DIR, exist_ok=True)
-    arrays, arrays_pool = None, ThreadPoolExecutor(max_workers=1)
-    source = os.path.join(CSRC, "mxopt_torch_arrays.cpp")
-    if not (incremental and os.path.exists(ARRAYS) and os.path.getmtime(ARRAYS) > max(os.path.getmtime(source), _headers_mtime())):
-        arrays = arrays_pool.submit(build_arrays, verbose)
     jobs, objs = [], []
     newest_header = _headers_mtime() if incremental else 0.0
     for s in SOURCES:
@@ -87,37 +83,75 @@ def build(verbose: bool = False, incremental: bool = False) -> str:
         if incremental and os.path.exists(obj) and os.path.getmtime(obj) > max(os.path.getmtime(src), newest_header):
             continue
         jobs.append(([hipcc] + FLAGS + ["-x", "hip", "-c", src, "-o", obj], obj))
-    with ThreadPoolExecutor(max_workers=min(max(len(jobs), 1), os.cpu_count() or 1, 8)) as pool:
-        list(pool.map(lambda j: _run(j[0], verbose), jobs))
-    jobs = [(None, o) for o in objs]
-    _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC"] + [obj for _, obj in jobs] + ["-o", LIB + ".tmp"], verbose)
-    os.replace(LIB + ".tmp", LIB)
-    if arrays is not None:
-        arrays.result()
-    arrays_pool.shutdown()
-    build_demo(verbose)
-    build_napi(verbose)
+    with ThreadPoolExecutor(max_workers=1) as arrays_pool:
+        # the Python package's extension compiles beside the library; whatever becomes of it, the library, the demo and the
+        # N-API binding, which need neither torch nor Python's headers, are finished first
+        arrays = None if incremental and _arrays_current() else arrays_pool.submit(build_arrays, verbose)
+        with ThreadPoolExecutor(max_workers=min(max(len(jobs), 1), os.cpu_count() or 1, 8)) as pool:
+            list(pool.map(lambda j: _run(j[0], verbose), jobs))
+        _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC"] + objs + ["-o", LIB + ".tmp"], verbose)
+        os.replace(LIB + ".tmp", LIB)
+        build_demo(verbose)
+        build_napi(verbose)
+        if arrays is not None:
+            arrays.result()
     return LIB
 
 
 ARRAYS = os.path.join(HERE, "mxopt", "_arrays.so")
+ARRAYS_SOURCE = os.path.join(CSRC, "mxopt_torch_arrays.cpp")
 
 
-def build_arrays(verbose: bool = False) -> str:
-    """csrc/mxopt_torch_arrays.cpp -> mxopt/_arrays.so, the part of the Python package that reads torch's tensors in
-    C++.  Tied to the torch it is compiled against, whose libraries the importing process has loaded."""
+def _torch_dir():
     import importlib.util
+    spec = importlib.util.find_spec("torch")
+    return None if spec is None else spec.submodule_search_locations[0]
+
+
+def _arrays_stamp():
+    """Which torch and Python _arrays.so is compiled for (None: torch is not installed), read from torch's version.py
+    without importing it."""
+    torch_dir = _torch_dir()
+    if torch_dir is None:
+        return None
+    with open(os.path.join(torch_dir, "version.py")) as f:
+        return "\n".join([sys.version, torch_dir, f.read()])
+
+
+def _stamp_file() -> str:
+    return os.path.join(OBJ_DIR, "_arrays.torch")
+
+
+def _arrays_current() -> bool:
+    """_arrays.so is newer than what it is made of and made for the torch and the Python at hand."""
+    if not (os.path.exists(ARRAYS) and os.path.exists(_stamp_file())):
+        return False
+    with open(_stamp_file()) as f:
+        same = f.read() == _arrays_stamp()
+    return same and os.path.getmtime(ARRAYS) > max(os.path.getmtime(ARRAYS_SOURCE), _headers_mtime())
+
+
+def build_arrays(verbose: bool = False):
+    """csrc/mxopt_torch_arrays.cpp -> mxopt/_arrays.so, the part of the Python package that reads torch's tensors in
+    C++.  Tied to the torch it is compiled against, whose libraries the importing process has loaded.  Without torch
+    there is no Python package and nothing to build (None)."""
     import sysconfig
-    torch_dir = importlib.util.find_spec("torch").submodule_search_locations[0]
+    torch_dir = _torch_dir()
+    if torch_dir is None:
+        sys.stderr.write("torch is not installed: mxopt/_arrays.so, which only the Python package needs, is not built\n")
+        return None
     inc, lib = os.path.join(torch_dir, "include"), os.path.join(torch_dir, "lib")
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(ROOT, "include"),
            "-isystem", inc, "-isystem", os.path.join(inc, "torch", "csrc", "api", "include"),
            "-isystem", os.path.join(rocm, "include"), "-I", sysconfig.get_paths()["include"],
-           os.path.join(CSRC, "mxopt_torch_arrays.cpp"), "-o", ARRAYS + ".tmp",
+           ARRAYS_SOURCE, "-o", ARRAYS + ".tmp",
            "-L", lib, "-ltorch_python", "-ltorch_cpu", "-lc10"]
     _run(cmd, verbose)
     os.replace(ARRAYS + ".tmp", ARRAYS)
+    os.makedirs(OBJ_DIR, exist_ok=True)
+    with open(_stamp_file(), "w") as f:
+        f.write(_arrays_stamp())
     return ARRAYS
 
 
