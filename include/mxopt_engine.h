@@ -102,7 +102,8 @@ void mxopt_engine_free(mxopt_engine* e);
  * SFT (sft/engine.rs:268-371): acc += g (names the accumulator does not hold are dropped);
  *   every N-th micro-batch p -= lr * (clamp(clip_norm(acc/N)) + wd*p).
  * A gradient whose name is not a parameter is refused before anything is touched with the
- * message of models/qwen3/model.rs:2427-2432 (the reference fails at apply time).
+ * message of models/qwen3/model.rs:2427-2432 (the reference fails at apply time).  A name given
+ * twice counts once, with its first gradient (the reference's maps hold one per name).
  * `out` may be NULL. */
 int mxopt_engine_micro_batch(mxopt_engine* e, size_t n, const char* const* names, const mxopt_array* grads,
                              mxopt_engine_metrics* out);

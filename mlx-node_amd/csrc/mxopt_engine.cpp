@@ -155,22 +155,35 @@ int ensure_acc(mxopt_engine* e, Slot& s, int dtype) {
   return MXOPT_OK;
 }
 
-// Checks names and sizes; on success idx[i] is the slot of gradient i.
-int resolve(mxopt_engine* e, size_t n, const char* const* names, const mxopt_array* grads, std::vector<size_t>* idx) {
+// Checks names and sizes; on success idx[i] is the slot of gradient (*grads)[i].  A name given twice keeps its first
+// gradient, as the maps of the reference hold one per name: everything behind this call sees every slot once (two rows of
+// one launch must not write the same buffer).  `once` then holds the gradients that are left and *grads points to it.
+int resolve(mxopt_engine* e, size_t n, const char* const* names, const mxopt_array** grads, std::vector<size_t>* idx,
+            std::vector<mxopt_array>* once) {
   mxopt_ctx* ctx = e->ctx;
-  if (n && (!names || !grads)) return fail(ctx, MXOPT_ERR_INVALID_ARG, "engine: null names or gradients");
-  idx->resize(n);
+  const mxopt_array* g = *grads;
+  if (n && (!names || !g)) return fail(ctx, MXOPT_ERR_INVALID_ARG, "engine: null names or gradients");
+  idx->clear();
+  idx->reserve(n);
+  std::vector<char> seen(e->slots.size(), 0);
   for (size_t i = 0; i < n; ++i) {
     if (!names[i]) return fail(ctx, MXOPT_ERR_INVALID_ARG, "engine: null gradient name");
     auto it = e->index.find(names[i]);
     if (it == e->index.end())  // models/qwen3/model.rs:2427-2432
       return fail(ctx, MXOPT_ERR_FAILURE, std::string("Parameter '") + names[i] + "' not found in model");
-    int rc = check_array(ctx, &grads[i], "engine: gradient");
+    int rc = check_array(ctx, &g[i], "engine: gradient");
     if (rc) return rc;
-    if (grads[i].n != e->slots[it->second].param.n)
+    if (g[i].n != e->slots[it->second].param.n)
       return fail(ctx, MXOPT_ERR_INVALID_ARG, std::string("engine: gradient '") + names[i] + "' has the wrong size");
-    (*idx)[i] = it->second;
+    if (seen[it->second]) {
+      if (once->empty()) once->assign(g, g + i);
+      continue;
+    }
+    seen[it->second] = 1;
+    idx->push_back(it->second);
+    if (!once->empty()) once->push_back(g[i]);
   }
+  if (!once->empty()) *grads = once->data();
   return MXOPT_OK;
 }
 
@@ -230,33 +243,19 @@ void end_cycle(mxopt_engine* e) {
 // ---- deferred accumulation ---------------------------------------------------------------
 
 // Remembers where this micro-batch's gradients lie.  The first micro-batch of a cycle fixes the set of
-// names (a name given twice keeps its first gradient, as the maps of the reference would); later ones
-// must bring exactly that set.
+// names; later ones must bring exactly that set.
 int defer_record(mxopt_engine* e, const std::vector<size_t>& idx, const mxopt_array* grads) {
   mxopt_ctx* ctx = e->ctx;
   const size_t n = idx.size();
   if (e->held.empty()) {
-    std::vector<char> seen(e->slots.size(), 0);
-    e->held_slots.clear();
-    std::vector<mxopt_array> first;
-    for (size_t i = 0; i < n; ++i) {
-      if (seen[idx[i]]) continue;
-      seen[idx[i]] = 1;
-      e->held_slots.push_back(idx[i]);
-      first.push_back(grads[i]);
-    }
-    e->held.push_back(std::move(first));
+    e->held_slots = idx;
+    e->held.emplace_back(grads, grads + n);
     return MXOPT_OK;
   }
   std::vector<const mxopt_array*> by_slot(e->slots.size(), nullptr);
-  size_t distinct = 0;
-  for (size_t i = 0; i < n; ++i) {
-    if (by_slot[idx[i]]) continue;
-    by_slot[idx[i]] = &grads[i];
-    ++distinct;
-  }
+  for (size_t i = 0; i < n; ++i) by_slot[idx[i]] = &grads[i];
   const char* same_names = "engine: deferred accumulation needs the same gradient names in every micro-batch of a cycle";
-  if (distinct != e->held_slots.size()) return fail(ctx, MXOPT_ERR_INVALID_ARG, same_names);
+  if (n != e->held_slots.size()) return fail(ctx, MXOPT_ERR_INVALID_ARG, same_names);
   std::vector<mxopt_array> row;
   const int pending_dtype = e->held.size() > 1 && !e->held[1].empty() ? e->held[1][0].dtype : -1;
   for (size_t slot : e->held_slots) {
@@ -505,7 +504,6 @@ int grpo_micro_batch(mxopt_engine* e, const std::vector<size_t>& idx, const mxop
     std::vector<mxopt_tensor> pending, direct, acc_only;
     for (size_t i = 0; i < n; ++i) {
       Slot& s = e->slots[idx[i]];
-      if (in_batch[idx[i]]) continue;
       in_batch[idx[i]] = 1;
       mxopt_tensor r = blank_tensor();
       r.p = s.param.data; r.p_out = s.param.data;
@@ -783,7 +781,6 @@ int sft_micro_batch(mxopt_engine* e, const std::vector<size_t>& idx, const mxopt
     if (!first_cycle_step && !s.in_acc) continue;  // sft/engine.rs:283-287: silently dropped
     const int want = e->cfg.accumulate_in_f32 ? MXOPT_F32 : grads[i].dtype;
     if (first_cycle_step) {
-      if (s.in_acc) continue;  // the same name twice in one call: the map keeps one
       if (!direct && (rc = ensure_acc(e, s, want))) return rc;
       s.in_acc = true;
     } else if (s.acc_dtype != want && !(s.acc_dtype == MXOPT_F32)) {
@@ -804,15 +801,7 @@ int sft_micro_batch(mxopt_engine* e, const std::vector<size_t>& idx, const mxopt
   // A 16-bit accumulator takes the same way (both passes round the sum to its dtype): r(acc, g) + r(p, acc, g) w(p) is
   // as many bytes as r(acc, g) w(acc) + r(p, acc) w(p), but half the writes.  bf16, 596 M elements: 705 + 667 us of
   // accumulation with norm and update -> 411 + 835 us, the step of four micro-batches 3.18 -> 3.05 ms.
-  bool all_f32 = true, twice = false;
-  std::vector<char> seen(e->slots.size(), 0);
-  for (const mxopt_tensor& r : rows) all_f32 = all_f32 && r.g_out_dtype == MXOPT_F32;
-  for (size_t i = 0; i < n; ++i) {  // a name given twice: the buffer holds one of the sums
-    twice = twice || seen[idx[i]];
-    seen[idx[i]] = 1;
-  }
-  const bool pending = boundary && !first_cycle_step && e->cfg.apply == MXOPT_ENGINE_APPLY_SGD && (all_f32 || !twice) &&
-                       rows.size() == held;
+  const bool pending = boundary && !first_cycle_step && e->cfg.apply == MXOPT_ENGINE_APPLY_SGD && rows.size() == held;
   if ((direct || pending) && !rows.empty()) {
     mxopt_grad_prep prep = no_prep();
     prep.has_pre_mul = 1;
@@ -999,8 +988,8 @@ int mxopt_engine_micro_batch(mxopt_engine* e, size_t n, const char* const* names
   int rc = settle(e, nullptr);
   if (rc) return rc;
   std::vector<size_t> idx;
-  rc = resolve(e, n, names, grads, &idx);
-  if (rc) return rc;
+  std::vector<mxopt_array> once;
+  if ((rc = resolve(e, n, names, &grads, &idx, &once))) return rc;
   if (e->cfg.kind != MXOPT_ENGINE_GRPO) return sft_micro_batch(e, idx, grads, out);
   // Plain SGD: everything is enqueued at once, the kernels obey the validity flag on the device, and the host waits for
   // the flag only then; waited for in between, it left the device idle from the norm pass to the host's next launch
@@ -1028,7 +1017,8 @@ int mxopt_engine_micro_batch_async(mxopt_engine* e, size_t n, const char* const*
   int rc = settle(e, nullptr);  // the previous micro-batch's flag has long arrived; a skip is booked now
   if (rc) return rc;
   std::vector<size_t> idx;
-  if ((rc = resolve(e, n, names, grads, &idx))) return rc;
+  std::vector<mxopt_array> once;
+  if ((rc = resolve(e, n, names, &grads, &idx, &once))) return rc;
   bool enqueued = false, skipped = false;
   mxopt_engine_metrics m;
   rc = grpo_enqueue(e, idx, grads, &m, &enqueued, &skipped);
