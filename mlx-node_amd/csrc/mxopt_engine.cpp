@@ -394,6 +394,17 @@ int ensure_pinned(mxopt_engine* e) {
   return MXOPT_OK;
 }
 
+// For a call that waits for the norm behind the update it has enqueued: under stream capture nothing runs that could be
+// waited for.  Refused in front of the update, with the bookkeeping as it was; found out by the wait, the update would have
+// been captured and the micro-batch booked.
+int refuse_capture(mxopt_engine* e) {
+  DeviceGuard guard(e->ctx->device);
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  HIP_TRY(e->ctx, hipStreamIsCapturing(e->ctx->stream, &status));
+  if (status == hipStreamCaptureStatusNone) return MXOPT_OK;
+  return hip_fail(e->ctx, hipErrorStreamCaptureUnsupported, "engine: the call waits for the norm on the host");
+}
+
 // The result of the norm pass starts its way to pinned host memory; nobody waits for it here.
 int enqueue_flag_copy(mxopt_engine* e, const mxopt_norm_result* d_result) {
   mxopt_ctx* ctx = e->ctx;
@@ -628,7 +639,8 @@ int grpo_enqueue(mxopt_engine* e, const std::vector<size_t>& idx, const mxopt_ar
 // enqueued, so that the update follows the norm pass at once.  (Read in between, the device idled for the read-back and
 // the host's work on the update: 10 - 50 us of a step of 0.9 - 3 ms.)
 int norm_leaves(mxopt_engine* e) {
-  int rc = ensure_pinned(e);
+  int rc = refuse_capture(e);
+  if (!rc) rc = ensure_pinned(e);
   if (rc) return rc;
   DeviceGuard guard(e->ctx->device);
   launch_mirror_result(e->ctx->stream, e->d_result, e->h_pinned);
@@ -995,6 +1007,7 @@ int mxopt_engine_micro_batch(mxopt_engine* e, size_t n, const char* const* names
   // the flag only then; waited for in between, it left the device idle from the norm pass to the host's next launch
   // (bf16, 596 M elements, one micro-batch per step: 926 -> 891 us).  With AdamW a skipped micro-batch would have created moments.
   if (e->cfg.apply != MXOPT_ENGINE_APPLY_SGD) return grpo_micro_batch(e, idx, grads, out);
+  if (!idx.empty() && (rc = refuse_capture(e))) return rc;
   bool enqueued = false, skipped = false;
   mxopt_engine_metrics m;
   rc = grpo_enqueue(e, idx, grads, &m, &enqueued, &skipped);

@@ -128,3 +128,47 @@ def test_deferred_accumulation_step_replays_from_a_graph():
         torch.cuda.synchronize()
     table.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("kind", ["grpo", "sft", "sft-16-bit"])
+def test_engine_call_that_waits_is_refused_under_capture(kind):
+    """A micro-batch that hands its norm back cannot be part of a capture.  The call fails in front of the update, and the
+    engine goes on as if it had not been made."""
+    import torch
+    import mxopt as mx
+    rng = np.random.default_rng(9)
+    ps = {str(n): O.f32_to_bf16(rng.normal(0, 0.5, n).astype(F)) for n in SIZES}
+    grads = {k: to_dev(O.f32_to_bf16(rng.normal(0, 0.1, p.size).astype(F))) for k, p in ps.items()}
+    micro = 1 if kind == "grpo" else 2
+    stream = torch.cuda.Stream()
+    ctxs = [mx.Context(stream=stream), mx.Context()]
+    engines, params = [], []
+    for ctx in ctxs:
+        params.append({k: to_dev(p) for k, p in ps.items()})
+        torch.cuda.synchronize()
+        if kind == "grpo":
+            engines.append(mx.GRPOEngineOptimizerSide(params[-1], learning_rate=0.5, ctx=ctx))
+        else:
+            engines.append(mx.SFTEngineOptimizerSide(params[-1], learning_rate=0.5, gradient_accumulation_steps=2,
+                                                     accumulate_in_f32=kind == "sft", ctx=ctx))
+        for _ in range(2 * micro - 1):                # tables, buffers and pinned memory exist; the next call applies
+            engines[-1].micro_batch(grads)
+    captured, plain = engines
+    before = captured.metrics()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=stream):
+        with pytest.raises(mx.MxoptError, match="waits for the norm"):
+            captured.micro_batch(grads)
+    after = captured.metrics()
+    for name in ("step", "micro_step", "nan_gradient_count", "consecutive_nan_count"):
+        assert getattr(after, name) == getattr(before, name), name
+    for _ in range(1 + micro):
+        a, b = (eng.micro_batch(grads) for eng in engines)
+        torch.cuda.synchronize()
+        assert (a.step, a.gradients_applied, a.norm_measured) == (b.step, b.gradients_applied, b.norm_measured)
+        assert not a.norm_measured or a.grad_sumsq == b.grad_sumsq
+        for k in ps:
+            assert torch.equal(params[0][k], params[1][k]), k
+    del engines, captured, plain
+    for ctx in ctxs:
+        ctx.close()
