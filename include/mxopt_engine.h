@@ -104,7 +104,7 @@ void mxopt_engine_free(mxopt_engine* e);
  * A gradient whose name is not a parameter is refused before anything is touched with the
  * message of models/qwen3/model.rs:2427-2432 (the reference fails at apply time).  A name given
  * twice counts once, with its first gradient (the reference's maps hold one per name).  A call that
- * hands a norm back waits for it, so it is refused, with nothing applied or booked, while the
+ * hands a norm back (flush_gradients too) waits for it, so it is refused, with nothing applied or booked, while the
  * context's stream is being captured.
  * `out` may be NULL. */
 int mxopt_engine_micro_batch(mxopt_engine* e, size_t n, const char* const* names, const mxopt_array* grads,

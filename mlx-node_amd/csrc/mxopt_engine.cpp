@@ -395,8 +395,7 @@ int ensure_pinned(mxopt_engine* e) {
 }
 
 // For a call that waits for the norm behind the update it has enqueued: under stream capture nothing runs that could be
-// waited for.  Refused in front of the update, with the bookkeeping as it was; found out by the wait, the update would have
-// been captured and the micro-batch booked.
+// waited for.  Refused first of all; found out by the wait, the kernels would have been captured and the micro-batch booked.
 int refuse_capture(mxopt_engine* e) {
   DeviceGuard guard(e->ctx->device);
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
@@ -639,8 +638,7 @@ int grpo_enqueue(mxopt_engine* e, const std::vector<size_t>& idx, const mxopt_ar
 // enqueued, so that the update follows the norm pass at once.  (Read in between, the device idled for the read-back and
 // the host's work on the update: 10 - 50 us of a step of 0.9 - 3 ms.)
 int norm_leaves(mxopt_engine* e) {
-  int rc = refuse_capture(e);
-  if (!rc) rc = ensure_pinned(e);
+  int rc = ensure_pinned(e);
   if (rc) return rc;
   DeviceGuard guard(e->ctx->device);
   launch_mirror_result(e->ctx->stream, e->d_result, e->h_pinned);
@@ -759,9 +757,12 @@ int sft_micro_batch(mxopt_engine* e, const std::vector<size_t>& idx, const mxopt
                     mxopt_engine_metrics* out) {
   mxopt_ctx* ctx = e->ctx;
   const size_t n = idx.size();
+  int rc;
+  if (out && e->cfg.has_gradient_clip_norm && e->micro_step + 1 >= acc_steps(e) && (n || e->have_acc) &&
+      (rc = refuse_capture(e)))
+    return rc;
   e->consecutive_nan_count = 0;  // sft/engine.rs:261-267
   if (e->cfg.defer_accumulation) {
-    int rc;
     if (e->held.size() > (size_t)MXOPT_MAX_PENDING && (rc = defer_spill(e))) return rc;
     if ((rc = defer_record(e, idx, grads))) return rc;
     e->held_result.push_back(-1);
@@ -785,7 +786,6 @@ int sft_micro_batch(mxopt_engine* e, const std::vector<size_t>& idx, const mxopt
   const bool boundary = e->micro_step + 1 >= N;
   const bool direct = boundary && first_cycle_step;  // N = 1: no accumulator is needed at all
   std::vector<mxopt_tensor> rows;
-  int rc;
   size_t held = 0;
   for (const Slot& s : e->slots) held += s.in_acc ? 1 : 0;
   for (size_t i = 0; i < n; ++i) {
@@ -1060,8 +1060,10 @@ int mxopt_engine_flush_gradients(mxopt_engine* e, int* flushed, mxopt_engine_met
   }
   mxopt_norm_result h;
   bool measured = false;
-  int rc = e->cfg.defer_accumulation ? sft_apply_deferred(e, e->micro_step, out, &h, &measured)
-                                     : sft_apply(e, e->micro_step, false, out, &h, &measured);
+  int rc = out && e->cfg.has_gradient_clip_norm ? refuse_capture(e) : MXOPT_OK;
+  if (rc) return rc;
+  rc = e->cfg.defer_accumulation ? sft_apply_deferred(e, e->micro_step, out, &h, &measured)
+                                 : sft_apply(e, e->micro_step, false, out, &h, &measured);
   if (rc) return rc;
   if (flushed) *flushed = 1;
   fill_metrics(e, out, 1, 0);

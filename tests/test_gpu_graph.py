@@ -130,10 +130,10 @@ def test_deferred_accumulation_step_replays_from_a_graph():
     ctx.close()
 
 
-@pytest.mark.parametrize("kind", ["grpo", "sft", "sft-16-bit"])
+@pytest.mark.parametrize("kind", ["grpo", "sft", "sft-16-bit", "sft-adamw", "sft-deferred"])
 def test_engine_call_that_waits_is_refused_under_capture(kind):
-    """A micro-batch that hands its norm back cannot be part of a capture.  The call fails in front of the update, and the
-    engine goes on as if it had not been made."""
+    """A micro-batch that hands its norm back cannot be part of a capture.  The call fails before anything is enqueued or
+    booked, and the engine goes on as if it had not been made."""
     import torch
     import mxopt as mx
     rng = np.random.default_rng(9)
@@ -150,7 +150,9 @@ def test_engine_call_that_waits_is_refused_under_capture(kind):
             engines.append(mx.GRPOEngineOptimizerSide(params[-1], learning_rate=0.5, ctx=ctx))
         else:
             engines.append(mx.SFTEngineOptimizerSide(params[-1], learning_rate=0.5, gradient_accumulation_steps=2,
-                                                     accumulate_in_f32=kind == "sft", ctx=ctx))
+                                                     accumulate_in_f32=kind != "sft-16-bit",
+                                                     apply="adamw" if kind == "sft-adamw" else "sgd",
+                                                     defer_accumulation=kind == "sft-deferred", ctx=ctx))
         for _ in range(2 * micro - 1):                # tables, buffers and pinned memory exist; the next call applies
             engines[-1].micro_batch(grads)
     captured, plain = engines
@@ -159,6 +161,9 @@ def test_engine_call_that_waits_is_refused_under_capture(kind):
     with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=stream):
         with pytest.raises(mx.MxoptError, match="waits for the norm"):
             captured.micro_batch(grads)
+        if kind != "grpo":
+            with pytest.raises(mx.MxoptError, match="waits for the norm"):
+                captured.flush_gradients()
     after = captured.metrics()
     for name in ("step", "micro_step", "nan_gradient_count", "consecutive_nan_count"):
         assert getattr(after, name) == getattr(before, name), name
