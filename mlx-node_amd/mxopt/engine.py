@@ -190,7 +190,7 @@ class SFTEngineOptimizerSide(_EngineOptimizerSide):
         flushed = C.c_int()
         m = L.EngineMetrics()
         self._check(self.lib.mxopt_engine_flush_gradients(self.handle, C.byref(flushed), C.byref(m)))
-        self._held = []
+        self._release_held()
         self.last_metrics = m
         return bool(flushed.value)
 
