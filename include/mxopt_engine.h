@@ -94,25 +94,34 @@ int mxopt_engine_new(mxopt_ctx* ctx, const mxopt_engine_config* config, size_t n
 void mxopt_engine_free(mxopt_engine* e);
 
 /* One micro-batch of gradients.
- * GRPO (grpo/engine.rs:561-704): any NaN/Inf element => nothing is touched, the NaN counters
- *   advance, `step` advances, skipped = 1 (status MXOPT_ERR_FAILURE with the reference's
- *   "Training stopped" message once nan_gradient_count reaches max_nan_gradients); otherwise
- *   acc += clip_norm(clamp(g)), and every gradient_accumulation_steps-th accepted micro-batch
- *   p -= (lr/N) * acc.
+ * GRPO (grpo/engine.rs:561-704): any NaN/Inf element => no parameter, moment or accumulated value
+ *   changes, the NaN counters advance, `step` advances, skipped = 1 (status MXOPT_ERR_FAILURE with the
+ *   reference's "Training stopped" message once nan_gradient_count reaches max_nan_gradients);
+ *   otherwise acc += clip_norm(clamp(g)), and every gradient_accumulation_steps-th accepted
+ *   micro-batch p -= (lr/N) * acc.  With apply = SGD everything is enqueued at once, the kernels obey
+ *   the validity flag on the device, and the call waits for the flag last; a skipped one may therefore
+ *   have allocated accumulation buffers or, with defer_accumulation, added the oldest held micro-batches
+ *   into them (which changes no result).  With apply = ADAMW the call waits for the flag first.  A
+ *   call that is refused behind the norm pass (names or dtypes that do not fit a deferred cycle) leaves
+ *   the counters as they were, unless its gradients held a NaN/Inf: then it is that skip.
  * SFT (sft/engine.rs:268-371): acc += g (names the accumulator does not hold are dropped);
  *   every N-th micro-batch p -= lr * (clamp(clip_norm(acc/N)) + wd*p).
  * A gradient whose name is not a parameter is refused before anything is touched with the
  * message of models/qwen3/model.rs:2427-2432 (the reference fails at apply time).  A name given
- * twice counts once, with its first gradient (the reference's maps hold one per name).  A call that
- * hands a norm back (flush_gradients too) waits for it, so it is refused, with nothing applied or booked, while the
- * context's stream is being captured.
+ * twice counts once, with its first gradient (the reference's maps hold one per name).
+ * The kernels read the gradients in stream order: when the call returns -- with metrics too, they only
+ * say that the norm pass has run -- kernels that read this micro-batch's gradients may still be running.
+ * A buffer is freed, rewritten or reused on the context's stream, or ordered after the work that the call
+ * enqueued there (defer_accumulation asks for more, see there).
+ * A call that hands a norm back (flush_gradients too) waits for it, so it is refused, with nothing
+ * applied or booked, while the context's stream is being captured.
  * `out` may be NULL. */
 int mxopt_engine_micro_batch(mxopt_engine* e, size_t n, const char* const* names, const mxopt_array* grads,
                              mxopt_engine_metrics* out);
 
 /* mxopt_engine_micro_batch for the GRPO engine (either apply mode) without its one host synchronisation: the
- * blocking call reads the validity flag back (32 bytes) before it decides whether to accumulate, where
- * the reference reads every gradient back for the same test (grpo/engine.rs:563-569).  Here the flag
+ * blocking call waits for the validity flag (32 bytes; the reference reads every gradient back for the
+ * same test, grpo/engine.rs:563-569).  Here the flag
  * stays on the device: the norm pass writes it, every kernel of the call that would change memory
  * does nothing when it is set, and a copy of it is on its way to pinned host memory when the call
  * returns.  The host books the micro-batch as valid for the time being; the next engine call of any

@@ -65,7 +65,9 @@ class _EngineOptimizerSide:
         L.check(rc, self.ctx.handle)
 
     def micro_batch(self, gradients: Dict[str, torch.Tensor]) -> L.EngineMetrics:
-        """The part of train_step after the backward pass, for one micro-batch of gradients."""
+        """The part of train_step after the backward pass, for one micro-batch of gradients.  Kernels that read them may
+        still be running on the context's stream when this returns.  Where that is not the stream the tensors belong to,
+        the caller records it on them (record_stream); for a deferred cycle this shim does."""
         names = list(gradients)
         cnames = _names(names)
         arrs = _arrs([gradients[nm] for nm in names])

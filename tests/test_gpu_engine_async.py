@@ -243,3 +243,59 @@ def test_async_call_that_fails_after_its_flag_was_requested(mx, kind):
     m = dev.settle()
     assert m.gradients_applied
     check_state(dev, ref, dparams, "end of the cycle")
+
+
+@pytest.mark.parametrize("kind", ["ok", "nan"])
+@pytest.mark.parametrize("wrong", ["names", "dtype"])
+def test_blocking_call_that_fails_behind_its_norm_pass(mx, kind, wrong):
+    """The blocking call enqueues behind the norm pass like the asynchronous one and waits for the flag last.  A deferred
+    micro-batch that is refused there (other names or another dtype than the cycle's) leaves the bookkeeping as it was; if
+    it held a NaN as well, it is the skip that the validity test in front of everything else makes of it."""
+    rng = np.random.default_rng(61)
+    params = make_params(rng, False)
+    dparams = {k: to_dev(v) for k, v in params.items()}
+    kw = dict(learning_rate=0.05, gradient_accumulation_steps=3, gradient_clip_norm=1e9, gradient_clip_value=0.02,
+              max_nan_gradients=50, emergency_save_threshold=3)
+    dev = mx.GRPOEngineOptimizerSide(dparams, defer_accumulation=True, **kw)
+    ref = O.GRPOEngineOptimizerSide(params, **kw)
+    keep = []
+
+    def both(grads):
+        keep.append({k: to_dev(g) for k, g in grads.items()})
+        m = dev.micro_batch(keep[-1])
+        r = ref.micro_batch(grads)
+        assert (bool(m.skipped), bool(m.gradients_applied), m.step) == (r["skipped"], r["gradients_applied"], r["step"])
+
+    both(make_grads(rng, False, 0.01))
+    both(make_grads(rng, False, 0.01))
+    both(poisoned(rng, False, 0, "nan"))              # counters that a failing call could disturb
+    bad = poisoned(rng, False, 1, kind)
+    if wrong == "names":
+        del bad["ln"]
+    keep.append({k: to_dev(O.f32_to_bf16(g) if wrong == "dtype" else g) for k, g in bad.items()})
+    if kind == "nan":
+        m = dev.micro_batch(keep[-1])
+        r = ref.micro_batch(bad)
+        assert m.skipped and r["skipped"] and not m.gradients_applied
+    else:
+        with pytest.raises(mx.InvalidArg, match="same gradient names" if wrong == "names" else "one gradient dtype"):
+            dev.micro_batch(keep[-1])
+    check_state(dev, ref, dparams, "after the refused call")
+    both(make_grads(rng, False, 0.01))                # the cycle goes on and ends
+    assert ref.state.micro_step == 0
+    check_state(dev, ref, dparams, "end of the cycle")
+
+
+def test_blocking_call_that_fails_on_its_last_permitted_nan_stops_the_training(mx):
+    rng = np.random.default_rng(67)
+    params = make_params(rng, False)
+    dparams = {k: to_dev(v) for k, v in params.items()}
+    dev = mx.GRPOEngineOptimizerSide(dparams, defer_accumulation=True, gradient_accumulation_steps=3, max_nan_gradients=1)
+    first = {k: to_dev(g) for k, g in make_grads(rng, False, 0.01).items()}
+    dev.micro_batch(first)
+    bad = poisoned(rng, False, 1, "nan")
+    del bad["ln"]
+    with pytest.raises(mx.TrainingStopped):
+        dev.micro_batch({k: to_dev(g) for k, g in bad.items()})
+    m = dev.metrics()
+    assert (m.nan_gradient_count, m.micro_step, m.step) == (1, 1, 1)
