@@ -131,15 +131,18 @@ __global__ __launch_bounds__(kThreads) void update_kernel(const DevTensor* __res
 // add != 0: g_out = g_out + prep(g) (one float32 add, rounded to g_out's dtype by the store): the
 // engines' "clamp, clip-norm, then accumulate" (grpo/engine.rs:636-661) without materialising the
 // clipped gradient.
-template <int GD, int OD, bool NT, bool ADD, bool WIDE>
+template <int GD, int OD, bool NT, bool ADD>
 __global__ __launch_bounds__(kThreads) void transform_kernel(const DevTensor* __restrict__ T,
                                                              const DevChunk* __restrict__ C, DevTensor one,
                                                              uint32_t nchunks, DevPrep prep) {
   constexpr bool add = ADD;
   // Elements per lane and group: 4 when the kernel adds into g_out (every access then covers whole sectors and
   // streams: the GRPO engine's accumulate of clamp * scale, bf16 into float32, 13.0 against 13.4 ms on the
-  // Qwen3-8B list), 8 when a 16-bit stream stays 16-bit.  Widened, WIDE says which (see launch_transform_t).
-  constexpr int E = ((GD != MXOPT_F32 || OD != MXOPT_F32) && !ADD && (WIDE || OD != MXOPT_F32)) ? 8 : 4;
+  // Qwen3-8B list) and when it writes float32 (a wavefront's store is one contiguous kilobyte; of 16-bit input in
+  // groups of 8 it was every other 16 bytes of two.  bf16, 8 -> 4: 16 M elements 25.1 -> 20.4 us, 63 M 66.4 -> 59.8,
+  // 128 M 137.7 -> 133.9, 256 M 267 -> 266, 600 M 620 -> 627, 1.7 G 1,790 -> 1,799; float16 16 M 25.1 -> 20.4, 256 M
+  // 272 -> 266, 1.7 G 1,832 -> 1,800), 8 when a 16-bit stream stays 16-bit.
+  constexpr int E = (OD != MXOPT_F32 && !ADD) ? 8 : 4;
   constexpr int U = kElemsPerLane / E;
   if (skip_requested(prep)) return;
   const PrepRegs pr = load_prep(prep);
@@ -334,24 +337,15 @@ bool launch_sgd_plain(int pd, int gd, int od, const Launch& L, float lr_p, float
   return false;
 }
 
-// 16-bit into float32: in groups of 4 a wavefront's store is one contiguous kilobyte instead of every other 16 bytes of
-// two.  That is the faster one while the memory-side cache (256 MB) takes a good part of the output, and the slower one
-// of a list so long that memory sets the pace.  bf16, groups of 8 -> 4: 16 M elements 25.2 -> 21.7 us, 63 M 66.5 -> 59.4,
-// 128 M 137 -> 134, 192 - 400 M the same, 600 M 621 -> 626.  The line lies at twice the cache (131 M elements).
-constexpr uint32_t kNarrowChunks = (512u << 20) / (4u * kChunkElems);
-
-template <int GD, int OD, bool ADD, bool WIDE>
-static void launch_transform_nt(const Launch& L, const DevPrep& prep) {
-  if (L.nontemporal) MXOPT_LAUNCH((transform_kernel<GD, OD, true, ADD, WIDE>), L, prep);
-  else MXOPT_LAUNCH((transform_kernel<GD, OD, false, ADD, WIDE>), L, prep);
-}
-
 template <int GD, int OD>
 static void launch_transform_t(const Launch& L, const DevPrep& prep, int add) {
-  constexpr bool kWidens = GD != MXOPT_F32 && OD == MXOPT_F32;
-  if (add) launch_transform_nt<GD, OD, true, true>(L, prep);
-  else if (kWidens && L.nchunks <= kNarrowChunks) launch_transform_nt<GD, OD, false, !kWidens>(L, prep);
-  else launch_transform_nt<GD, OD, false, true>(L, prep);
+  if (L.nontemporal) {
+    if (add) MXOPT_LAUNCH((transform_kernel<GD, OD, true, true>), L, prep);
+    else MXOPT_LAUNCH((transform_kernel<GD, OD, true, false>), L, prep);
+  } else {
+    if (add) MXOPT_LAUNCH((transform_kernel<GD, OD, false, true>), L, prep);
+    else MXOPT_LAUNCH((transform_kernel<GD, OD, false, false>), L, prep);
+  }
 }
 
 template <int GD>

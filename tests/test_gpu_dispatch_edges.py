@@ -128,7 +128,7 @@ def test_descriptors_made_in_c_equal_the_ones_made_in_python(mx):
 
 @pytest.mark.parametrize("n", [1, 7, CHUNK + 3, 32768 * CHUNK, 32768 * CHUNK + 1])
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
-def test_widening_transform_on_both_sides_of_its_line(mx, ctx, n, dtype):
+def test_widening_transform(mx, ctx, n, dtype):
     """A power of two times the gradient: exact, so the reference is the same product in torch."""
     import torch
     dt = torch.bfloat16 if dtype == "bf16" else torch.float16
