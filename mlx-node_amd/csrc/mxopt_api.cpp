@@ -581,7 +581,7 @@ int mxopt::table_retarget_quiet(mxopt_table* t, const mxopt_tensor* tensors, siz
                       (!a.p_out || a.p_out_dtype == b.p_out_dtype) && (!a.g || a.g_dtype == b.g_dtype) &&
                       (!a.g_out || a.g_out_dtype == b.g_out_dtype);
     fill_dev_tensor(b, dev[i]);
-    // The chunk list depends on the head and on which path the tensor takes.
+    // The chunk list depends on the head; whether the streams share their phase decides which pending streams fit.
     if (!same || dev[i].head != t->dev[i].head || ((dev[i].flags ^ t->dev[i].flags) & kTfUnaligned)) {
       *why = "tensor " + std::to_string(i) + " has a different layout";
       return MXOPT_ERR_INVALID_ARG;

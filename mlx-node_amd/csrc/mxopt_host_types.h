@@ -15,7 +15,8 @@ namespace mxopt {
 
 constexpr int kChunkElems = MXOPT_CHUNK_ELEMS;
 constexpr uint32_t kTfFirst = MXOPT_TF_FIRST;
-constexpr uint32_t kTfUnaligned = 0x80000000u;  // set by the table builder: no head aligns every stream
+// Set by the table builder: no head aligns every stream.  For the host's checks (retarget, set_pending); kernels do not read it.
+constexpr uint32_t kTfUnaligned = 0x80000000u;
 constexpr uint32_t kMaxHead = 7;                // a shifted tensor peels at most this many elements
 
 // One per tensor, in device memory.

@@ -588,8 +588,8 @@ void launch_norm_finish(hipStream_t stream, const double* partial_sum, uint32_t 
                        has_max, clip_mode, d_out);
 }
 
-// One result of the second pass copied into pinned host memory by a kernel (a 40-byte store over the
-// bus instead of a copy command): the engines' asynchronous micro-batch call looks at it later.
+// One result of the second pass copied into pinned host memory by a kernel (a 32-byte store over the
+// bus instead of a copy command): the engines look at it behind the update they have enqueued.
 __global__ void mirror_result_kernel(const mxopt_norm_result* __restrict__ src, mxopt_norm_result* __restrict__ dst) {
   *dst = *src;
   __threadfence_system();

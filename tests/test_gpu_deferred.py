@@ -83,11 +83,11 @@ def test_adamw_over_deferred_micro_batches(mx, ctx, combo, k, layout):
     """layout "head": every stream becomes 16-byte aligned after one element (float32 buffers start 12
     bytes, 16-bit buffers 14 bytes past a boundary), so the vector path runs behind a peeled head;
     "elementwise": all buffers start three elements in, the 16-bit and the float32 ones then disagree
-    about the head and the tensor is walked element by element."""
+    about the head and each is accessed at its own phase."""
     pk, gk, xk = combo
     seed = 1000 + 10 * k + len(layout)
     if layout == "elementwise" and pk == gk == "f32" and xk != "f32":
-        pytest.skip("float32 rows keep the vector path; 16-bit pending streams three elements in are rejected")
+        pytest.skip("float32 rows share a phase that 16-bit pending streams three elements in do not have: rejected")
     off = {"aligned": {"f32": 0, "bf16": 0, "f16": 0}, "head": {"f32": 3, "bf16": 7, "f16": 7},
            "elementwise": {"f32": 3, "bf16": 3, "f16": 3}}[layout]
 

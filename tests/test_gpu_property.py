@@ -295,7 +295,7 @@ def test_deferred_accumulation_kernels_match_the_oracle(mx, sizes, k, head, pd, 
     sum's norm; "sgd_plain_each": every stream clamped and clipped by its own norm before the add (the
     GRPO order).  The oracle accumulates into a float32 buffer, micro-batch by micro-batch.  head = h:
     every buffer becomes 16-byte aligned after h elements (vector path behind a peeled head); "mixed":
-    every buffer starts one element in, so 16-bit and float32 streams disagree (element-wise path)."""
+    every buffer starts one element in, so 16-bit and float32 streams disagree about their 16-byte phase."""
     import torch
     rng = np.random.default_rng(seed)
     ctx = mx.default_context()
