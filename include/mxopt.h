@@ -78,7 +78,9 @@ int mxopt_synchronize(mxopt_ctx* ctx);
  * 0 = plain loads and stores; the list kernels of deferred accumulation always stream),
  * "pipelined_norm" (the plain norm of a 16-bit stream: 0 = the general reduction kernel always; 2 (default)
  * or 4 = a kernel that takes that many chunks per trip, for tables whose chunks are under 90 % full on
- * average, i.e. many small tensors; 1 = that kernel, two chunks per trip, for every table). */
+ * average, i.e. many small tensors; 1 = that kernel, two chunks per trip, for every table),
+ * "tiles" (kernels that take 32,768 consecutive elements of a tensor per workgroup: 0 = never, 1 (default) = where a
+ * launch is long enough for them to pay, 2 = wherever they can; same results). */
 int mxopt_set_option(mxopt_ctx* ctx, const char* name, int64_t value);
 int mxopt_get_option(const mxopt_ctx* ctx, const char* name, int64_t* value);
 

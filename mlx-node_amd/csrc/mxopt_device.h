@@ -252,6 +252,16 @@ __device__ __forceinline__ float prep_all(const PrepRegs& r, float g) {
   return g;
 }
 
+// prep_all as straight-line code: an absent stage multiplies by 1 or clamps to +-infinity (make_prep's and load_prep's
+// defaults), which changes no value.
+template <bool kStages>
+__device__ __forceinline__ float prep_branchless(const PrepRegs& r, float g) {
+  if (kStages) g = clamp_keep_nan(g * r.pre_mul, r.pre_lo, r.pre_hi);
+  g = g * r.scale;
+  if (kStages) g = clamp_keep_nan(g, r.post_lo, r.post_hi);
+  return g;
+}
+
 // ---- block reduction: wavefront shuffle -> LDS -> lane 0 ---------------------------
 
 __device__ __forceinline__ double wave_sum(double x) {

@@ -43,6 +43,18 @@ struct DevChunk {
   uint32_t index;   // chunk number inside that tensor; first element = head + index * kChunkElems
 };
 
+// A run of at most kTileChunks consecutive entries of the chunk list, in device memory.  kTileWhole: kTileChunks full
+// chunks of one tensor, the first of them a multiple of kTileChunks.
+constexpr uint32_t kTileChunks = 8;
+constexpr uint64_t kTileElems = (uint64_t)kTileChunks * kChunkElems;
+constexpr uint32_t kTileWhole = 0x80000000u;
+struct DevTile {
+  uint32_t entry;   // first entry, relative to the group's first
+  uint32_t count;   // entries, | kTileWhole
+  uint32_t tensor;  // the first entry's chunk
+  uint32_t index;
+};
+
 constexpr uint32_t kPrepPreMul = 1u, kPrepClampPre = 2u, kPrepClampPost = 4u;
 constexpr uint32_t kPrepPendingOnly = 8u;  // update kernels with a pending gradient: g + prep(g2), not prep(g + g2)
 constexpr uint32_t kPrepEachStream = 16u;  // list kernels: prep every stream (own clip factor), then add
@@ -70,6 +82,8 @@ struct StreamScales {
 struct Group {
   int pd, gd, pod, god;
   uint32_t chunk_begin, nchunks;
+  uint32_t tile_begin = 0, ntiles = 0;  // its tiles
+  uint32_t whole_tiles = 0;
   uint64_t elems = 0;          // elements of the group's tensors (chunks * kChunkElems when every chunk is full)
 };
 
@@ -84,6 +98,7 @@ struct mxopt_ctx {
   int num_cus = 0;
   int grid_blocks_per_cu = 16;  // bounded grids (reductions, accumulation): workgroups per CU
   int persistent = 0;           // update kernels: 0 = one workgroup per chunk, 1 = bounded grid
+  int tiles = 1;                // tiled kernels: 0 never, 1 by their rules, 2 always
   int nontemporal = 1;          // streaming-hint loads/stores in update, transform, accumulate kernels
   int nontemporal_reduce = 1;   // streaming-hint loads in the read-only reduction kernels
   int persistent_accumulate = 0;  // bounded grid also for accumulation passes that take no norm
@@ -108,6 +123,8 @@ struct mxopt_table {
   std::vector<mxopt::Group> groups;
   mxopt::DevTensor* d_tensors = nullptr;
   mxopt::DevChunk* d_chunks = nullptr;
+  mxopt::DevTile* d_tiles = nullptr;          // behind the chunks, in their allocation
+  bool in_place = false;                      // p_out == p in every tensor
   uint64_t total_elems = 0;
   uint64_t num_chunks = 0;
   uint32_t have_mask = 0;                     // which pointers are non-NULL in every non-empty tensor

@@ -2,126 +2,22 @@
 // Every kernel walks a device-side chunk table so that thousands of tensors share one launch; each is
 // a pure streaming pass whose roof is HBM bandwidth.  Build with -ffp-contract=off: one IEEE float32
 // rounding per reference op.
-#include "mxopt_kernels_common.h"
+#include "mxopt_update_tile.h"
 
 namespace mxopt {
 
 // ------------------------------------------------------------------------------------
-// Update kernel.  G2 >= 0: a second gradient stream of that dtype in tensor.g_out is added to g
-// first (one float32 add, rounded to the buffer's dtype GD: the last micro-batch folded into the
-// update instead of being written back to the accumulation buffer).
+// Update kernel, chunk by chunk.
 // ------------------------------------------------------------------------------------
 
 template <int PD, int GD, int OD, int G2, class Math, bool NT>
 __global__ __launch_bounds__(kThreads) void update_kernel(const DevTensor* __restrict__ T,
                                                           const DevChunk* __restrict__ C, DevTensor one,
                                                           uint32_t nchunks, Math math, DevPrep prep) {
-  constexpr bool kHasG2 = G2 >= 0;
-  constexpr int G2D = kHasG2 ? G2 : MXOPT_F32;
-  constexpr bool kSum16 = kHasG2 && GD != MXOPT_F32;  // the sum is what a 16-bit buffer would have held
-  // Elements per lane and group.  With a 16-bit stream in the mix, 8 (one 16-byte access of the 16-bit stream,
-  // two of every float32 stream) when a second gradient stream is folded in, 4 (8-byte accesses of the 16-bit
-  // streams, one 16-byte access of the float32 ones) without: then every access covers whole sectors and can
-  // stream (see load_group).  Measured for bf16 AdamW: no difference on a large list (6.05 against 6.07 ms on
-  // Qwen3-1.7B), 11 % less time on a list that a few passes of the memory-side cache cover (10,000 small tensors,
-  // 2 GB of traffic per step: 0.316 against 0.353 ms) -- accesses that all stream leave a part of the list
-  // resident from one step to the next, plain ones push it out.  With the second stream the wider group wins
-  // (fewer, larger requests for three 16-bit streams): 8 there.
-  constexpr bool kMixed = PD != MXOPT_F32 || GD != MXOPT_F32 || OD != MXOPT_F32 || (kHasG2 && G2D != MXOPT_F32);
-  constexpr int E = (kMixed && kHasG2) ? 8 : 4;
-  constexpr int U = kElemsPerLane / E;
   if (skip_requested(prep)) return;
   const PrepRegs pr = load_prep(prep);
-  const uint32_t tid = threadIdx.x;
-  // The gradient the update sees: prep(g), prep(g + g2) (an accumulation buffer plus the micro-batch
-  // that was not written back to it), or g + prep(g2) (the buffer holds already-clipped gradients and
-  // the pending micro-batch still has to be clipped: grpo/engine.rs:636-661).
-  const bool pending_only = kHasG2 && (pr.flags & kPrepPendingOnly);
-  auto combine = [&](float g, float g2) {
-    if (!kHasG2) return prep_all(pr, g);
-    if (kSum16) return prep_all(pr, Elem<GD>::round(g + g2));
-    return pending_only ? g + prep_all(pr, g2) : prep_all(pr, g + g2);
-  };
-
-  for (uint32_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
-    const ChunkView cv = locate(T, C, one, c);
-    const uint64_t start = cv.start;
-    const uint32_t len = cv.len, flags = cv.t.flags;
-    const float bc1 = cv.t.bc1, bc2 = cv.t.bc2;
-    const void* P = cv.t.p;
-    void* PO = cv.t.p_out;
-    const void* G = cv.t.g;
-    const void* G2P = cv.t.g_out;
-    float* M = cv.t.m;
-    float* V = cv.t.v;
-    const bool use_v = math.uses_v(flags), read_v = math.reads_v(flags);
-    auto one_element = [&](uint64_t off) {
-      float p = Elem<PD>::load(P, off);
-      const float ge = combine(Elem<GD>::load(G, off), kHasG2 ? Elem<G2D>::load(G2P, off) : 0.0f);
-      float m = Math::kM ? Elem<MXOPT_F32>::load(M, off) : 0.0f;
-      float v = read_v ? Elem<MXOPT_F32>::load(V, off) : 0.0f;
-      math(p, ge, m, v, bc1, bc2, flags);
-      Elem<OD>::store(PO, off, p);
-      if (Math::kM) Elem<MXOPT_F32>::store(M, off, m);
-      if (use_v) Elem<MXOPT_F32>::store(V, off, v);
-    };
-
-    if (cv.fast) {
-      // Full chunk: issue every load of the chunk before the first use.
-      float p[U][E], g[U][E], g2[U][E], m[U][E], v[U][E];
-#pragma unroll
-      for (int j = 0; j < U; ++j) {
-        const uint64_t off = start + (uint64_t)(j * kThreads + tid) * E;
-        load_group<PD, E, NT>(P, off, p[j]);
-        load_group<GD, E, NT>(G, off, g[j]);
-        if (kHasG2) load_group<G2D, E, NT>(G2P, off, g2[j]);
-        if (Math::kM) load_group<MXOPT_F32, E, NT>(M, off, m[j]);
-        if (read_v) load_group<MXOPT_F32, E, NT>(V, off, v[j]);
-      }
-#pragma unroll
-      for (int j = 0; j < U; ++j) {
-        if (kSum16) {
-#pragma unroll
-          for (int e = 0; e < E; ++e) g[j][e] = g[j][e] + g2[j][e];
-          round_group<GD, E>(g[j]);
-        }
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-          const float ge = kSum16 ? prep_all(pr, g[j][e]) : combine(g[j][e], g2[j][e]);
-          math(p[j][e], ge, m[j][e], v[j][e], bc1, bc2, flags);
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < U; ++j) {
-        const uint64_t off = start + (uint64_t)(j * kThreads + tid) * E;
-        if (PO == P) store_group<OD, E, NT>(PO, off, p[j]);  // streaming only where the line was read
-        else store_group<OD, E, false>(PO, off, p[j]);
-        if (Math::kM) store_group<MXOPT_F32, E, NT>(M, off, m[j]);
-        if (use_v) store_group<MXOPT_F32, E, NT>(V, off, v[j]);
-      }
-    } else {
-      // Last chunk of a tensor.
-      const uint32_t ngroups = len / E;
-      for (uint32_t q = tid; q < ngroups; q += kThreads) {
-        const uint64_t off = start + (uint64_t)q * E;
-        float p[E], g[E], g2[E], m[E], v[E];
-        load_group<PD, E, false>(P, off, p);
-        load_group<GD, E, false>(G, off, g);
-        if (kHasG2) load_group<G2D, E, false>(G2P, off, g2);
-        if (Math::kM) load_group<MXOPT_F32, E, false>(M, off, m);
-        if (read_v) load_group<MXOPT_F32, E, false>(V, off, v);
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-          math(p[e], combine(g[e], g2[e]), m[e], v[e], bc1, bc2, flags);
-        }
-        store_group<OD, E, false>(PO, off, p);
-        if (Math::kM) store_group<MXOPT_F32, E, false>(M, off, m);
-        if (use_v) store_group<MXOPT_F32, E, false>(V, off, v);
-      }
-      for (uint32_t i = ngroups * E + tid; i < len; i += kThreads) one_element(start + i);
-    }
-    if (tid < cv.head) one_element(tid);  // elements in front of the first aligned group
-  }
+  for (uint32_t c = blockIdx.x; c < nchunks; c += gridDim.x)
+    update_chunk<PD, GD, OD, G2, Math, NT>(locate(T, C, one, c), threadIdx.x, math, pr);
 }
 
 // ------------------------------------------------------------------------------------
@@ -212,6 +108,9 @@ __global__ __launch_bounds__(kThreads) void transform_kernel(const DevTensor* __
 
 template <int PD, int GD, int OD, int G2, class Math>
 static void launch_update_t(const Launch& L, const Math& math, const DevPrep& prep) {
+  if constexpr (OD == PD) {
+    if (launch_update_tiles<PD, GD, G2>(L, math, prep)) return;
+  }
   if (L.nontemporal)
     MXOPT_LAUNCH((update_kernel<PD, GD, OD, G2, Math, true>), L, math, prep);
   else

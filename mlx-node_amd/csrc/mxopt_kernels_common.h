@@ -25,16 +25,22 @@ __device__ __forceinline__ float round_square_to(int dtype, float sq) {
 struct AdamMath {
   mxopt_adam_hp hp;
   int gsq_dtype = MXOPT_F32;  // dtype the square of the gradient is rounded to (adamw.rs:92, adam.rs:88)
-  static constexpr bool kM = true;
+  static constexpr bool kM = true, kV = true, kSquare = true;
   __device__ __forceinline__ bool uses_v(uint32_t) const { return true; }
   __device__ __forceinline__ bool reads_v(uint32_t) const { return true; }
+  __device__ __forceinline__ bool rounds_square() const { return gsq_dtype != MXOPT_F32; }
+  __device__ __forceinline__ float squared(float, float g) const { return g; }
   __device__ __forceinline__ void operator()(float& p, float g, float& m, float& v, float bc1, float bc2,
-                                             uint32_t) const {
+                                             uint32_t flags) const {
+    apply(p, g, m, v, bc1, bc2, flags, round_square_to(gsq_dtype, g * g));
+  }
+  // gsq: the square of squared(p, g), rounded to gsq_dtype.
+  __device__ __forceinline__ void apply(float& p, float g, float& m, float& v, float bc1, float bc2, uint32_t,
+                                        float gsq) const {
     float pd = hp.decoupled_decay ? p * hp.decay : p;
     float b1m = m * hp.beta1;
     float g1 = g * hp.one_minus_beta1;
     float nm = b1m + g1;
-    float gsq = round_square_to(gsq_dtype, g * g);
     float b2v = v * hp.beta2;
     float g2 = gsq * hp.one_minus_beta2;
     float nv = b2v + g2;
@@ -52,11 +58,15 @@ struct AdamMath {
 // SGD::update_single (optimizers/sgd.rs:84-150).
 struct SgdMath {
   mxopt_sgd_hp hp;
-  static constexpr bool kM = false;
+  static constexpr bool kM = false, kV = true, kSquare = false;
   __device__ __forceinline__ bool uses_v(uint32_t) const { return hp.has_momentum != 0; }
   __device__ __forceinline__ bool reads_v(uint32_t flags) const { return hp.has_momentum && !(flags & kTfFirst); }
-  __device__ __forceinline__ void operator()(float& p, float g, float&, float& v, float, float,
+  __device__ __forceinline__ bool rounds_square() const { return false; }
+  __device__ __forceinline__ void operator()(float& p, float g, float& m, float& v, float bc1, float bc2,
                                              uint32_t flags) const {
+    apply(p, g, m, v, bc1, bc2, flags, 0.0f);
+  }
+  __device__ __forceinline__ void apply(float& p, float g, float&, float& v, float, float, uint32_t flags, float) const {
     float ge = g;
     if (hp.has_weight_decay) {
       float w = p * hp.weight_decay;
@@ -84,16 +94,25 @@ struct SgdMath {
 struct RmspropMath {
   mxopt_rmsprop_hp hp;
   int gsq_dtype = MXOPT_F32;  // as in AdamMath (rmsprop.rs:80)
-  static constexpr bool kM = false;
+  static constexpr bool kM = false, kV = true, kSquare = true;
   __device__ __forceinline__ bool uses_v(uint32_t) const { return true; }
   __device__ __forceinline__ bool reads_v(uint32_t) const { return true; }
-  __device__ __forceinline__ void operator()(float& p, float g, float&, float& v, float, float, uint32_t) const {
+  __device__ __forceinline__ bool rounds_square() const { return gsq_dtype != MXOPT_F32; }
+  __device__ __forceinline__ float squared(float p, float g) const {
     float ge = g;
     if (hp.has_weight_decay) {
       float w = p * hp.weight_decay;
       ge = g + w;
     }
-    float gsq = round_square_to(gsq_dtype, ge * ge);
+    return ge;
+  }
+  __device__ __forceinline__ void operator()(float& p, float g, float& m, float& v, float bc1, float bc2,
+                                             uint32_t flags) const {
+    const float ge = squared(p, g);
+    apply(p, g, m, v, bc1, bc2, flags, round_square_to(gsq_dtype, ge * ge));
+  }
+  __device__ __forceinline__ void apply(float& p, float g, float&, float& v, float, float, uint32_t, float gsq) const {
+    const float ge = squared(p, g);
     float av = v * hp.alpha;
     float g2 = gsq * hp.one_minus_alpha;
     float nv = av + g2;
@@ -112,10 +131,15 @@ template <int PD, bool ROUND_PRODUCT>
 struct PlainSgdMath {
   float lr_p, weight_decay;
   int has_weight_decay;
-  static constexpr bool kM = false;
+  static constexpr bool kM = false, kV = false, kSquare = false;
   __device__ __forceinline__ bool uses_v(uint32_t) const { return false; }
   __device__ __forceinline__ bool reads_v(uint32_t) const { return false; }
-  __device__ __forceinline__ void operator()(float& p, float g, float&, float&, float, float, uint32_t) const {
+  __device__ __forceinline__ bool rounds_square() const { return false; }
+  __device__ __forceinline__ void operator()(float& p, float g, float& m, float& v, float bc1, float bc2,
+                                             uint32_t flags) const {
+    apply(p, g, m, v, bc1, bc2, flags, 0.0f);
+  }
+  __device__ __forceinline__ void apply(float& p, float g, float&, float&, float, float, uint32_t, float) const {
     float ge = g;
     if (has_weight_decay) {  // sft/engine.rs:345-365: g + f32(wd)*p, promoted to float32
       float w = p * weight_decay;

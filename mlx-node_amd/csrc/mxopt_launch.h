@@ -18,6 +18,13 @@ struct Launch {
   DevTensor one{};
   uint32_t nchunks = 0;
   uint32_t grid = 0;                 // workgroups (<= nchunks)
+  // The launch cut into tiles (none when ntiles is 0): with a chunk list by `tiles`; tile i of a single tensor are its
+  // chunks [i * kTileChunks, ...).  Whether a kernel takes them depends on tiles_per_cu, the whole tiles that the launch's
+  // elements would make for each compute unit.
+  const DevTile* tiles = nullptr;
+  uint32_t ntiles = 0;
+  uint32_t tiles_per_cu = 0;
+  bool in_place = false;             // p_out == p in every tensor
   hipStream_t stream = nullptr;
   int nontemporal = 1;               // non-zero: streaming-hint loads and stores
   int pipelined_norm = 2;            // plain 16-bit norms take the software-pipelined kernel

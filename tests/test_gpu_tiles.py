@@ -1,0 +1,222 @@
+"""GPU: kernels that work tile by tile (option "tiles" = 2) against the same entry points chunk by chunk (0), bit for bit, at
+the edges of tiles, over every type, order of stages and alignment that the entry points take."""
+import itertools
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+TILE = 32768
+# one element, the edges of a chunk, of a tile and of several, and many small tensors between large ones
+SIZES = [1, 5, 4095, 4096, TILE - 1, TILE, 3, TILE + 1, 2 * TILE + 4099, 100, 100, 100, 4097, 100, 3 * TILE, 7, TILE + 3 * 4096]
+LAYOUTS = ["apart", "packed", "shifted", "phases"]
+
+
+@pytest.fixture(scope="module")
+def mx():
+    import torch
+    import mxopt
+    assert torch.cuda.is_available()
+    return mxopt
+
+
+@pytest.fixture(scope="module")
+def ctx(mx):
+    c = mx.Context()
+    yield c
+    c.close()
+
+
+def views(slab, layout, stream):
+    """SIZES as views of one slab: each at a multiple of 64 elements, back to back, 3 elements behind a multiple, or 3 + stream."""
+    out, at = [], 0
+    for n in SIZES:
+        lead = {"apart": 0, "packed": 0, "shifted": 3, "phases": 3 + stream}[layout]
+        out.append(slab[at + lead:at + lead + n])
+        at += n if layout == "packed" else -(-(n + 16) // 64) * 64
+    return out
+
+
+SLAB = sum(-(-(n + 16) // 64) * 64 for n in SIZES) + 64
+
+
+def slab(torch, dtype, gen, std, square=False):
+    x = torch.empty(SLAB, dtype=dtype, device="cuda").normal_(0.0, std, generator=gen)
+    return x.square_() if square else x
+
+
+def bits(torch, t):
+    return t.view(torch.int32 if t.element_size() == 4 else torch.int16)
+
+
+def run_both(torch, mx, ctx, streams, layout, call):
+    """call(table rows' streams) with tiles off and on, over copies of the same slabs; whole slabs compared."""
+    results = []
+    for tiles in (0, 2):
+        own = {k: s.clone() for k, s in streams.items()}
+        v = {k: views(s, layout, i) for i, (k, s) in enumerate(own.items())}
+        rows = []
+        for i in range(len(SIZES)):
+            row = {k: v[k][i] for k in v}
+            if "p" in row:
+                row["p_out"] = row["p"]
+            rows.append(mx.TensorSpec(**row))
+        ctx.set_option("tiles", tiles)
+        try:
+            call(ctx.table(rows))
+        finally:
+            ctx.set_option("tiles", 1)
+        results.append(own)
+    torch.cuda.synchronize()
+    for k in streams:
+        a, b = bits(torch, results[0][k]), bits(torch, results[1][k])
+        assert torch.equal(a, b), (k, int((a != b).sum()), int((a != b).nonzero()[0]))
+    assert any(not torch.equal(bits(torch, results[0][k]), bits(torch, streams[k])) for k in streams)
+
+
+def preps(mx, res):
+    return {"none": None, "scale": mx.make_prep(scale=res), "mul": mx.make_prep(pre_mul=0.5),
+            "grpo": mx.make_prep(clamp_pre=(-0.8e-3, 0.9e-3), scale=res),
+            "all": mx.make_prep(pre_mul=0.75, clamp_pre=(-1e-3, float("inf")), scale=res, clamp_post=(-4e-4, 5e-4))}
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("pd,gd", list(itertools.product(["float32", "bfloat16", "float16"], repeat=2)))
+def test_updates(mx, ctx, pd, gd, layout):
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(1)
+    PD, GD, F = getattr(torch, pd), getattr(torch, gd), torch.float32
+    p, g = slab(torch, PD, gen, 0.5), slab(torch, GD, gen, 1e-3)
+    g[5], g[70000], g[130001] = float("nan"), float("inf"), -0.0
+    m, v = slab(torch, F, gen, 1e-3), slab(torch, F, gen, 1e-3, square=True)
+    res = ctx.norm_result()
+    finite = torch.full((1000,), 0.1, device="cuda")
+    ctx.global_norm(ctx.table([mx.TensorSpec(g=finite)]), res, max_norm=1.0)  # a clip factor under 1
+    for name, prep in preps(mx, res).items():
+        for hp in (mx.adam_hp(1e-2, 0.9, 0.999, 1e-8, 0.01), mx.adam_hp(1e-2, 0.9, 0.999, 1e-8, None)):
+            run_both(torch, mx, ctx, dict(p=p, g=g, m=m, v=v), layout, lambda t: ctx.adam(t, hp, prep))
+        for hp in (mx.sgd_hp(0.1, 0.9, 0.01), mx.sgd_hp(0.1, 0.9, 0.0, nesterov=True), mx.sgd_hp(0.1, 0.0, 0.01)):
+            run_both(torch, mx, ctx, dict(p=p, g=g, v=v), layout, lambda t: ctx.sgd(t, hp, prep))
+        for wd in (0.0, 0.01):
+            run_both(torch, mx, ctx, dict(p=p, g=g, v=v), layout, lambda t: ctx.rmsprop(t, mx.rmsprop_hp(1e-2, 0.99, 1e-8, wd), prep))
+            run_both(torch, mx, ctx, dict(p=p, g=g), layout, lambda t: ctx.sgd_plain(t, 0.3, wd, prep))
+
+
+@pytest.mark.parametrize("layout", ["apart", "shifted", "phases"])
+@pytest.mark.parametrize("pd,xd", list(itertools.product(["float32", "bfloat16", "float16"], repeat=2)))
+def test_updates_with_a_pending_gradient(mx, ctx, pd, xd, layout):
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(2)
+    PD, XD, F = getattr(torch, pd), getattr(torch, xd), torch.float32
+    p, g, x = slab(torch, PD, gen, 0.5), slab(torch, F, gen, 1e-3), slab(torch, XD, gen, 1e-3)
+    m, v = slab(torch, F, gen, 1e-3), slab(torch, F, gen, 1e-3, square=True)
+    res = ctx.norm_result()
+    ctx.global_norm(ctx.table([mx.TensorSpec(g=torch.full((1000,), 0.1, device="cuda"))]), res, max_norm=1.0)
+    hp = mx.adam_hp(1e-2, 0.9, 0.999, 1e-8, 0.01)
+    for name, prep in preps(mx, res).items():
+        run_both(torch, mx, ctx, dict(p=p, g=g, g_out=x, m=m, v=v), layout, lambda t: ctx.adam_with_pending(t, hp, prep))
+        for covers in (0, 1):
+            run_both(torch, mx, ctx, dict(p=p, g=g, g_out=x), layout,
+                     lambda t: ctx.sgd_plain_with_pending(t, 0.3, 0.01, prep, prep_covers_sum=covers))
+
+
+def test_first_step_of_sgd_and_a_skipped_step(mx, ctx):
+    """SGD's first step does not read the velocity; a step with an invalid gradient changes nothing."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(3)
+    F = torch.float32
+    p, g, v = slab(torch, F, gen, 0.5), slab(torch, F, gen, 1e-3), slab(torch, F, gen, 1.0)
+    v[::7] = float("nan")
+
+    def first(t):
+        t.set_step_scalars(flags=[mx.TF_FIRST] * len(SIZES))
+        ctx.sgd(t, mx.sgd_hp(0.1, 0.9, 0.01), None)
+    run_both(torch, mx, ctx, dict(p=p, g=g, v=v), "apart", first)
+
+    g[TILE] = float("inf")
+    table = [mx.TensorSpec(p=p, p_out=p, g=g)]
+    res = ctx.norm_result()
+    ctx.global_norm(ctx.table([mx.TensorSpec(g=g)]), res, max_norm=1.0)
+    before = p.clone()
+    ctx.set_option("tiles", 2)
+    try:
+        ctx.sgd_plain(ctx.table(table), 0.3, 0.0, mx.make_prep(scale=res, skip_if_nonfinite=res))
+    finally:
+        ctx.set_option("tiles", 1)
+    assert torch.equal(bits(torch, p), bits(torch, before))
+
+
+@pytest.mark.parametrize("n", [1, 4095, TILE - 1, TILE, TILE + 1, 5 * TILE + 4096 + 3])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_single_tensor(mx, ctx, n, shift):
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(4)
+    base = torch.empty(n + 8, device="cuda").normal_(0.0, 0.5, generator=gen)
+    g = torch.empty(n + 8, device="cuda").normal_(0.0, 1e-3, generator=gen)
+    outs = []
+    for tiles in (0, 2):
+        p = base.clone()
+        opt = mx.AdamW(1e-2, weight_decay=0.01, ctx=ctx)
+        ctx.set_option("tiles", tiles)
+        try:
+            for _ in range(2):
+                opt.update_single("w", p[shift:shift + n], g[shift:shift + n], out=p[shift:shift + n])
+        finally:
+            ctx.set_option("tiles", 1)
+        outs.append(p)
+    assert torch.equal(bits(torch, outs[0]), bits(torch, outs[1])) and not torch.equal(outs[0], base)
+
+
+def test_rule_takes_tiles_for_long_lists_only(mx, ctx):
+    """The default rule on both sides of its line gives the results of either route."""
+    import torch
+    for n in (TILE * ctx.get_option("num_cus") * 2 - 5, TILE * ctx.get_option("num_cus") * 2 + 5):
+        gen = torch.Generator(device="cuda")
+        gen.manual_seed(5)
+        p = torch.empty(n, device="cuda").normal_(0.0, 0.5, generator=gen)
+        g = torch.empty(n, device="cuda").normal_(0.0, 1e-3, generator=gen)
+        v = torch.zeros(n, device="cuda")
+        outs = []
+        for tiles in (0, 1):
+            own = [p.clone(), g, v.clone()]
+            ctx.set_option("tiles", tiles)
+            try:
+                ctx.sgd(ctx.table([mx.TensorSpec(p=own[0], p_out=own[0], g=own[1], v=own[2])]), mx.sgd_hp(0.1, 0.9, 0.01), None)
+            finally:
+                ctx.set_option("tiles", 1)
+            outs.append(own)
+        assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][2], outs[1][2])
+
+
+@pytest.mark.parametrize("kind,defer", [("grpo", False), ("sft", False), ("sft", True)])
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16", "float32"])
+def test_engines(mx, ctx, kind, defer, dtype):
+    """The engines' updates: plain SGD behind the norm, and with the last micro-batch folded in (into 16-bit sums too)."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(6)
+    D = getattr(torch, dtype)
+    names = ["w%d" % i for i in range(len(SIZES))]
+    base = slab(torch, D, gen, 0.5)
+    grads = [views(slab(torch, D, gen, 0.1), "apart", 0) for _ in range(3)]
+    outs = []
+    for tiles in (0, 2):
+        p = base.clone()
+        params = dict(zip(names, views(p, "apart", 0)))
+        ctx.set_option("tiles", tiles)
+        try:
+            if kind == "grpo":
+                engine = mx.GRPOEngineOptimizerSide(params, learning_rate=1.0, gradient_accumulation_steps=1, ctx=ctx)
+            else:
+                engine = mx.SFTEngineOptimizerSide(params, learning_rate=1.0, gradient_accumulation_steps=3, weight_decay=0.01,
+                                                   accumulate_in_f32=defer, defer_accumulation=False, ctx=ctx)
+            for g in grads:
+                engine.micro_batch(dict(zip(names, g)))
+        finally:
+            ctx.set_option("tiles", 1)
+        outs.append(p)
+    assert torch.equal(bits(torch, outs[0]), bits(torch, outs[1])) and not torch.equal(outs[0], base)
