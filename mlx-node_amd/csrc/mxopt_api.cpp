@@ -164,6 +164,8 @@ Launch make_launch(const mxopt_ctx* ctx, const mxopt_table* t, const Group& g, b
   L.nontemporal = ctx->nontemporal;
   L.pipelined_norm = ctx->pipelined_norm;
   L.partial_chunks = g.elems * 10 < (uint64_t)g.nchunks * kChunkElems * 9;
+  L.elems = g.elems;
+  L.num_cus = (uint32_t)ctx->num_cus;
   return L;
 }
 
@@ -236,6 +238,7 @@ static int run_sumsq(mxopt_ctx* ctx, const mxopt_table* t, int mode, int first, 
     // take no norm follow the update kernels' launch policy (one workgroup per chunk: 6.12 against
     // 6.04 TB/s for acc += g on region-interleaved memory).
     Launch L = make_launch(ctx, t, g, want || mode != 2 || ctx->persistent != 0 || (ctx->persistent_accumulate != 0 && !first));
+    if (mode == 2 && !want && ctx->persistent_accumulate == 0) offer_tiles(ctx, L, t->d_tiles + g.tile_begin, g.ntiles, g.whole_tiles, g.elems);
     if (L.grid < g.nchunks) L.grid = reduction_grid(g);  // a bounded grid: the size this reduction wants
     if (mode != 2) L.nontemporal = ctx->nontemporal_reduce;
     const int ad = mode == 0 ? g.gd : g.god;
@@ -321,6 +324,8 @@ Launch make_single_launch(const mxopt_ctx* ctx, const mxopt_tensor& t, bool pers
               (uint32_t)((L.one.n - L.one.head) / kTileElems), L.one.n);
   L.in_place = t.p == t.p_out;
   L.partial_chunks = L.one.n * 10 < (uint64_t)L.nchunks * kChunkElems * 9;
+  L.elems = L.one.n;
+  L.num_cus = (uint32_t)ctx->num_cus;
   return L;
 }
 

@@ -212,6 +212,29 @@ __device__ __forceinline__ float norm_value(const PrepRegs& pr, float x, bool cl
   return __builtin_amdgcn_fmed3f(x, pr.pre_lo, pr.pre_hi);
 }
 
+// How many workgroups of a launch share a compute unit.  The passes that read and write long lists run at 5.3 - 5.7 TB/s in memory
+// of one region with as many as the registers allow, and at 6.1 - 6.5 with fewer, as many as keep some 64 - 100 KB of reads a unit in
+// flight: what is in flight, and what is written behind it, then lies in fewer places at a time, and the memory turns from
+// reading to writing less often.  Too few leave it waiting; each launcher says what it measured.
+struct Crowd {
+  int per_cu;         // workgroups (of kThreads) per compute unit
+  int fill;           // only where the chunks are at least this full on average, in per cent (short chunks need company), and
+  int chunks_per_cu;  // only where the launch has at least this many for each compute unit
+};
+constexpr Crowd kNoLimit{0, 0, 0};
+
+// Dynamic LDS that leaves room for crowd.per_cu workgroups: an equal part of a compute unit's 160 KB in units of its allocation
+// (1,280 bytes), one unit less for what a kernel declares itself.
+inline uint32_t crowd_lds(const Launch& L, Crowd crowd) {
+  if (crowd.per_cu == 0 || (uint64_t)L.nchunks < (uint64_t)crowd.chunks_per_cu * L.num_cus ||
+      L.elems * 100u < (uint64_t)L.nchunks * kChunk * (uint32_t)crowd.fill)
+    return 0;
+  return ((163840u / (uint32_t)crowd.per_cu) / 1280u - 1u) * 1280u;
+}
+
+#define MXOPT_LAUNCH_CROWD(kernel, crowd, L, ...)                                                                        \
+  hipLaunchKernelGGL(kernel, dim3((L).grid), dim3(kThreads), crowd_lds(L, crowd), (L).stream, (L).tensors, (L).chunks, \
+                     (L).one, (L).nchunks, __VA_ARGS__)
 #define MXOPT_LAUNCH(kernel, L, ...)                                                                          \
   hipLaunchKernelGGL(kernel, dim3((L).grid), dim3(kThreads), 0, (L).stream, (L).tensors, (L).chunks, (L).one, \
                      (L).nchunks, __VA_ARGS__)

@@ -19,8 +19,8 @@ struct Launch {
   uint32_t nchunks = 0;
   uint32_t grid = 0;                 // workgroups (<= nchunks)
   // The launch cut into tiles (none when ntiles is 0): with a chunk list by `tiles`; tile i of a single tensor are its
-  // chunks [i * kTileChunks, ...).  Whether a kernel takes them depends on tiles_per_cu, the whole tiles that the launch's
-  // elements would make for each compute unit.
+  // chunks [i * kTileChunks, ...).  Whether a kernel takes them depends on tiles_per_cu, the whole tiles there are for each
+  // compute unit.
   const DevTile* tiles = nullptr;
   uint32_t ntiles = 0;
   uint32_t tiles_per_cu = 0;
@@ -29,6 +29,8 @@ struct Launch {
   int nontemporal = 1;               // non-zero: streaming-hint loads and stores
   int pipelined_norm = 2;            // plain 16-bit norms take the software-pipelined kernel
   bool partial_chunks = false;       // the chunks are under 90 % full on average (many small tensors)
+  uint64_t elems = 0;                // elements of the launch
+  uint32_t num_cus = 1;
   // Deferred accumulation (the *_list launchers): stream j of table row r is pending[j * ntensors + r].
   const void* const* pending = nullptr;
   uint32_t ntensors = 0;

@@ -3,7 +3,7 @@
 #include <mutex>
 #include <type_traits>
 
-#include "mxopt_kernels_common.h"
+#include "mxopt_tiles.h"
 #include "mxopt_gauss_table.h"
 
 namespace mxopt {
@@ -26,10 +26,11 @@ __device__ __forceinline__ float accumulate_op(float acc, float g, bool first) {
   return Elem<AD>::round(s);
 }
 
-template <int MODE, int AD, int GD, bool NT>
+// GROUP: elements per lane and group, 0 = the mode's own.
+template <int MODE, int AD, int GD, bool NT, int GROUP = 0>
 struct SumsqChunk {
   static constexpr bool kTwoStreams = MODE >= 2;
-  static constexpr int E = (AD != MXOPT_F32 || (kTwoStreams && GD != MXOPT_F32)) ? 8 : 4;
+  static constexpr int E = GROUP ? GROUP : (AD != MXOPT_F32 || (kTwoStreams && GD != MXOPT_F32)) ? 8 : 4;
   static constexpr int U = kElemsPerLane / E;
   float x[U][E], g[U][E];
 
@@ -57,11 +58,11 @@ struct SumsqChunk {
   // The new sum of group j.  A streaming store pays off where the pass has just read the line it writes; the
   // first pass of a cycle writes lines nobody read (acc = widen(g)), and there streaming stores cost 60 % more
   // time (measured on the bf16 -> float32 pass, whose float32 stores come in sector-sharing pairs that
-  // store_group no longer streams anyway; single-piece stores were not measured on their own).
+  // store_group no longer streams anyway).  A later pass into another buffer than it reads is no different.
   static __device__ __forceinline__ void store_sum(const ChunkView& cv, uint32_t tid, int j, bool first,
                                                    const float (&v)[E]) {
     const uint64_t off = cv.start + (uint64_t)(j * kThreads + tid) * E;
-    if (first) store_group<AD, E, false>(cv.t.g_out, off, v);
+    if (first || (cv.t.p != nullptr && cv.t.p != cv.t.g_out)) store_group<AD, E, false>(cv.t.g_out, off, v);
     else store_group<AD, E, NT>(cv.t.g_out, off, v);
   }
 
@@ -147,6 +148,18 @@ struct SumsqChunk {
     }
   }
 
+  // The whole chunk, MODE 2 without the norm.
+  static __device__ __forceinline__ void accumulate(const ChunkView& cv, const PrepRegs& pr, uint32_t tid, bool first) {
+    if (cv.fast) {
+      SumsqChunk k;
+      k.load(cv, tid, first);
+      k.finish_store_only(cv, tid, first);
+    } else {
+      (void)slow(cv, pr, tid, first);
+    }
+    if (tid < cv.head) (void)one_element(cv, pr, tid, first, 0.0f);
+  }
+
   // Partial chunk.
   static __device__ __forceinline__ float slow(const ChunkView& cv, const PrepRegs& pr, uint32_t tid, bool first) {
     const void* X = squared_stream(cv);
@@ -208,20 +221,6 @@ __global__ __launch_bounds__(kThreads) void sumsq_kernel(const DevTensor* __rest
   double acc_sum = 0.0;
 
   uint32_t c = blockIdx.x;
-  if (MODE == 2 && partial_sum == nullptr) {  // accumulation only
-    for (; c < nchunks; c += gridDim.x) {
-      const ChunkView cv = locate(T, C, one, c);
-      if (cv.fast) {
-        Chunk k;
-        k.load(cv, tid, first);
-        k.finish_store_only(cv, tid, first);
-      } else {
-        (void)Chunk::slow(cv, pr, tid, first);
-      }
-      if (tid < cv.head) (void)Chunk::one_element(cv, pr, tid, first, 0.0f);
-    }
-    return;
-  }
   for (; c < nchunks; c += gridDim.x) {
     const ChunkView cv = locate(T, C, one, c);
     float s;
@@ -269,13 +268,91 @@ __global__ __launch_bounds__(kThreads) void sumsq_kernel(const DevTensor* __rest
     acc_sum += (double)s;
   }
 
-  if (partial_sum != nullptr) {
-    unsigned long long unused = 0;
-    block_sum(acc_sum, unused);
-    if (tid == 0) partial_sum[blockIdx.x] = acc_sum;
-  }
+  unsigned long long unused = 0;
+  block_sum(acc_sum, unused);
+  if (tid == 0) partial_sum[blockIdx.x] = acc_sum;
 }
 
+// Accumulation that is not asked for the norm.  The first pass of a cycle writes lines nobody read, in groups of 8 where a
+// stream has 16 bits (of 1.72 G elements in 1,608 us, in groups of 4 in 1,857); later passes read what they write and take
+// groups of 4, so that every access is one that streams (see load_group).  Later passes, microseconds in groups of 8 and of 4:
+// bf16 into float32 1.72 G elements 3,103 and 2,972, 10,000 tensors of 64 - 65,536 179 and 150; bf16 into bf16 596 M 654 and
+// 600, the 10,000 tensors 115 and 92.
+template <int AD, int GD, bool NT, bool FIRST>
+__global__ __launch_bounds__(kThreads) void accumulate_kernel(const DevTensor* __restrict__ T, const DevChunk* __restrict__ C,
+                                                              DevTensor one, uint32_t nchunks, DevPrep prep) {
+  using Chunk = SumsqChunk<2, AD, GD, NT, FIRST ? 0 : 4>;
+  const PrepRegs pr = load_prep(prep);
+  for (uint32_t c = blockIdx.x; c < nchunks; c += gridDim.x) Chunk::accumulate(locate(T, C, one, c), pr, threadIdx.x, FIRST);
+}
+
+// Later passes into float32 by tiles (mxopt_tiles.h).  Microseconds in groups of 4 by chunks and by tiles: a bf16 gradient,
+// 128 M elements (16 tiles per compute unit) 214 and 218, 256 M 439 and 433, 430 M 727 and 706, 596 M 1,014 and 987, 1.72 G 2,984
+// and 2,809; a float32 one, 8 M (1 tile) 22 and 21, 64 M 147 and 131, 596 M 1,293 and 1,134.  16-bit sums gain nothing (596 M
+// 587 and 579, 1.72 G 1,737 and 1,748) and keep the chunks.
+template <int GD>
+__global__ __launch_bounds__(kTileThreads) void accumulate_tile_kernel(const DevTensor* __restrict__ T,
+                                                                       const DevChunk* __restrict__ C, DevTensor one,
+                                                                       uint32_t nchunks, const DevTile* __restrict__ tiles,
+                                                                       DevPrep prep) {
+  constexpr int AD = MXOPT_F32;
+  using Chunk = SumsqChunk<2, AD, GD, true, 4>;
+  constexpr int U = kTileChunks;
+  const uint32_t tid = threadIdx.x;
+  const TileView tv = this_tile(T, one, nchunks, tiles);
+  if (!tv.whole || (tv.t.p != nullptr && tv.t.p != tv.t.g_out)) {  // into another buffer the stores must not stream (see store_sum)
+    const PrepRegs pr = load_prep(prep);
+    chunks_of_tile(T, C, one, tv.tile, [&](const ChunkView& cv, uint32_t lane) { Chunk::accumulate(cv, pr, lane, false); });
+    return;
+  }
+  const uint64_t first = tv.t.head + (uint64_t)tv.tile.index * kChunk;
+  const void* A = tv.t.p != nullptr ? tv.t.p : tv.t.g_out;
+  typename Piece<AD>::T a[U];
+  typename Piece<GD>::T g[U];
+  MXOPT_ROWS g[j] = load_piece<GD, true>(tv.t.g, first + j * kChunk, tid);
+  MXOPT_ROWS a[j] = load_piece<AD, true>(A, first + j * kChunk, tid);
+  MXOPT_ROWS {
+    pin(a[j]); pin(g[j]);
+    float xa[4], xg[4];
+    Piece<AD>::unpack(a[j], xa);
+    Piece<GD>::unpack(g[j], xg);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) xa[e] = xa[e] + xg[e];
+    a[j] = Piece<AD>::pack(xa);
+    pin(a[j]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  MXOPT_ROWS store_piece<AD, true>(tv.t.g_out, first + j * kChunk, tid, a[j]);
+  if (tv.tile.index == 0 && tid < tv.t.head)  // elements in front of the first aligned group
+    (void)Chunk::one_element(locate(T, C, one, tv.tile.entry), load_prep(prep), tid, false, 0.0f);
+}
+
+// Microseconds without a limit and with it.  First pass: 16-bit into float32 32 M elements 41 and 40, 128 M 146 and 133, 1.72 G
+// 1,908 and 1,598; into 16 bits 128 M 92 and 87, 596 M 421 and 372 (32 M 27 and 28; 10,000 tensors of 64 - 65,536 74 and 80);
+// float32 128 M 189 and 172, 256 M 379 and 335.  Later passes: 16-bit into float32, the 10,000 tensors 149 and 139; into 16 bits 128 M
+// 129 and 127, 256 M 263 and 251, 596 M 595 and 570 (the 10,000 tensors 85 and 91).
+template <int AD, int GD, bool FIRST>
+constexpr Crowd kAccumulateCrowd =
+    AD != MXOPT_F32 ? (FIRST ? Crowd{5, 90, 128} : Crowd{4, 90, 128})
+                    : GD != MXOPT_F32 ? (FIRST ? Crowd{5, 75, 16} : Crowd{4, 75, 16}) : (FIRST ? Crowd{2, 75, 16} : kNoLimit);
+
+template <int AD, int GD>
+static void launch_accumulate(const Launch& L, const DevPrep& prep, int first) {
+  if constexpr (AD == MXOPT_F32) {
+    if (!first && L.ntiles != 0 && L.tiles_per_cu >= (GD == MXOPT_F32 ? 2u : 32u)) {
+      hipLaunchKernelGGL(accumulate_tile_kernel<GD>, dim3(L.ntiles), dim3(kTileThreads), kOnePerCu, L.stream, L.tensors,
+                         L.chunks, L.one, L.nchunks, L.tiles, prep);
+      return;
+    }
+  }
+  if (L.nontemporal) {
+    if (first) MXOPT_LAUNCH_CROWD((accumulate_kernel<AD, GD, true, true>), (kAccumulateCrowd<AD, GD, true>), L, prep);
+    else MXOPT_LAUNCH_CROWD((accumulate_kernel<AD, GD, true, false>), (kAccumulateCrowd<AD, GD, false>), L, prep);
+  } else {
+    if (first) MXOPT_LAUNCH((accumulate_kernel<AD, GD, false, true>), L, prep);
+    else MXOPT_LAUNCH((accumulate_kernel<AD, GD, false, false>), L, prep);
+  }
+}
 
 // ------------------------------------------------------------------------------------
 // The plain norm of a 16-bit stream (no stage in front of the squares), several chunks per trip.  A trip of
@@ -449,6 +526,9 @@ __global__ __launch_bounds__(THREADS) void norm_finish_kernel(const double* __re
 
 template <int MODE, int AD, int GD>
 static void launch_sumsq_t(const Launch& L, const DevPrep& prep, int first, double* ps) {
+  if constexpr (MODE == 2) {
+    if (ps == nullptr) { launch_accumulate<AD, GD>(L, prep, first); return; }
+  }
   if (L.nontemporal) MXOPT_LAUNCH((sumsq_kernel<MODE, AD, GD, true>), L, prep, first, ps);
   else MXOPT_LAUNCH((sumsq_kernel<MODE, AD, GD, false>), L, prep, first, ps);
 }

@@ -66,6 +66,39 @@ __device__ __forceinline__ void pin(T& piece) {
   asm volatile("" : "+v"(piece));
 }
 
+// The workgroup's tile and the descriptor of its first chunk's tensor.
+struct TileView {
+  DevTile tile;
+  DevTensor t;
+  bool whole;
+};
+__device__ __forceinline__ TileView this_tile(const DevTensor* __restrict__ T, const DevTensor& one, uint32_t nchunks,
+                                              const DevTile* __restrict__ tiles) {
+  TileView tv;
+  if (tiles != nullptr) {
+    tv.tile = load_constant<DevTile>(tiles, blockIdx.x);
+    tv.t = load_constant<DevTensor>(T, tv.tile.tensor);
+    tv.whole = (tv.tile.count & kTileWhole) != 0;
+    tv.tile.count &= ~kTileWhole;
+  } else {  // a single tensor described in the kernel arguments
+    tv.t = one;
+    const uint32_t entry = blockIdx.x * kTileChunks;
+    tv.tile = DevTile{entry, nchunks - entry < kTileChunks ? nchunks - entry : kTileChunks, 0u, entry};
+    tv.whole = entry + kTileChunks <= (uint32_t)((one.n - one.head) >> 12);
+  }
+  return tv;
+}
+
+// Calls chunk(view, lane) for each chunk of a tile that is not whole, four at a time.
+template <class F>
+__device__ __forceinline__ void chunks_of_tile(const DevTensor* __restrict__ T, const DevChunk* __restrict__ C, const DevTensor& one,
+                                               const DevTile& tile, F&& chunk) {
+  for (uint32_t k = __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads); k < tile.count; k += kTileThreads / kThreads)
+    chunk(locate(T, C, one, tile.entry + k), threadIdx.x % kThreads);
+}
+
+#define MXOPT_ROWS _Pragma("unroll") for (int j = 0; j < U; ++j)
+
 // Dynamic LDS of every tiled launch, unused: more than half a compute unit's 160 KB, so that one workgroup has it to itself.
 // Plain SGD on 596 M bf16 elements: 586 us with it, 659 without (AdamW's registers have the same effect).
 constexpr unsigned kOnePerCu = 84 * 1024;

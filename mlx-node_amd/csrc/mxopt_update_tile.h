@@ -29,33 +29,24 @@ __global__ __launch_bounds__(kTileThreads) void update_tile_kernel(const DevTens
   const PrepRegs pr = load_prep(prep);
   const uint32_t tid = threadIdx.x;
 
-  DevTile tile;
-  DevTensor t;
-  if (tiles != nullptr) {
-    tile = load_constant<DevTile>(tiles, blockIdx.x);
-    t = load_constant<DevTensor>(T, tile.tensor);
-  } else {  // a single tensor described in the kernel arguments
-    t = one;
-    tile.index = tile.entry = blockIdx.x * kTileChunks;
-    tile.count = nchunks - tile.entry < kTileChunks ? nchunks - tile.entry : kTileChunks;
-    if (tile.entry + kTileChunks <= (uint32_t)((t.n - t.head) >> 12)) tile.count |= kTileWhole;
-  }
-  if (!(tile.count & kTileWhole)) {  // four chunks at a time
-    for (uint32_t k = __builtin_amdgcn_readfirstlane(tid / kThreads); k < tile.count; k += kTileThreads / kThreads)
-      update_chunk<PD, GD, PD, G2, Math, NT>(locate(T, C, one, tile.entry + k), tid % kThreads, math, pr);
+  const TileView tv = this_tile(T, one, nchunks, tiles);
+  if (!tv.whole) {
+    chunks_of_tile(T, C, one, tv.tile, [&](const ChunkView& cv, uint32_t lane) {
+      update_chunk<PD, GD, PD, G2, Math, NT>(cv, lane, math, pr);
+    });
     return;
   }
+  const DevTensor& t = tv.t;
   const uint32_t flags = t.flags;
   const float bc1 = t.bc1, bc2 = t.bc2;
   const bool use_v = math.uses_v(flags), read_v = math.reads_v(flags);
 #pragma unroll 1
   for (uint32_t h = 0; h < kTileChunks / U; ++h) {
-    const uint64_t first = t.head + (uint64_t)(tile.index + h * U) * kChunk;
+    const uint64_t first = t.head + (uint64_t)(tv.tile.index + h * U) * kChunk;
     typename Piece<PD>::T p[U];
     typename Piece<GD>::T g[U];
     typename Piece<G2D>::T g2[U];
     f32x4 m[U], v[U];
-#define MXOPT_ROWS _Pragma("unroll") for (int j = 0; j < U; ++j)
     MXOPT_ROWS g[j] = load_piece<GD, NT>(t.g, first + j * kChunk, tid);
     if (kHasG2) { MXOPT_ROWS g2[j] = load_piece<G2D, NT>(t.g_out, first + j * kChunk, tid); }
     MXOPT_ROWS p[j] = load_piece<PD, NT>(t.p, first + j * kChunk, tid);
@@ -104,8 +95,8 @@ __global__ __launch_bounds__(kTileThreads) void update_tile_kernel(const DevTens
     __builtin_amdgcn_sched_barrier(0);
     if (use_v) { MXOPT_ROWS store_piece<MXOPT_F32, NT>(t.v, first + j * kChunk, tid, v[j]); }
   }
-  if (tile.index == 0 && tid < t.head) {  // elements in front of the first aligned group
-    ChunkView head = locate(T, C, one, tile.entry);
+  if (tv.tile.index == 0 && tid < t.head) {  // elements in front of the first aligned group
+    ChunkView head = locate(T, C, one, tv.tile.entry);
     head.fast = false;
     head.len = 0;
     update_chunk<PD, GD, PD, G2, Math, NT>(head, tid, math, pr);

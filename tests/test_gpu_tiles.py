@@ -174,7 +174,7 @@ def test_single_tensor(mx, ctx, n, shift):
 def test_rule_takes_tiles_for_long_lists_only(mx, ctx):
     """The default rule on both sides of its line gives the results of either route."""
     import torch
-    for n in (TILE * ctx.get_option("num_cus") * 2 - 5, TILE * ctx.get_option("num_cus") * 2 + 5):
+    for n in (TILE * ctx.get_option("num_cus") * 3 - 5, TILE * ctx.get_option("num_cus") * 3 + 5):
         gen = torch.Generator(device="cuda")
         gen.manual_seed(5)
         p = torch.empty(n, device="cuda").normal_(0.0, 0.5, generator=gen)
@@ -220,3 +220,30 @@ def test_engines(mx, ctx, kind, defer, dtype):
             ctx.set_option("tiles", 1)
         outs.append(p)
     assert torch.equal(bits(torch, outs[0]), bits(torch, outs[1])) and not torch.equal(outs[0], base)
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("ad,gd", list(itertools.product(["float32", "bfloat16", "float16"], repeat=2)))
+def test_accumulation(mx, ctx, ad, gd, layout):
+    """Later passes without the norm, in place and into another buffer; chunk by chunk they also give what torch gives (one
+    float32 addition, rounded to the buffer's type)."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(8)
+    a, g = slab(torch, getattr(torch, ad), gen, 1e-2), slab(torch, getattr(torch, gd), gen, 1e-2)
+    a[70000], g[70001] = float("inf"), -0.0
+    run_both(torch, mx, ctx, dict(g_out=a, g=g), layout, lambda t: ctx.accumulate(t, first=False))
+    out = a.clone()
+    va, vg, vo = views(a, layout, 0), views(g, layout, 1), views(out, layout, 0)
+    ctx.accumulate(ctx.table([mx.TensorSpec(g_out=o, g=x) for o, x in zip(vo, vg)]), first=False)
+    for o, x, y in zip(vo, va, vg):
+        assert torch.equal(bits(torch, o.clone()), bits(torch, (x.float() + y.float()).to(o.dtype)))
+    other = [slab(torch, a.dtype, gen, 1.0) for _ in range(2)]
+    for tiles, dst in zip((0, 2), other):
+        ctx.set_option("tiles", tiles)
+        try:
+            ctx.accumulate(ctx.table([mx.TensorSpec(p=x, g_out=o, g=y) for x, o, y in zip(va, views(dst, layout, 0), vg)]), first=False)
+        finally:
+            ctx.set_option("tiles", 1)
+    for p, q, o in zip(views(other[0], layout, 0), views(other[1], layout, 0), vo):
+        assert torch.equal(bits(torch, p.clone()), bits(torch, q.clone())) and torch.equal(bits(torch, p.clone()), bits(torch, o.clone()))
