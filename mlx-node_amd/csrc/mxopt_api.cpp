@@ -169,16 +169,16 @@ Launch make_launch(const mxopt_ctx* ctx, const mxopt_table* t, const Group& g, b
   return L;
 }
 
-// Offers the tiled kernels a cut of `elems` elements into `ntiles` tiles, `whole` of them whole.  Lists that are hardly
-// whole tiles anywhere stay with the chunks: a mixed tile occupies a compute unit for a few short chunks.  bf16 AdamW, microseconds
-// by chunks and by tiles, with the share of elements in whole tiles: 10,000 tensors of 100 - 3,000 elements, none: 50, 65;
-// 10,000 of 64 - 65,536, 35 %: 385, 382; 10,000 of 20,000 - 40,000, 33 %: 1,228, 1,178; 2,000 of 1,000 - 200,000, 80 %: 305, 281.
+// Offers the tiled kernels a cut of `elems` elements into `ntiles` tiles, `whole` of them whole, where two thirds of the
+// elements lie in whole ones: a mixed tile occupies a compute unit for a few short chunks.  Microseconds by tiles and by chunks (two
+// workgroups per compute unit): 10,000 tensors of 64 - 65,536 elements, 35 % of them in whole tiles, bf16 AdamW 391 and 367,
+// float32 511 and 488, SGD 366 and 356; 2,000 of 1,000 - 200,000, 69 %, float32 AdamW 375 and 391, SGD 272 and 292.
 static void offer_tiles(const mxopt_ctx* ctx, Launch& L, const DevTile* tiles, uint32_t ntiles, uint32_t whole, uint64_t elems) {
   if (ctx->tiles == 0 || ctx->persistent || !ctx->nontemporal || ntiles == 0) return;
-  if (ctx->tiles == 1 && (uint64_t)whole * kTileElems * 4u < elems) return;
+  if (ctx->tiles == 1 && (uint64_t)whole * kTileElems * 3u < elems * 2u) return;
   L.tiles = tiles;
   L.ntiles = ntiles;
-  L.tiles_per_cu = ctx->tiles == 1 ? (uint32_t)(elems / kTileElems / (uint32_t)ctx->num_cus) : 0xffffffffu;
+  L.tiles_per_cu = ctx->tiles == 1 ? whole / (uint32_t)ctx->num_cus : 0xffffffffu;
 }
 
 std::string dtype_names(const Group& g) {

@@ -106,13 +106,20 @@ __global__ __launch_bounds__(kThreads) void transform_kernel(const DevTensor* __
 // Launchers (dtype dispatch)
 // ------------------------------------------------------------------------------------
 
+// Microseconds with as many workgroups as the registers allow (4 or 5) and with two: bf16 AdamW, 10,000 tensors of 64 - 65,536
+// elements 405 and 367, one of 24 M 93 and 95, 48 M 185 and 181, 96 M 395 and 369; float32, the 10,000 518 and 488; float32 SGD 378 and
+// 356.  10,000 tensors of 100 - 3,000 (chunks 27 %
+// full) 52 and 86.  16-bit parameters without the first moment gain nothing (SGD, 32 M: 79 and 86).
+template <int PD, int GD, class Math>
+constexpr Crowd kUpdateCrowd = Math::kM || (Math::kV && PD == MXOPT_F32 && GD == MXOPT_F32) ? Crowd{2, 75, 32} : kNoLimit;
+
 template <int PD, int GD, int OD, int G2, class Math>
 static void launch_update_t(const Launch& L, const Math& math, const DevPrep& prep) {
   if constexpr (OD == PD) {
     if (launch_update_tiles<PD, GD, G2>(L, math, prep)) return;
   }
   if (L.nontemporal)
-    MXOPT_LAUNCH((update_kernel<PD, GD, OD, G2, Math, true>), L, math, prep);
+    MXOPT_LAUNCH_CROWD((update_kernel<PD, GD, OD, G2, Math, true>), (kUpdateCrowd<PD, GD, Math>), L, math, prep);
   else
     MXOPT_LAUNCH((update_kernel<PD, GD, OD, G2, Math, false>), L, math, prep);
 }
@@ -236,11 +243,20 @@ bool launch_sgd_plain(int pd, int gd, int od, const Launch& L, float lr_p, float
   return false;
 }
 
+// Microseconds without a limit and with it.  Into a buffer of its own: 16-bit into float32 32 M elements 39 and 37, 64 M 74 and
+// 68, 256 M 277 and 247, 1.72 G 1,852 and 1,596 (10,000 tensors whose chunks are 82 % full 107 and 122); 16-bit into 16-bit 64 M 49
+// and 47, 256 M 182 and 168, 596 M 419 and 374; float32 64 M 93 and 89, 256 M 360 and 351.  Added into a float32 buffer 256 M 435
+// and 426, 596 M 1,005 and 954; into a 16-bit one 128 M 131 and 128, 596 M 589 and 553.
+template <int GD, int OD, bool ADD>
+constexpr Crowd kTransformCrowd =
+    ADD ? (OD == MXOPT_F32 ? (GD == MXOPT_F32 ? kNoLimit : Crowd{2, 90, 256}) : Crowd{4, 90, 128})
+        : (OD != MXOPT_F32 ? Crowd{6, 90, 16} : GD != MXOPT_F32 ? Crowd{4, 90, 16} : Crowd{3, 90, 32});
+
 template <int GD, int OD>
 static void launch_transform_t(const Launch& L, const DevPrep& prep, int add) {
   if (L.nontemporal) {
-    if (add) MXOPT_LAUNCH((transform_kernel<GD, OD, true, true>), L, prep);
-    else MXOPT_LAUNCH((transform_kernel<GD, OD, true, false>), L, prep);
+    if (add) MXOPT_LAUNCH_CROWD((transform_kernel<GD, OD, true, true>), (kTransformCrowd<GD, OD, true>), L, prep);
+    else MXOPT_LAUNCH_CROWD((transform_kernel<GD, OD, true, false>), (kTransformCrowd<GD, OD, false>), L, prep);
   } else {
     if (add) MXOPT_LAUNCH((transform_kernel<GD, OD, false, true>), L, prep);
     else MXOPT_LAUNCH((transform_kernel<GD, OD, false, false>), L, prep);

@@ -103,12 +103,13 @@ __global__ __launch_bounds__(kTileThreads) void update_tile_kernel(const DevTens
   }
 }
 
-// Where tiles begin to pay, in whole tiles per compute unit.  Microseconds by chunks and by tiles: float32 AdamW of 12 M
-// elements 66 and 68, 16 M (2 tiles) 86 and 86, 24 M 130 and 123; SGD 8 M 33 and 34, 16 M 65 and 60; bf16 AdamW 48 M 187 and
-// 193, 64 M (8 tiles) 261 and 252; plain bf16 SGD 64 M 71 and 76, 96 M (12 tiles) 111 and 108.  Below, the ramp of few large
+// Where tiles begin to pay, in whole tiles per compute unit.  Microseconds by chunks and by tiles: float32 AdamW of 16 M
+// elements (2 tiles) 86 and 86, 24 M 130 and 124 (in memory of two regions 117 and 123), 48 M 251 and 240; SGD 8 M 33 and 34,
+// 16 M 65 and 60, 32 M 123 and 112; bf16 AdamW 64 M (8 tiles) 250
+// and 255, 96 M 369 and 372; plain bf16 SGD 64 M 71 and 76, 96 M (12 tiles) 111 and 108.  Below, the ramp of few large
 // workgroups costs more than their order gains.
 template <int PD, int GD, int G2, class Math>
-constexpr uint32_t kUpdateTilesPerCu = (PD == MXOPT_F32 && GD == MXOPT_F32 && G2 <= MXOPT_F32) ? 2 : Math::kV ? 8 : 12;
+constexpr uint32_t kUpdateTilesPerCu = (PD == MXOPT_F32 && GD == MXOPT_F32 && G2 <= MXOPT_F32) ? (Math::kM ? 6 : 3) : Math::kM ? 16 : 12;
 
 template <int PD, int GD, int G2, class Math>
 static bool launch_update_tiles(const Launch& L, const Math& math, const DevPrep& prep) {
