@@ -116,21 +116,28 @@ uint32_t persistent_grid(const mxopt_ctx* ctx, uint32_t nchunks) {
   return (uint32_t)std::min<uint64_t>(nchunks, std::max<uint64_t>(cap, 1));
 }
 
-int ensure_partials(mxopt_ctx* ctx, size_t need) {
+static int ensure_partials(mxopt_ctx* ctx, size_t need) {
   if (need <= ctx->partial_cap) return MXOPT_OK;
-  size_t cap = std::max<size_t>(need, 4096);
-  double* ps = nullptr;
-  HIP_TRY(ctx, hipMalloc((void**)&ps, cap * sizeof(double)));
-  // Earlier launches may still be reading the old buffer.
-  if (ctx->d_partial_sum) {
-    (void)hipStreamSynchronize(ctx->stream);
-    (void)hipFree(ctx->d_partial_sum);
+  constexpr size_t kFront = 256;  // the counter of arrivals, on lines of its own
+  const size_t cap = std::max<size_t>(need, 4096);
+  char* base = nullptr;
+  HIP_TRY(ctx, hipMalloc((void**)&base, kFront + cap * sizeof(double)));
+  launch_clear_arrivals(ctx->stream, (uint32_t*)base);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    (void)hipFree(base);
+    return hip_fail(ctx, e, "clear_arrivals_kernel");
   }
-  ctx->d_partial_sum = ps;
+  // Earlier launches may still be reading the old buffer.
+  if (ctx->d_arrived) {
+    (void)hipStreamSynchronize(ctx->stream);
+    (void)hipFree(ctx->d_arrived);
+  }
+  ctx->d_arrived = (uint32_t*)base;
+  ctx->d_partial_sum = (double*)(base + kFront);
   ctx->partial_cap = cap;
   return MXOPT_OK;
 }
-
 
 int check_launch(mxopt_ctx* ctx, const char* what) {
   hipError_t e = hipGetLastError();
@@ -186,12 +193,32 @@ std::string dtype_names(const Group& g) {
   return std::string("p=") + nm(g.pd) + " g=" + nm(g.gd) + " p_out=" + nm(g.pod) + " g_out=" + nm(g.god);
 }
 
-// Second pass shared by mxopt_global_norm and mxopt_accumulate.
-int finish_norm(mxopt_ctx* ctx, uint32_t npartials, double max_norm, int clip_mode,
-                       mxopt_norm_result* d_result, const double* partials) {
-  const int has_max = max_norm >= 0.0;
-  launch_norm_finish(ctx->stream, partials ? partials : ctx->d_partial_sum, npartials, max_norm, has_max, clip_mode,
-                     d_result);
+int begin_norm(mxopt_ctx* ctx, size_t npartials, double max_norm, int clip_mode, mxopt_norm_result* d_result,
+               mxopt_norm_result* host_out, NormFold* fold) {
+  const int rc = ensure_partials(ctx, std::max<size_t>(npartials, 1));
+  if (rc) return rc;
+  fold->partials = ctx->d_partial_sum;
+  fold->arrived = ctx->d_arrived;
+  fold->count = npartials <= kMaxFolded ? (uint32_t)npartials : 0u;
+  fold->has_max = max_norm >= 0.0;
+  fold->clip_mode = clip_mode;
+  fold->max_norm = max_norm;
+  fold->out = d_result;
+  fold->host_out = host_out;
+  return MXOPT_OK;
+}
+
+// The end of a call whose launches carried `fold`: `launched` workgroups.  A call that failed behind its first launch: those
+// workgroups have been counted, and the next call counts from zero.
+static int end_norm(mxopt_ctx* ctx, const NormFold& fold, size_t launched, int rc) {
+  if (rc == MXOPT_OK && fold.count != 0 && launched != fold.count)
+    rc = fail(ctx, MXOPT_ERR_FAILURE, "norm: workgroups launched and counted differ");
+  if (rc != MXOPT_OK) {
+    if (fold.count != 0 && launched != 0) launch_clear_arrivals(ctx->stream, fold.arrived);
+    return rc;
+  }
+  if (fold.count != 0) return MXOPT_OK;
+  launch_norm_finish(ctx->stream, fold, (uint32_t)launched);
   return check_launch(ctx, "norm_finish_kernel");
 }
 
@@ -199,7 +226,7 @@ int finish_norm(mxopt_ctx* ctx, uint32_t npartials, double max_norm, int clip_mo
 // buffer, and nothing is allocated; a table that wants more workgroups than the array has slots is refused.
 static int run_sumsq(mxopt_ctx* ctx, const mxopt_table* t, int mode, int first, const mxopt_grad_prep* prep,
                      double max_norm, int clip_mode, mxopt_norm_result* d_result, const char* op,
-                     bool static_partials = false) {
+                     bool static_partials = false, mxopt_norm_result* host_out = nullptr) {
   if (clip_mode != MXOPT_CLIP_ALWAYS_MULTIPLY && clip_mode != MXOPT_CLIP_IF_ABOVE)
     return fail(ctx, MXOPT_ERR_INVALID_ARG, std::string(op) + ": unknown clip mode");
   DeviceGuard guard(ctx->device);
@@ -219,6 +246,7 @@ static int run_sumsq(mxopt_ctx* ctx, const mxopt_table* t, int mode, int first, 
   for (const Group& g : t->groups) total_grid += reduction_grid(g);
   const bool want = d_result != nullptr;
   double* partials = nullptr;
+  NormFold fold;
   if (static_partials) {
     if (total_grid > kStaticPartials)
       return fail(ctx, MXOPT_ERR_INVALID_ARG,
@@ -227,12 +255,19 @@ static int run_sumsq(mxopt_ctx* ctx, const mxopt_table* t, int mode, int first, 
                       std::to_string(kStaticPartials) + "; lower grid_blocks_per_cu or use mxopt_global_norm");
     if (!ctx->d_static_partials) return fail(ctx, MXOPT_ERR_FAILURE, std::string(op) + ": the fixed array has no address");
     partials = ctx->d_static_partials;
+    // two passes: the array has no counters
+    fold.partials = partials;
+    fold.has_max = max_norm >= 0.0;
+    fold.clip_mode = clip_mode;
+    fold.max_norm = max_norm;
+    fold.out = d_result;
   } else if (want) {
-    int rc = ensure_partials(ctx, std::max<size_t>(total_grid, 1));
+    int rc = begin_norm(ctx, total_grid, max_norm, clip_mode, d_result, host_out, &fold);
     if (rc) return rc;
     partials = ctx->d_partial_sum;
   }
   size_t offset = 0;
+  int rc = MXOPT_OK;
   for (const Group& g : t->groups) {
     // Reductions need one partial per workgroup, so they keep a bounded grid.  Accumulation passes that
     // take no norm follow the update kernels' launch policy (one workgroup per chunk: 6.12 against
@@ -244,14 +279,14 @@ static int run_sumsq(mxopt_ctx* ctx, const mxopt_table* t, int mode, int first, 
     const int ad = mode == 0 ? g.gd : g.god;
     MXOPT_DEBUG("%s (reduction mode %d%s): %s, %u chunks in %u workgroups", op, mode, first ? ", first" : "",
                 dtype_names(g).c_str(), g.nchunks, L.grid);
-    if (!launch_sumsq(mode, ad, g.gd, L, dp, first, want ? partials + offset : nullptr))
-      return fail(ctx, MXOPT_ERR_INVALID_ARG, std::string(op) + ": unsupported dtypes " + dtype_names(g));
-    int rc = check_launch(ctx, op);
-    if (rc) return rc;
+    if (!launch_sumsq(mode, ad, g.gd, L, dp, first, want ? partials + offset : nullptr, fold)) {
+      rc = fail(ctx, MXOPT_ERR_INVALID_ARG, std::string(op) + ": unsupported dtypes " + dtype_names(g));
+      break;
+    }
+    if ((rc = check_launch(ctx, op))) break;
     offset += L.grid;
   }
-  if (want) return finish_norm(ctx, (uint32_t)offset, max_norm, clip_mode, d_result, partials);
-  return MXOPT_OK;
+  return want ? end_norm(ctx, fold, offset, rc) : rc;
 }
 
 template <class F>
@@ -374,10 +409,11 @@ void mxopt_destroy(mxopt_ctx* ctx) {
     (void)hipStreamSynchronize(ctx->stream);
     (void)hipFree(ctx->d_norm_scratch);
   }
-  if (ctx->d_partial_sum) {
+  if (ctx->d_arrived) {
     (void)hipStreamSynchronize(ctx->stream);
-    (void)hipFree(ctx->d_partial_sum);
+    (void)hipFree(ctx->d_arrived);
   }
+  if (ctx->h_norm) (void)hipHostFree(ctx->h_norm);
   delete ctx;
 }
 
@@ -1032,13 +1068,22 @@ int mxopt_fill_synthetic(mxopt_ctx* ctx, void* out, uint64_t n, int dtype, uint6
   return check_launch(ctx, "mxopt_fill_synthetic");
 }
 
-int mxopt_global_norm(mxopt_ctx* ctx, const mxopt_table* t, int which, const mxopt_grad_prep* prep, double max_norm,
-                      int clip_mode, mxopt_norm_result* d_result) {
+}  // extern "C"
+
+int mxopt::global_norm(mxopt_ctx* ctx, const mxopt_table* t, int which, const mxopt_grad_prep* prep, double max_norm,
+                       int clip_mode, mxopt_norm_result* d_result, mxopt_norm_result* host_out) {
   if (which != 0 && which != 1) return fail(ctx, MXOPT_ERR_INVALID_ARG, "mxopt_global_norm: which must be 0 or 1");
   int rc = require(ctx, t, which == 0 ? kNeedG : kNeedGOut, "mxopt_global_norm");
   if (rc) return rc;
   if (!d_result) return fail(ctx, MXOPT_ERR_INVALID_ARG, "mxopt_global_norm: d_result is NULL");
-  return run_sumsq(ctx, t, which, 0, prep, max_norm, clip_mode, d_result, "mxopt_global_norm");
+  return run_sumsq(ctx, t, which, 0, prep, max_norm, clip_mode, d_result, "mxopt_global_norm", false, host_out);
+}
+
+extern "C" {
+
+int mxopt_global_norm(mxopt_ctx* ctx, const mxopt_table* t, int which, const mxopt_grad_prep* prep, double max_norm,
+                      int clip_mode, mxopt_norm_result* d_result) {
+  return global_norm(ctx, t, which, prep, max_norm, clip_mode, d_result, nullptr);
 }
 
 int mxopt_global_norm_static(mxopt_ctx* ctx, const mxopt_table* t, int which, const mxopt_grad_prep* prep,
@@ -1058,16 +1103,18 @@ int mxopt_accumulate(mxopt_ctx* ctx, const mxopt_table* t, int first, const mxop
   return run_sumsq(ctx, t, 2, first ? 1 : 0, prep, max_norm, clip_mode, d_result, "mxopt_accumulate");
 }
 
-int mxopt_accumulate_norm_only(mxopt_ctx* ctx, const mxopt_table* t, const mxopt_grad_prep* prep, double max_norm,
-                               int clip_mode, mxopt_norm_result* d_result) {
+}  // extern "C"
+
+int mxopt::accumulate_norm_only(mxopt_ctx* ctx, const mxopt_table* t, const mxopt_grad_prep* prep, double max_norm,
+                                int clip_mode, mxopt_norm_result* d_result, mxopt_norm_result* host_out) {
   int rc = require(ctx, t, kNeedG | kNeedGOut, "mxopt_accumulate_norm_only");
   if (rc) return rc;
   if (!d_result) return fail(ctx, MXOPT_ERR_INVALID_ARG, "mxopt_accumulate_norm_only: d_result is NULL");
-  return run_sumsq(ctx, t, 3, 0, prep, max_norm, clip_mode, d_result, "mxopt_accumulate_norm_only");
+  return run_sumsq(ctx, t, 3, 0, prep, max_norm, clip_mode, d_result, "mxopt_accumulate_norm_only", false, host_out);
 }
 
-int mxopt_norm_with_pending_list(mxopt_ctx* ctx, const mxopt_table* t, const mxopt_grad_prep* prep, double max_norm,
-                                 int clip_mode, mxopt_norm_result* d_result) {
+int mxopt::norm_with_pending_list(mxopt_ctx* ctx, const mxopt_table* t, const mxopt_grad_prep* prep, double max_norm,
+                                  int clip_mode, mxopt_norm_result* d_result, mxopt_norm_result* host_out) {
   const char* op = "mxopt_norm_with_pending_list";
   int rc = require(ctx, t, kNeedG, op);
   if (rc) return rc;
@@ -1084,8 +1131,8 @@ int mxopt_norm_with_pending_list(mxopt_ctx* ctx, const mxopt_table* t, const mxo
   };
   size_t total_grid = 0;
   for (const Group& g : t->groups) total_grid += list_grid(g.nchunks);
-  rc = ensure_partials(ctx, std::max<size_t>(total_grid, 1));
-  if (rc) return rc;
+  NormFold fold;
+  if ((rc = begin_norm(ctx, total_grid, max_norm, clip_mode, d_result, host_out, &fold))) return rc;
   size_t offset = 0;
   for (const Group& g : t->groups) {
     Launch L = make_launch(ctx, t, g, true);
@@ -1094,13 +1141,26 @@ int mxopt_norm_with_pending_list(mxopt_ctx* ctx, const mxopt_table* t, const mxo
     attach_pending(t, L);
     MXOPT_DEBUG("%s: %s, %d pending stream(s), %u chunks in %u workgroups", op, dtype_names(g).c_str(), t->pending_k,
                 g.nchunks, L.grid);
-    if (!launch_sumsq_list(g.gd, t->pending_k ? t->pending_dtype : g.gd, L, dp, ctx->d_partial_sum + offset))
-      return fail(ctx, MXOPT_ERR_INVALID_ARG, std::string(op) + ": unsupported dtypes " + dtype_names(g));
-    rc = check_launch(ctx, op);
-    if (rc) return rc;
+    if (!launch_sumsq_list(g.gd, t->pending_k ? t->pending_dtype : g.gd, L, dp, ctx->d_partial_sum + offset, fold)) {
+      rc = fail(ctx, MXOPT_ERR_INVALID_ARG, std::string(op) + ": unsupported dtypes " + dtype_names(g));
+      break;
+    }
+    if ((rc = check_launch(ctx, op))) break;
     offset += L.grid;
   }
-  return finish_norm(ctx, (uint32_t)offset, max_norm, clip_mode, d_result);
+  return end_norm(ctx, fold, offset, rc);
+}
+
+extern "C" {
+
+int mxopt_accumulate_norm_only(mxopt_ctx* ctx, const mxopt_table* t, const mxopt_grad_prep* prep, double max_norm,
+                               int clip_mode, mxopt_norm_result* d_result) {
+  return accumulate_norm_only(ctx, t, prep, max_norm, clip_mode, d_result, nullptr);
+}
+
+int mxopt_norm_with_pending_list(mxopt_ctx* ctx, const mxopt_table* t, const mxopt_grad_prep* prep, double max_norm,
+                                 int clip_mode, mxopt_norm_result* d_result) {
+  return norm_with_pending_list(ctx, t, prep, max_norm, clip_mode, d_result, nullptr);
 }
 
 int mxopt_read_norm_result(mxopt_ctx* ctx, const mxopt_norm_result* d_result, mxopt_norm_result* host_out) {

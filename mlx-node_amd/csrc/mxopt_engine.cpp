@@ -404,13 +404,10 @@ int refuse_capture(mxopt_engine* e) {
   return hip_fail(e->ctx, hipErrorStreamCaptureUnsupported, "engine: the call waits for the norm on the host");
 }
 
-// The result of the norm pass starts its way to pinned host memory; nobody waits for it here.
+// The norm pass just enqueued writes its result to pinned host memory too: where the host can wait for it.
 int enqueue_flag_copy(mxopt_engine* e, const mxopt_norm_result* d_result) {
   mxopt_ctx* ctx = e->ctx;
   DeviceGuard guard(ctx->device);
-  launch_mirror_result(ctx->stream, d_result, e->h_pinned);
-  int rc = check_launch(ctx, "mirror_result_kernel");
-  if (rc) return rc;
   HIP_TRY(ctx, hipEventRecord(e->copied, ctx->stream));
   e->async_skip = &d_result->nonfinite;
   e->async_enqueued = true;
@@ -462,7 +459,9 @@ int grpo_micro_batch(mxopt_engine* e, const std::vector<size_t>& idx, const mxop
     mxopt_table* t = nullptr;
     if ((rc = cached_table(ctx, rows, &t))) return rc;
     const double max_norm = e->cfg.has_gradient_clip_norm ? e->cfg.gradient_clip_norm : -1.0;
-    if ((rc = mxopt_global_norm(ctx, t, 0, &prep, max_norm, MXOPT_CLIP_ALWAYS_MULTIPLY, d_result))) return rc;
+    if ((rc = global_norm(ctx, t, 0, &prep, max_norm, MXOPT_CLIP_ALWAYS_MULTIPLY, d_result,
+                          e->async_mode ? e->h_pinned : nullptr)))
+      return rc;
     // async: the flag is not waited for; every kernel below obeys it on the device instead
     if ((rc = e->async_mode ? enqueue_flag_copy(e, d_result) : mxopt_read_norm_result(ctx, d_result, &h))) return rc;
   }
@@ -637,12 +636,15 @@ int grpo_enqueue(mxopt_engine* e, const std::vector<size_t>& idx, const mxopt_ar
 // The norm on its way to the host: it leaves right behind the norm pass, and the host looks for it once the update is
 // enqueued, so that the update follows the norm pass at once.  (Read in between, the device idled for the read-back and
 // the host's work on the update: 10 - 50 us of a step of 0.9 - 3 ms.)
-int norm_leaves(mxopt_engine* e) {
+// written: the norm pass has been given h_pinned and writes it itself.
+int norm_leaves(mxopt_engine* e, bool written) {
   int rc = ensure_pinned(e);
   if (rc) return rc;
   DeviceGuard guard(e->ctx->device);
-  launch_mirror_result(e->ctx->stream, e->d_result, e->h_pinned);
-  if ((rc = check_launch(e->ctx, "mirror_result_kernel"))) return rc;
+  if (!written) {
+    launch_mirror_result(e->ctx->stream, e->d_result, e->h_pinned);
+    if ((rc = check_launch(e->ctx, "mirror_result_kernel"))) return rc;
+  }
   HIP_TRY(e->ctx, hipEventRecord(e->copied, e->ctx->stream));
   return MXOPT_OK;
 }
@@ -663,6 +665,7 @@ int sft_apply(mxopt_engine* e, int32_t count, bool norm_ready, mxopt_engine_metr
   prep.pre_mul = (float)(1.0 / (double)count);  // mul_scalar(scale): float64, then one cast
   int rc;
   *measured = false;
+  bool written = false;
   if (e->cfg.has_gradient_clip_norm) {
     if (!norm_ready) {
       std::vector<mxopt_tensor> rows;
@@ -675,8 +678,10 @@ int sft_apply(mxopt_engine* e, int32_t count, bool norm_ready, mxopt_engine_metr
       if (!rows.empty()) {
         mxopt_table* t = nullptr;
         if ((rc = cached_table(ctx, rows, &t))) return rc;
-        if ((rc = mxopt_global_norm(ctx, t, 1, &prep, e->cfg.gradient_clip_norm, MXOPT_CLIP_ALWAYS_MULTIPLY,
-                                    e->d_result)))
+        if (out && (rc = ensure_pinned(e))) return rc;
+        written = out != nullptr;
+        if ((rc = global_norm(ctx, t, 1, &prep, e->cfg.gradient_clip_norm, MXOPT_CLIP_ALWAYS_MULTIPLY, e->d_result,
+                              out ? e->h_pinned : nullptr)))
           return rc;
         norm_ready = true;
       }
@@ -684,7 +689,7 @@ int sft_apply(mxopt_engine* e, int32_t count, bool norm_ready, mxopt_engine_metr
     if (norm_ready) {
       prep.d_scale = &e->d_result->scale;
       if (out) {  // only a caller that wants the figures pays for the read-back
-        if ((rc = norm_leaves(e))) return rc;
+        if ((rc = norm_leaves(e, written))) return rc;
         *measured = true;
       }
     }
@@ -735,15 +740,21 @@ int sft_apply_deferred(mxopt_engine* e, int32_t count, mxopt_engine_metrics* out
       mxopt_table* t = nullptr;
       if ((rc = defer_table(e, &t))) return rc;
       if (clip) {
-        rc = mxopt_norm_with_pending_list(ctx, t, &prep, e->cfg.gradient_clip_norm, MXOPT_CLIP_ALWAYS_MULTIPLY,
-                                          e->d_result);
+        if (out) rc = ensure_pinned(e);
+        if (!rc)
+          rc = norm_with_pending_list(ctx, t, &prep, e->cfg.gradient_clip_norm, MXOPT_CLIP_ALWAYS_MULTIPLY, e->d_result,
+                                      out ? e->h_pinned : nullptr);
+        if (!rc && out) rc = norm_leaves(e, true);
+        *measured = !rc && out != nullptr;
         prep.d_scale = &e->d_result->scale;
       }
       if (!rc) rc = mxopt_sgd_plain_with_pending_list(ctx, t, e->cfg.learning_rate, e->cfg.weight_decay, &prep);
       (void)mxopt_table_set_pending(t, 0, nullptr, 0);
     }
     if (rc) return rc;
-    if (clip && out) {
+    if (*measured) {
+      if ((rc = norm_arrives(e, h_out))) return rc;
+    } else if (clip && out) {
       if ((rc = mxopt_read_norm_result(ctx, e->d_result, h_out))) return rc;
       *measured = true;
     }
@@ -823,13 +834,15 @@ int sft_micro_batch(mxopt_engine* e, const std::vector<size_t>& idx, const mxopt
     bool measured = false;
     if (e->cfg.has_gradient_clip_norm) {
       if ((rc = cached_table(ctx, rows, &t))) return rc;
-      rc = direct ? mxopt_global_norm(ctx, t, 0, &prep, e->cfg.gradient_clip_norm, MXOPT_CLIP_ALWAYS_MULTIPLY, e->d_result)
-                  : mxopt_accumulate_norm_only(ctx, t, &prep, e->cfg.gradient_clip_norm, MXOPT_CLIP_ALWAYS_MULTIPLY,
-                                               e->d_result);
+      if (out && (rc = ensure_pinned(e))) return rc;
+      mxopt_norm_result* host_out = out ? e->h_pinned : nullptr;
+      rc = direct ? global_norm(ctx, t, 0, &prep, e->cfg.gradient_clip_norm, MXOPT_CLIP_ALWAYS_MULTIPLY, e->d_result, host_out)
+                  : accumulate_norm_only(ctx, t, &prep, e->cfg.gradient_clip_norm, MXOPT_CLIP_ALWAYS_MULTIPLY, e->d_result,
+                                         host_out);
       if (rc) return rc;
       prep.d_scale = &e->d_result->scale;
       if (out) {
-        if ((rc = norm_leaves(e))) return rc;
+        if ((rc = norm_leaves(e, true))) return rc;
         measured = true;
       }
     }

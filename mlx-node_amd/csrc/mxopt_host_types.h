@@ -105,8 +105,10 @@ struct mxopt_ctx {
   int pipelined_norm = 2;         // plain 16-bit norms: the software-pipelined kernel
   double* d_partial_sum = nullptr;            // one float64 partial per workgroup of a reduction
   size_t partial_cap = 0;
+  uint32_t* d_arrived = nullptr;              // NormFold::arrived, in front of the partial sums in their allocation
   double* d_static_partials = nullptr;        // this device's copy of the library's fixed partial-sum array
   mxopt_norm_result* d_norm_scratch = nullptr;  // result slot of the gradient utilities
+  mxopt_norm_result* h_norm = nullptr;          // pinned: the norm that a gradient utility hands back
   mxopt_hbm_pool* state_pool = nullptr;         // where the host layer takes moments and accumulation buffers from
   struct CachedTable {                          // tables built by the host layer, most recent last
     std::vector<mxopt_tensor> key;

@@ -54,11 +54,19 @@ float round_to_dtype(float x, int dt);
 DevPrep make_prep(const mxopt_grad_prep* p);
 bool prep_active(const mxopt_grad_prep* p);
 uint32_t persistent_grid(const mxopt_ctx* ctx, uint32_t nchunks);
-int ensure_partials(mxopt_ctx* ctx, size_t need);
 int check_launch(mxopt_ctx* ctx, const char* what);
-// partials == NULL: the context's own buffer.
-int finish_norm(mxopt_ctx* ctx, uint32_t npartials, double max_norm, int clip_mode, mxopt_norm_result* d_result,
-                const double* partials = nullptr);
+// The fold of a norm over `npartials` workgroups in the context's buffer, which is made large enough; *fold is for the
+// launchers.  host_out: pinned memory that gets the result too.
+int begin_norm(mxopt_ctx* ctx, size_t npartials, double max_norm, int clip_mode, mxopt_norm_result* d_result,
+               mxopt_norm_result* host_out, NormFold* fold);
+// mxopt_global_norm, mxopt_accumulate_norm_only and mxopt_norm_with_pending_list whose result also goes to pinned host memory
+// (host_out, may be NULL): there once an event recorded behind the call has passed.
+int global_norm(mxopt_ctx* ctx, const mxopt_table* t, int which, const mxopt_grad_prep* prep, double max_norm, int clip_mode,
+                mxopt_norm_result* d_result, mxopt_norm_result* host_out);
+int accumulate_norm_only(mxopt_ctx* ctx, const mxopt_table* t, const mxopt_grad_prep* prep, double max_norm, int clip_mode,
+                         mxopt_norm_result* d_result, mxopt_norm_result* host_out);
+int norm_with_pending_list(mxopt_ctx* ctx, const mxopt_table* t, const mxopt_grad_prep* prep, double max_norm, int clip_mode,
+                           mxopt_norm_result* d_result, mxopt_norm_result* host_out);
 void fill_dev_tensor(const mxopt_tensor& s, DevTensor& d);
 uint64_t chunks_of(const DevTensor& d);  // chunk-table entries (= workgroups of work) of one tensor
 // A launch over the single tensor `t` (descriptor passed in the kernel arguments).

@@ -38,6 +38,19 @@ struct Launch {
   StreamScales scales{};             // used when the prep carries kPrepEachStream
 };
 
+// The second pass of a norm, done by the workgroup that finishes last: `count` partial sums of all launches of the call,
+// folded into *out.  count 0: the launches leave their partial sums for launch_norm_finish.
+constexpr uint32_t kMaxFolded = 64;  // see finish_partial
+struct NormFold {
+  const double* partials = nullptr;
+  uint32_t* arrived = nullptr;  // workgroups that have stored theirs; 0 between calls
+  uint32_t count = 0;
+  int has_max = 0, clip_mode = 0;
+  double max_norm = 0.0;
+  mxopt_norm_result* out = nullptr;
+  mxopt_norm_result* host_out = nullptr;  // pinned host memory that gets the result too, or NULL
+};
+
 // Each returns false when the dtype combination has no kernel.
 // g2d >= 0: tensor.g_out holds a second gradient of that dtype which is added to g (float32) first.
 bool launch_adam(int pd, int gd, int od, int g2d, const Launch& L, const mxopt_adam_hp& hp, const DevPrep& prep);
@@ -56,7 +69,8 @@ bool launch_transform(int gd, int od, const Launch& L, const DevPrep& prep, int 
 // mode 0: square g; 1: square g_out; 2: g_out = first ? g : g_out + g, square the result;
 // 3: square g_out + g without storing it.
 // partial_sum (one entry per workgroup) may be NULL in mode 2.
-bool launch_sumsq(int mode, int ad, int gd, const Launch& L, const DevPrep& prep, int first, double* partial_sum);
+bool launch_sumsq(int mode, int ad, int gd, const Launch& L, const DevPrep& prep, int first, double* partial_sum,
+                  const NormFold& fold);
 // Deferred accumulation: the gradient is g + pending_0 + ... (float32 adds, left to right); xd is the
 // pending streams' dtype, gd either xd or float32.  Parameters are updated in their own dtype.
 bool launch_adam_list(int pd, int gd, int od, int xd, const Launch& L, const mxopt_adam_hp& hp, const DevPrep& prep);
@@ -65,16 +79,18 @@ bool launch_sgd_plain_list(int pd, int gd, int od, int xd, const Launch& L, floa
 bool launch_sgd_list(int pd, int gd, int od, int xd, const Launch& L, const mxopt_sgd_hp& hp, const DevPrep& prep);
 bool launch_rmsprop_list(int pd, int gd, int od, int xd, const Launch& L, const mxopt_rmsprop_hp& hp,
                          const DevPrep& prep);
-bool launch_sumsq_list(int gd, int xd, const Launch& L, const DevPrep& prep, double* partial_sum);
+bool launch_sumsq_list(int gd, int xd, const Launch& L, const DevPrep& prep, double* partial_sum, const NormFold& fold);
 bool launch_synth(int od, void* out, uint64_t n, uint64_t seed, uint64_t first_index, int dist, float a, float b,
                   uint32_t grid, hipStream_t stream);
+// *arrived = 0 by a kernel.
+void launch_clear_arrivals(hipStream_t stream, uint32_t* arrived);
 // *host_mapped_dst = *d_src by a one-lane kernel (dst: pinned host memory, visible to the device).
 void launch_mirror_result(hipStream_t stream, const mxopt_norm_result* d_src, mxopt_norm_result* host_mapped_dst);
 // Address, on `device` (which must be the current device), of the library's fixed array of
 // kStaticPartials float64 partial sums: every GPU holds its own copy at its own address.
 constexpr uint32_t kStaticPartials = MXOPT_STATIC_NORM_WORKGROUPS;
 hipError_t static_partials_address(int device, double** out);
-void launch_norm_finish(hipStream_t stream, const double* partial_sum, uint32_t npartials, double max_norm,
-                        int has_max, int clip_mode, mxopt_norm_result* d_out);
+// The second pass on its own: `npartials` sums at fold.partials.
+void launch_norm_finish(hipStream_t stream, const NormFold& fold, uint32_t npartials);
 
 }  // namespace mxopt

@@ -1,6 +1,7 @@
 // mxopt kernels for gfx950, part 3: deferred accumulation -- the norm over gradient streams that were never
 // summed into a buffer, and the Adam/AdamW and plain-SGD updates over them.
 #include "mxopt_list_kernels.h"
+#include "mxopt_norm_fold.h"
 
 namespace mxopt {
 
@@ -10,7 +11,7 @@ __global__ __launch_bounds__(kThreads) void sumsq_list_kernel(const DevTensor* _
                                                               const DevChunk* __restrict__ C, DevTensor one,
                                                               uint32_t nchunks, uint32_t ntensors,
                                                               const void* const* __restrict__ X, int kx, DevPrep prep,
-                                                              double* __restrict__ partial_sum) {
+                                                              double* __restrict__ partial_sum, NormFold fold) {
   constexpr int E = (GD != MXOPT_F32 || XD != MXOPT_F32) ? 8 : 4;
   constexpr int U = kElemsPerLane / E;
   const PrepRegs pr = load_prep(prep);
@@ -103,9 +104,7 @@ __global__ __launch_bounds__(kThreads) void sumsq_list_kernel(const DevTensor* _
     acc_sum += (double)((bad || poison != poison) ? __builtin_nanf("") : s32);
   }
 
-  unsigned long long unused = 0;
-  block_sum(acc_sum, unused);
-  if (tid == 0) partial_sum[blockIdx.x] = acc_sum;
+  finish_partial(acc_sum, partial_sum, fold);
 }
 
 bool launch_adam_list(int pd, int gd, int od, int xd, const Launch& L, const mxopt_adam_hp& hp, const DevPrep& prep) {
@@ -133,28 +132,28 @@ bool launch_sgd_plain_list(int pd, int gd, int od, int xd, const Launch& L, floa
 }
 
 template <int GD, int XD>
-static void launch_sumsq_list_t(const Launch& L, const DevPrep& prep, double* ps) {
+static void launch_sumsq_list_t(const Launch& L, const DevPrep& prep, double* ps, const NormFold& fold) {
   if (L.npending <= kFewPending) {
-    if (L.nontemporal) MXOPT_LAUNCH_LIST((sumsq_list_kernel<GD, XD, kFewPending, true>), L, prep, ps);
-    else MXOPT_LAUNCH_LIST((sumsq_list_kernel<GD, XD, kFewPending, false>), L, prep, ps);
+    if (L.nontemporal) MXOPT_LAUNCH_LIST((sumsq_list_kernel<GD, XD, kFewPending, true>), L, prep, ps, fold);
+    else MXOPT_LAUNCH_LIST((sumsq_list_kernel<GD, XD, kFewPending, false>), L, prep, ps, fold);
   } else {
-    if (L.nontemporal) MXOPT_LAUNCH_LIST((sumsq_list_kernel<GD, XD, MXOPT_MAX_PENDING, true>), L, prep, ps);
-    else MXOPT_LAUNCH_LIST((sumsq_list_kernel<GD, XD, MXOPT_MAX_PENDING, false>), L, prep, ps);
+    if (L.nontemporal) MXOPT_LAUNCH_LIST((sumsq_list_kernel<GD, XD, MXOPT_MAX_PENDING, true>), L, prep, ps, fold);
+    else MXOPT_LAUNCH_LIST((sumsq_list_kernel<GD, XD, MXOPT_MAX_PENDING, false>), L, prep, ps, fold);
   }
 }
 
-bool launch_sumsq_list(int gd, int xd, const Launch& L, const DevPrep& prep, double* partial_sum) {
+bool launch_sumsq_list(int gd, int xd, const Launch& L, const DevPrep& prep, double* partial_sum, const NormFold& fold) {
   if (gd != xd && gd != MXOPT_F32) return false;
   const bool same = gd == xd;
   switch (xd) {
-    case MXOPT_F32: launch_sumsq_list_t<MXOPT_F32, MXOPT_F32>(L, prep, partial_sum); return true;
+    case MXOPT_F32: launch_sumsq_list_t<MXOPT_F32, MXOPT_F32>(L, prep, partial_sum, fold); return true;
     case MXOPT_BF16:
-      if (same) launch_sumsq_list_t<MXOPT_BF16, MXOPT_BF16>(L, prep, partial_sum);
-      else launch_sumsq_list_t<MXOPT_F32, MXOPT_BF16>(L, prep, partial_sum);
+      if (same) launch_sumsq_list_t<MXOPT_BF16, MXOPT_BF16>(L, prep, partial_sum, fold);
+      else launch_sumsq_list_t<MXOPT_F32, MXOPT_BF16>(L, prep, partial_sum, fold);
       return true;
     case MXOPT_F16:
-      if (same) launch_sumsq_list_t<MXOPT_F16, MXOPT_F16>(L, prep, partial_sum);
-      else launch_sumsq_list_t<MXOPT_F32, MXOPT_F16>(L, prep, partial_sum);
+      if (same) launch_sumsq_list_t<MXOPT_F16, MXOPT_F16>(L, prep, partial_sum, fold);
+      else launch_sumsq_list_t<MXOPT_F32, MXOPT_F16>(L, prep, partial_sum, fold);
       return true;
   }
   return false;

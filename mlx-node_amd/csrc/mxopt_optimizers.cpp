@@ -668,6 +668,30 @@ int mxopt_optimizer_load_file(mxopt_optimizer* opt, const char* path) {
 
 // ---- GradientUtils ------------------------------------------------------------------------
 
+}  // extern "C"
+
+// Pinned memory that the norm pass of a call writes its result to: behind the call's synchronisation it is there, and no copy
+// stands in between.  Under stream capture nothing can be waited for: *to stays NULL, and the read-back refuses.
+static int norm_mailbox(mxopt_ctx* ctx, mxopt_norm_result** to) {
+  DeviceGuard guard(ctx->device);
+  *to = nullptr;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  HIP_TRY(ctx, hipStreamIsCapturing(ctx->stream, &status));
+  if (status != hipStreamCaptureStatusNone) return MXOPT_OK;
+  if (!ctx->h_norm) HIP_TRY(ctx, hipHostMalloc((void**)&ctx->h_norm, sizeof(mxopt_norm_result), hipHostMallocDefault));
+  *to = ctx->h_norm;
+  return MXOPT_OK;
+}
+static int collect_norm(mxopt_ctx* ctx, const mxopt_norm_result* to, const mxopt_norm_result* d_result, mxopt_norm_result* h) {
+  if (!to) return mxopt_read_norm_result(ctx, d_result, h);
+  DeviceGuard guard(ctx->device);
+  HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+  *h = *to;
+  return MXOPT_OK;
+}
+
+extern "C" {
+
 int mxopt_compute_gradient_norm(mxopt_ctx* ctx, size_t n, const mxopt_array* grads, double* norm_out) {
   if (!ctx || !norm_out) return fail(ctx, MXOPT_ERR_INVALID_ARG, "compute_gradient_norm: null argument");
   std::vector<mxopt_tensor> rows;
@@ -676,9 +700,11 @@ int mxopt_compute_gradient_norm(mxopt_ctx* ctx, size_t n, const mxopt_array* gra
   mxopt_table* t = nullptr;
   mxopt_norm_result* d = nullptr;
   if ((rc = cached_table(ctx, rows, &t)) || (rc = norm_scratch(ctx, &d))) return rc;
-  if ((rc = mxopt_global_norm(ctx, t, 0, nullptr, -1.0, MXOPT_CLIP_ALWAYS_MULTIPLY, d))) return rc;
+  mxopt_norm_result* to = nullptr;
+  if ((rc = norm_mailbox(ctx, &to))) return rc;
+  if ((rc = global_norm(ctx, t, 0, nullptr, -1.0, MXOPT_CLIP_ALWAYS_MULTIPLY, d, to))) return rc;
   mxopt_norm_result h;
-  if ((rc = mxopt_read_norm_result(ctx, d, &h))) return rc;
+  if ((rc = collect_norm(ctx, to, d, &h))) return rc;
   *norm_out = h.norm;  // float64 accumulation, as optimizers/mod.rs:47-54
   return MXOPT_OK;
 }
@@ -705,14 +731,16 @@ static int clip_by_norm(mxopt_ctx* ctx, size_t n, const mxopt_array* grads, cons
     prep.pre_lo = (float)(-*clip_value);
     prep.pre_hi = (float)(*clip_value);
   }
+  mxopt_norm_result* to = nullptr;
   if (max_norm) {
-    if ((rc = mxopt_global_norm(ctx, t, 0, &prep, *max_norm, clip_mode, d))) return rc;
+    if (norm_out && (rc = norm_mailbox(ctx, &to))) return rc;
+    if ((rc = global_norm(ctx, t, 0, &prep, *max_norm, clip_mode, d, to))) return rc;
     prep.d_scale = &d->scale;
   }
   if ((rc = mxopt_grad_transform(ctx, t, &prep))) return rc;
   if (norm_out) {
     mxopt_norm_result h;
-    if ((rc = mxopt_read_norm_result(ctx, d, &h))) return rc;
+    if ((rc = collect_norm(ctx, to, d, &h))) return rc;
     *norm_out = (double)h.norm_f32;  // item_at_float32(0) as f64 (optimizers/mod.rs:138)
   }
   return MXOPT_OK;

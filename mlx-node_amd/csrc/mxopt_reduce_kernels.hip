@@ -3,6 +3,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "mxopt_norm_fold.h"
 #include "mxopt_tiles.h"
 #include "mxopt_gauss_table.h"
 
@@ -213,7 +214,7 @@ template <int MODE, int AD, int GD, bool NT>
 __global__ __launch_bounds__(kThreads) void sumsq_kernel(const DevTensor* __restrict__ T,
                                                          const DevChunk* __restrict__ C, DevTensor one,
                                                          uint32_t nchunks, DevPrep prep, int first_i,
-                                                         double* __restrict__ partial_sum) {
+                                                         double* __restrict__ partial_sum, NormFold fold) {
   using Chunk = SumsqChunk<MODE, AD, GD, NT>;
   const PrepRegs pr = load_prep(prep);
   const uint32_t tid = threadIdx.x;
@@ -268,9 +269,7 @@ __global__ __launch_bounds__(kThreads) void sumsq_kernel(const DevTensor* __rest
     acc_sum += (double)s;
   }
 
-  unsigned long long unused = 0;
-  block_sum(acc_sum, unused);
-  if (tid == 0) partial_sum[blockIdx.x] = acc_sum;
+  finish_partial(acc_sum, partial_sum, fold);
 }
 
 // Accumulation that is not asked for the norm.  The first pass of a cycle writes lines nobody read, in groups of 8 where a
@@ -374,7 +373,7 @@ template <int AD, int WHICH, bool NT, int NCH>
 __global__ __launch_bounds__(kThreads) void sumsq16_multi_kernel(const DevTensor* __restrict__ T,
                                                                  const DevChunk* __restrict__ C, DevTensor one,
                                                                  uint32_t nchunks, DevPrep prep, int,
-                                                                 double* __restrict__ partial_sum) {
+                                                                 double* __restrict__ partial_sum, NormFold fold) {
   static_assert(AD != MXOPT_F32, "16-bit streams only");
   using Chunk = SumsqChunk<WHICH, AD, MXOPT_F32, NT>;
   (void)prep;  // no stage (the launcher's condition)
@@ -463,69 +462,23 @@ __global__ __launch_bounds__(kThreads) void sumsq16_multi_kernel(const DevTensor
     if (!more) break;
     c += (uint32_t)NCH * stride;
   }
-  unsigned long long unused = 0;
-  block_sum(acc_sum, unused);
-  if (tid == 0) partial_sum[blockIdx.x] = acc_sum;
+  finish_partial(acc_sum, partial_sum, fold);
 }
 
-// Pass 2: one workgroup folds the partials in a fixed order and derives norm and scale.  Bound by the latency of one
-// memory round trip, not by bytes (16,384 partials are 128 KB): every lane issues its next kFinishLoads loads before
-// it adds the first of them, and the workgroup has as many lanes as the partials can use.  With 256 lanes adding one
-// load after the other it took 18.5 us for 16,384 partials and 6.6 us for 4,096, between two passes that wait for it.
-constexpr int kFinishLoads = 8;
+// Pass 2 as a kernel of its own: one workgroup, as many lanes as the partial sums can use.
 template <int THREADS>
-__global__ __launch_bounds__(THREADS) void norm_finish_kernel(const double* __restrict__ partial_sum,
-                                                              uint32_t npartials, double max_norm, int has_max,
-                                                              int clip_mode, mxopt_norm_result* __restrict__ out) {
-  __shared__ double wave_sums[THREADS / 64];
-  const MXOPT_GLOBAL double* part = global_ptr<double>((const void*)partial_sum);
-  double s = 0.0;
-  for (uint32_t base = 0; base < npartials; base += THREADS * kFinishLoads) {
-    double x[kFinishLoads];
-#pragma unroll
-    for (int k = 0; k < kFinishLoads; ++k) {
-      const uint32_t i = base + (uint32_t)k * THREADS + threadIdx.x;
-      x[k] = i < npartials ? part[i] : 0.0;
-    }
-#pragma unroll
-    for (int k = 0; k < kFinishLoads; ++k) s += x[k];
-  }
-  s = wave_sum(s);
-  if ((threadIdx.x & 63u) == 0) wave_sums[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    s = wave_sums[0];
-#pragma unroll
-    for (int w = 1; w < THREADS / 64; ++w) s += wave_sums[w];
-  }
-  if (threadIdx.x == 0) {
-    const double sumsq = s;
-    const double norm = sqrt(sumsq);
-    const float norm32 = (float)norm;
-    float scale = 1.0f;
-    if (has_max) {
-      if (clip_mode == MXOPT_CLIP_ALWAYS_MULTIPLY) {
-        // optimizers/mod.rs:87-96: all float32 scalars
-        float d = norm32 + (float)1e-6;
-        float q = (float)max_norm / d;
-        scale = (q != q) ? q : fminf(q, 1.0f);  // a NaN norm gives a NaN scale
-      } else {
-        // gradients/mod.rs:255-270: float64 on the host, gradients unchanged when norm <= max
-        if (!(norm <= max_norm)) scale = (float)(max_norm / (norm + 1e-6));
-      }
-    }
-    out->sumsq = sumsq;
-    out->norm = norm;
-    out->norm_f32 = norm32;
-    out->scale = scale;
-    // NaN: some element was a NaN or an infinity (1).  +Inf: every element was finite and their squares left
-    // float32 range (2): the reference goes on with a clip factor of 0 there, and so does `scale` above.
-    out->nonfinite = (sumsq != sumsq) ? 1ull : (sumsq - sumsq == 0.0) ? 0ull : 2ull;
-  }
+__global__ __launch_bounds__(THREADS) void norm_finish_kernel(NormFold fold, uint32_t npartials) {
+  const double s = sum_of_partials<THREADS, false>(fold.partials, npartials);
+  if (threadIdx.x == 0) write_outcome(s, fold);
+}
+
+__global__ void clear_arrivals_kernel(uint32_t* arrived) { *arrived = 0u; }
+void launch_clear_arrivals(hipStream_t stream, uint32_t* arrived) {
+  hipLaunchKernelGGL(clear_arrivals_kernel, dim3(1), dim3(1), 0, stream, arrived);
 }
 
 template <int MODE, int AD, int GD>
-static void launch_sumsq_t(const Launch& L, const DevPrep& prep, int first, double* ps) {
+static void launch_sumsq_t(const Launch& L, const DevPrep& prep, int first, double* ps, const NormFold& fold) {
   if constexpr (MODE == 2) {
     if (ps == nullptr) { launch_accumulate<AD, GD>(L, prep, first); return; }
   }
@@ -533,43 +486,44 @@ static void launch_sumsq_t(const Launch& L, const DevPrep& prep, int first, doub
   // and 97, 256 M 253 and 239, 1.72 G 1,604 and 1,464 (64 M 68 and 69); 16-bit both 256 M 174 and 167, 596 M 377 and 361.  One
   // stream and two float32 ones gain nothing.
   constexpr Crowd kCrowd = MODE != 3 || GD == MXOPT_F32 ? kNoLimit : AD == MXOPT_F32 ? Crowd{2, 90, 96} : Crowd{4, 90, 256};
-  if (L.nontemporal) MXOPT_LAUNCH_CROWD((sumsq_kernel<MODE, AD, GD, true>), kCrowd, L, prep, first, ps);
-  else MXOPT_LAUNCH((sumsq_kernel<MODE, AD, GD, false>), L, prep, first, ps);
+  if (L.nontemporal) MXOPT_LAUNCH_CROWD((sumsq_kernel<MODE, AD, GD, true>), kCrowd, L, prep, first, ps, fold);
+  else MXOPT_LAUNCH((sumsq_kernel<MODE, AD, GD, false>), L, prep, first, ps, fold);
 }
 
 template <int MODE, int AD>
-static bool sumsq_for_ad(int gd, const Launch& L, const DevPrep& prep, int first, double* ps) {
-  if (MODE < 2) { launch_sumsq_t<MODE, AD, MXOPT_F32>(L, prep, first, ps); return true; }
+static bool sumsq_for_ad(int gd, const Launch& L, const DevPrep& prep, int first, double* ps, const NormFold& fold) {
+  if (MODE < 2) { launch_sumsq_t<MODE, AD, MXOPT_F32>(L, prep, first, ps, fold); return true; }
   switch (gd) {
-    case MXOPT_F32: launch_sumsq_t<MODE, AD, MXOPT_F32>(L, prep, first, ps); return true;
-    case MXOPT_BF16: launch_sumsq_t<MODE, AD, MXOPT_BF16>(L, prep, first, ps); return true;
-    case MXOPT_F16: launch_sumsq_t<MODE, AD, MXOPT_F16>(L, prep, first, ps); return true;
+    case MXOPT_F32: launch_sumsq_t<MODE, AD, MXOPT_F32>(L, prep, first, ps, fold); return true;
+    case MXOPT_BF16: launch_sumsq_t<MODE, AD, MXOPT_BF16>(L, prep, first, ps, fold); return true;
+    case MXOPT_F16: launch_sumsq_t<MODE, AD, MXOPT_F16>(L, prep, first, ps, fold); return true;
   }
   return false;
 }
 
 template <int MODE>
-static bool sumsq_for_mode(int ad, int gd, const Launch& L, const DevPrep& prep, int first, double* ps) {
+static bool sumsq_for_mode(int ad, int gd, const Launch& L, const DevPrep& prep, int first, double* ps, const NormFold& fold) {
   switch (ad) {
-    case MXOPT_F32: return sumsq_for_ad<MODE, MXOPT_F32>(gd, L, prep, first, ps);
-    case MXOPT_BF16: return sumsq_for_ad<MODE, MXOPT_BF16>(gd, L, prep, first, ps);
-    case MXOPT_F16: return sumsq_for_ad<MODE, MXOPT_F16>(gd, L, prep, first, ps);
+    case MXOPT_F32: return sumsq_for_ad<MODE, MXOPT_F32>(gd, L, prep, first, ps, fold);
+    case MXOPT_BF16: return sumsq_for_ad<MODE, MXOPT_BF16>(gd, L, prep, first, ps, fold);
+    case MXOPT_F16: return sumsq_for_ad<MODE, MXOPT_F16>(gd, L, prep, first, ps, fold);
   }
   return false;
 }
 
 template <int AD, int NCH>
-static void launch_sumsq16_multi(int which, const Launch& L, const DevPrep& prep, double* ps) {
+static void launch_sumsq16_multi(int which, const Launch& L, const DevPrep& prep, double* ps, const NormFold& fold) {
   if (which == 0) {
-    if (L.nontemporal) MXOPT_LAUNCH((sumsq16_multi_kernel<AD, 0, true, NCH>), L, prep, 0, ps);
-    else MXOPT_LAUNCH((sumsq16_multi_kernel<AD, 0, false, NCH>), L, prep, 0, ps);
+    if (L.nontemporal) MXOPT_LAUNCH((sumsq16_multi_kernel<AD, 0, true, NCH>), L, prep, 0, ps, fold);
+    else MXOPT_LAUNCH((sumsq16_multi_kernel<AD, 0, false, NCH>), L, prep, 0, ps, fold);
   } else {
-    if (L.nontemporal) MXOPT_LAUNCH((sumsq16_multi_kernel<AD, 1, true, NCH>), L, prep, 0, ps);
-    else MXOPT_LAUNCH((sumsq16_multi_kernel<AD, 1, false, NCH>), L, prep, 0, ps);
+    if (L.nontemporal) MXOPT_LAUNCH((sumsq16_multi_kernel<AD, 1, true, NCH>), L, prep, 0, ps, fold);
+    else MXOPT_LAUNCH((sumsq16_multi_kernel<AD, 1, false, NCH>), L, prep, 0, ps, fold);
   }
 }
 
-bool launch_sumsq(int mode, int ad, int gd, const Launch& L, const DevPrep& prep, int first, double* partial_sum) {
+bool launch_sumsq(int mode, int ad, int gd, const Launch& L, const DevPrep& prep, int first, double* partial_sum,
+                  const NormFold& fold) {
   // The plain norm of a 16-bit stream over many small tensors has a kernel of its own (option pipelined_norm:
   // 0 never, 1 always, 2 / 4 = that many chunks per trip where the chunks are partly empty).  Measured on
   // 10,000 tensors of 64 ... 65,536 elements: 45.9 against 53.1 us; on the Qwen3-1.7B list, whose chunks are
@@ -577,21 +531,21 @@ bool launch_sumsq(int mode, int ad, int gd, const Launch& L, const DevPrep& prep
   const bool wanted = L.pipelined_norm == 1 || (L.pipelined_norm > 1 && L.partial_chunks);
   if (mode < 2 && partial_sum != nullptr && prep.flags == 0 && wanted) {
     if (ad == MXOPT_BF16) {
-      if (L.pipelined_norm >= 4) launch_sumsq16_multi<MXOPT_BF16, 4>(mode, L, prep, partial_sum);
-      else launch_sumsq16_multi<MXOPT_BF16, 2>(mode, L, prep, partial_sum);
+      if (L.pipelined_norm >= 4) launch_sumsq16_multi<MXOPT_BF16, 4>(mode, L, prep, partial_sum, fold);
+      else launch_sumsq16_multi<MXOPT_BF16, 2>(mode, L, prep, partial_sum, fold);
       return true;
     }
     if (ad == MXOPT_F16) {
-      if (L.pipelined_norm >= 4) launch_sumsq16_multi<MXOPT_F16, 4>(mode, L, prep, partial_sum);
-      else launch_sumsq16_multi<MXOPT_F16, 2>(mode, L, prep, partial_sum);
+      if (L.pipelined_norm >= 4) launch_sumsq16_multi<MXOPT_F16, 4>(mode, L, prep, partial_sum, fold);
+      else launch_sumsq16_multi<MXOPT_F16, 2>(mode, L, prep, partial_sum, fold);
       return true;
     }
   }
   switch (mode) {
-    case 0: return sumsq_for_mode<0>(ad, gd, L, prep, first, partial_sum);
-    case 1: return sumsq_for_mode<1>(ad, gd, L, prep, first, partial_sum);
-    case 2: return sumsq_for_mode<2>(ad, gd, L, prep, first, partial_sum);
-    case 3: return sumsq_for_mode<3>(ad, gd, L, prep, first, partial_sum);
+    case 0: return sumsq_for_mode<0>(ad, gd, L, prep, first, partial_sum, fold);
+    case 1: return sumsq_for_mode<1>(ad, gd, L, prep, first, partial_sum, fold);
+    case 2: return sumsq_for_mode<2>(ad, gd, L, prep, first, partial_sum, fold);
+    case 3: return sumsq_for_mode<3>(ad, gd, L, prep, first, partial_sum, fold);
   }
   return false;
 }
@@ -661,15 +615,12 @@ bool launch_synth(int od, void* out, uint64_t n, uint64_t seed, uint64_t first_i
   return false;
 }
 
-void launch_norm_finish(hipStream_t stream, const double* partial_sum, uint32_t npartials, double max_norm,
-                        int has_max, int clip_mode, mxopt_norm_result* d_out) {
+void launch_norm_finish(hipStream_t stream, const NormFold& fold, uint32_t npartials) {
   // 1,024 lanes as soon as 256 would need a second trip.
-  if (npartials <= 256u * kFinishLoads)
-    hipLaunchKernelGGL(norm_finish_kernel<256>, dim3(1), dim3(256), 0, stream, partial_sum, npartials, max_norm, has_max,
-                       clip_mode, d_out);
+  if (npartials <= 256u * kFoldLoads)
+    hipLaunchKernelGGL(norm_finish_kernel<256>, dim3(1), dim3(256), 0, stream, fold, npartials);
   else
-    hipLaunchKernelGGL(norm_finish_kernel<1024>, dim3(1), dim3(1024), 0, stream, partial_sum, npartials, max_norm,
-                       has_max, clip_mode, d_out);
+    hipLaunchKernelGGL(norm_finish_kernel<1024>, dim3(1), dim3(1024), 0, stream, fold, npartials);
 }
 
 // One result of the second pass copied into pinned host memory by a kernel (a 32-byte store over the

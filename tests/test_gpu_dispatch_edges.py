@@ -136,3 +136,35 @@ def test_widening_transform(mx, ctx, n, dtype):
     out = torch.full((n + 4,), 7.0, dtype=torch.float32, device="cuda")
     ctx.grad_transform(ctx.table([mx.TensorSpec(g=g, g_out=out[:n])]), mx.make_prep(pre_mul=0.5))
     assert torch.equal(out[:n], g.float() * 0.5) and bool((out[n:] == 7.0).all())
+
+
+@pytest.mark.parametrize("chunks", [1, 2, 63, 64, 65, 1024])
+@pytest.mark.parametrize("which", ["norm", "sum", "list"])
+def test_norm_folded_by_the_last_workgroup(mx, ctx, chunks, which):
+    """Up to 64 partial sums are folded by the workgroup that stores the last one, more by a second kernel: the same call
+    again and again (the count of arrivals starts from zero each time), in two dtype groups, next to a call that fails
+    behind its first launch.  Elements are powers of two, so the sums are exact in any order."""
+    import torch
+    n = (chunks - 1) * CHUNK + 5
+    a, b = torch.full((n,), 2.0 ** -6, device="cuda"), torch.full((9,), 2.0 ** -3, dtype=torch.bfloat16, device="cuda")
+    res = ctx.norm_result()
+    if which == "norm":
+        table = ctx.table([mx.TensorSpec(g=a), mx.TensorSpec(g=b)])
+        call, want = (lambda: ctx.global_norm(table, res, max_norm=1.0)), n * 2.0 ** -12 + 9 * 2.0 ** -6
+    elif which == "sum":
+        table = ctx.table([mx.TensorSpec(g=a, g_out=a.clone())])
+        call, want = (lambda: ctx.accumulate_norm_only(table, res, max_norm=1.0)), n * 2.0 ** -10
+    else:
+        table = ctx.table([mx.TensorSpec(g=a)])
+        table.set_pending([[a.clone()]])
+        call, want = (lambda: ctx.norm_with_pending_list(table, res, max_norm=1.0)), n * 2.0 ** -10
+    for k in range(5):
+        call()
+        r = ctx.read_norm_result(res)
+        assert r.sumsq == want and r.nonfinite == 0, (k, r.sumsq, want)
+        if which == "list":
+            # the group of float32 rows goes out, bf16 rows with float32 pending streams have no kernel
+            bad = ctx.table([mx.TensorSpec(g=a), mx.TensorSpec(g=b)])
+            bad.set_pending([[a.clone(), torch.zeros(9, device="cuda")]])
+            with pytest.raises(Exception):
+                ctx.norm_with_pending_list(bad, res, max_norm=1.0)
