@@ -274,6 +274,7 @@ static int run_sumsq(mxopt_ctx* ctx, const mxopt_table* t, int mode, int first, 
     // 6.04 TB/s for acc += g on region-interleaved memory).
     Launch L = make_launch(ctx, t, g, want || mode != 2 || ctx->persistent != 0 || (ctx->persistent_accumulate != 0 && !first));
     if (mode == 2 && !want && ctx->persistent_accumulate == 0) offer_tiles(ctx, L, t->d_tiles + g.tile_begin, g.ntiles, g.whole_tiles, g.elems);
+    L.in_place = t->sums_in_place;
     if (L.grid < g.nchunks) L.grid = reduction_grid(g);  // a bounded grid: the size this reduction wants
     if (mode != 2) L.nontemporal = ctx->nontemporal_reduce;
     const int ad = mode == 0 ? g.gd : g.god;
@@ -334,10 +335,13 @@ void fill_dev_tensor(const mxopt_tensor& s, DevTensor& d) {
   }
 }
 
-static bool table_in_place(const std::vector<mxopt_tensor>& rows) {
-  for (const mxopt_tensor& r : rows)
-    if (r.n != 0 && r.p_out != r.p) return false;
-  return true;
+static void note_places(mxopt_table* t) {
+  t->in_place = t->sums_in_place = true;
+  for (const mxopt_tensor& r : t->host) {
+    if (r.n == 0) continue;
+    if (r.p_out != r.p) t->in_place = false;
+    if (r.p != nullptr && r.p != r.g_out) t->sums_in_place = false;
+  }
 }
 
 uint64_t chunks_of(const DevTensor& d) {
@@ -617,7 +621,7 @@ int mxopt_table_build(mxopt_ctx* ctx, const mxopt_tensor* tensors, size_t n, mxo
     return hip_fail(ctx, e, "mxopt_table_build");
   }
   t->d_tiles = reinterpret_cast<DevTile*>(t->d_chunks + tiles_at);
-  t->in_place = table_in_place(t->host);
+  note_places(t);
   MXOPT_DEBUG("table built: %zu tensors, %llu elements, %llu chunks, %zu dtype group(s)", n,
               (unsigned long long)t->total_elems, (unsigned long long)t->num_chunks, t->groups.size());
   *out = t;
@@ -685,7 +689,7 @@ int mxopt::table_retarget_quiet(mxopt_table* t, const mxopt_tensor* tensors, siz
   DeviceGuard guard(ctx->device);
   t->host.assign(tensors, tensors + n);
   t->dev.swap(dev);
-  t->in_place = table_in_place(t->host);
+  note_places(t);
   MXOPT_DEBUG("table retargeted: %zu tensors keep their chunk list", n);
   why->clear();
   return upload_descriptors(t);

@@ -127,6 +127,7 @@ struct mxopt_table {
   mxopt::DevChunk* d_chunks = nullptr;
   mxopt::DevTile* d_tiles = nullptr;          // behind the chunks, in their allocation
   bool in_place = false;                      // p_out == p in every tensor
+  bool sums_in_place = false;                 // p is NULL or g_out in every tensor: accumulation reads what it writes
   uint64_t total_elems = 0;
   uint64_t num_chunks = 0;
   uint32_t have_mask = 0;                     // which pointers are non-NULL in every non-empty tensor

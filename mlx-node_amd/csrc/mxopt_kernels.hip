@@ -10,14 +10,14 @@ namespace mxopt {
 // Update kernel, chunk by chunk.
 // ------------------------------------------------------------------------------------
 
-template <int PD, int GD, int OD, int G2, class Math, bool NT>
+template <int PD, int GD, int OD, int G2, class Math, bool NT, bool NTP>
 __global__ __launch_bounds__(kThreads) void update_kernel(const DevTensor* __restrict__ T,
                                                           const DevChunk* __restrict__ C, DevTensor one,
                                                           uint32_t nchunks, Math math, DevPrep prep) {
   if (skip_requested(prep)) return;
   const PrepRegs pr = load_prep(prep);
   for (uint32_t c = blockIdx.x; c < nchunks; c += gridDim.x)
-    update_chunk<PD, GD, OD, G2, Math, NT>(locate(T, C, one, c), threadIdx.x, math, pr);
+    update_chunk<PD, GD, OD, G2, Math, NT, NTP>(locate(T, C, one, c), threadIdx.x, math, pr);
 }
 
 // ------------------------------------------------------------------------------------
@@ -115,13 +115,18 @@ constexpr Crowd kUpdateCrowd = Math::kM || (Math::kV && PD == MXOPT_F32 && GD ==
 
 template <int PD, int GD, int OD, int G2, class Math>
 static void launch_update_t(const Launch& L, const Math& math, const DevPrep& prep) {
+  if (!L.nontemporal) {
+    MXOPT_LAUNCH((update_kernel<PD, GD, OD, G2, Math, false, false>), L, math, prep);
+    return;
+  }
   if constexpr (OD == PD) {
     if (launch_update_tiles<PD, GD, G2>(L, math, prep)) return;
+    if (L.in_place) {
+      MXOPT_LAUNCH_CROWD((update_kernel<PD, GD, OD, G2, Math, true, true>), (kUpdateCrowd<PD, GD, Math>), L, math, prep);
+      return;
+    }
   }
-  if (L.nontemporal)
-    MXOPT_LAUNCH_CROWD((update_kernel<PD, GD, OD, G2, Math, true>), (kUpdateCrowd<PD, GD, Math>), L, math, prep);
-  else
-    MXOPT_LAUNCH((update_kernel<PD, GD, OD, G2, Math, false>), L, math, prep);
+  MXOPT_LAUNCH_CROWD((update_kernel<PD, GD, OD, G2, Math, true, false>), (kUpdateCrowd<PD, GD, Math>), L, math, prep);
 }
 
 template <int PD, int GD, class Math>

@@ -24,7 +24,7 @@ struct Launch {
   const DevTile* tiles = nullptr;
   uint32_t ntiles = 0;
   uint32_t tiles_per_cu = 0;
-  bool in_place = false;             // p_out == p in every tensor
+  bool in_place = false;             // what is written has been read: p_out == p (updates), the sum's own buffer (accumulation)
   hipStream_t stream = nullptr;
   int nontemporal = 1;               // non-zero: streaming-hint loads and stores
   int pipelined_norm = 2;            // plain 16-bit norms take the software-pipelined kernel

@@ -27,8 +27,8 @@ __device__ __forceinline__ float accumulate_op(float acc, float g, bool first) {
   return Elem<AD>::round(s);
 }
 
-// GROUP: elements per lane and group, 0 = the mode's own.
-template <int MODE, int AD, int GD, bool NT, int GROUP = 0>
+// GROUP: elements per lane and group, 0 = the mode's own.  NTS: the sum's stores stream.
+template <int MODE, int AD, int GD, bool NT, int GROUP = 0, bool NTS = NT>
 struct SumsqChunk {
   static constexpr bool kTwoStreams = MODE >= 2;
   static constexpr int E = GROUP ? GROUP : (AD != MXOPT_F32 || (kTwoStreams && GD != MXOPT_F32)) ? 8 : 4;
@@ -59,12 +59,13 @@ struct SumsqChunk {
   // The new sum of group j.  A streaming store pays off where the pass has just read the line it writes; the
   // first pass of a cycle writes lines nobody read (acc = widen(g)), and there streaming stores cost 60 % more
   // time (measured on the bf16 -> float32 pass, whose float32 stores come in sector-sharing pairs that
-  // store_group no longer streams anyway).  A later pass into another buffer than it reads is no different.
+  // store_group no longer streams anyway).  A later pass into another buffer than it reads is no different (NTS false: a
+  // branch on the buffers here would have the compiler merge both stores into plain ones).
   static __device__ __forceinline__ void store_sum(const ChunkView& cv, uint32_t tid, int j, bool first,
                                                    const float (&v)[E]) {
     const uint64_t off = cv.start + (uint64_t)(j * kThreads + tid) * E;
-    if (first || (cv.t.p != nullptr && cv.t.p != cv.t.g_out)) store_group<AD, E, false>(cv.t.g_out, off, v);
-    else store_group<AD, E, NT>(cv.t.g_out, off, v);
+    if (first) store_group<AD, E, false>(cv.t.g_out, off, v);
+    else store_group<AD, E, NTS>(cv.t.g_out, off, v);
   }
 
   // Group j of the sum of the two streams, rounded as a store rounds it (bf16 + bf16 -> bf16 and friends).
@@ -273,33 +274,33 @@ __global__ __launch_bounds__(kThreads) void sumsq_kernel(const DevTensor* __rest
 }
 
 // Accumulation that is not asked for the norm.  The first pass of a cycle writes lines nobody read, in groups of 8 where a
-// stream has 16 bits (of 1.72 G elements in 1,608 us, in groups of 4 in 1,857); later passes read what they write and take
-// groups of 4, so that every access is one that streams (see load_group).  Later passes, microseconds in groups of 8 and of 4:
-// bf16 into float32 1.72 G elements 3,103 and 2,972, 10,000 tensors of 64 - 65,536 179 and 150; bf16 into bf16 596 M 654 and
-// 600, the 10,000 tensors 115 and 92.
-template <int AD, int GD, bool NT, bool FIRST>
+// stream has 16 bits (of 1.72 G elements in 1,608 us, in groups of 4 in 1,857).  Later passes read what they write and take
+// groups of 4, so that every access is one that streams (see load_group): microseconds in groups of 8 and of 4, bf16 into
+// float32 32 M elements 61 and 55, 128 M 236 and 210, 10,000 tensors of 64 - 65,536 181 and 150; float32 into float32 64 M 148 and
+// 126.  A 16-bit gradient into a long float32 buffer goes in groups of 8 again (kInPlaceWide), with two workgroups per compute
+// unit: 128 M 208, 256 M 412 (in groups of 4 430), 1.72 G 2,580 (2,970).
+enum AccumulateKind { kFirstPass, kInPlace, kInPlaceWide, kElsewhere };
+template <int AD, int GD, bool NT, int KIND>
 __global__ __launch_bounds__(kThreads) void accumulate_kernel(const DevTensor* __restrict__ T, const DevChunk* __restrict__ C,
                                                               DevTensor one, uint32_t nchunks, DevPrep prep) {
-  using Chunk = SumsqChunk<2, AD, GD, NT, FIRST ? 0 : 4>;
+  constexpr bool FIRST = KIND == kFirstPass;
+  using Chunk = SumsqChunk<2, AD, GD, NT, FIRST || KIND == kInPlaceWide ? 0 : 4, NT && KIND != kElsewhere>;
   const PrepRegs pr = load_prep(prep);
   for (uint32_t c = blockIdx.x; c < nchunks; c += gridDim.x) Chunk::accumulate(locate(T, C, one, c), pr, threadIdx.x, FIRST);
 }
 
-// Later passes into float32 by tiles (mxopt_tiles.h).  Microseconds in groups of 4 by chunks and by tiles: a bf16 gradient,
-// 128 M elements (16 tiles per compute unit) 214 and 218, 256 M 439 and 433, 430 M 727 and 706, 596 M 1,014 and 987, 1.72 G 2,984
-// and 2,809; a float32 one, 8 M (1 tile) 22 and 21, 64 M 147 and 131, 596 M 1,293 and 1,134.  16-bit sums gain nothing (596 M
-// 587 and 579, 1.72 G 1,737 and 1,748) and keep the chunks.
-template <int GD>
+// Later passes of float32 into float32 by tiles (mxopt_tiles.h): microseconds by chunks and by tiles 64 M elements 126 and 130, 256 M
+// 521 and 509, 596 M 1,205 and 1,145.
 __global__ __launch_bounds__(kTileThreads) void accumulate_tile_kernel(const DevTensor* __restrict__ T,
                                                                        const DevChunk* __restrict__ C, DevTensor one,
                                                                        uint32_t nchunks, const DevTile* __restrict__ tiles,
                                                                        DevPrep prep) {
-  constexpr int AD = MXOPT_F32;
+  constexpr int AD = MXOPT_F32, GD = MXOPT_F32;
   using Chunk = SumsqChunk<2, AD, GD, true, 4>;
   constexpr int U = kTileChunks;
   const uint32_t tid = threadIdx.x;
   const TileView tv = this_tile(T, one, nchunks, tiles);
-  if (!tv.whole || (tv.t.p != nullptr && tv.t.p != tv.t.g_out)) {  // into another buffer the stores must not stream (see store_sum)
+  if (!tv.whole) {
     const PrepRegs pr = load_prep(prep);
     chunks_of_tile(T, C, one, tv.tile, [&](const ChunkView& cv, uint32_t lane) { Chunk::accumulate(cv, pr, lane, false); });
     return;
@@ -328,29 +329,40 @@ __global__ __launch_bounds__(kTileThreads) void accumulate_tile_kernel(const Dev
 
 // Microseconds without a limit and with it.  First pass: 16-bit into float32 32 M elements 41 and 40, 128 M 146 and 133, 1.72 G
 // 1,908 and 1,598; into 16 bits 128 M 92 and 87, 596 M 421 and 372 (32 M 27 and 28; 10,000 tensors of 64 - 65,536 74 and 80);
-// float32 128 M 189 and 172, 256 M 379 and 335.  Later passes: 16-bit into float32, the 10,000 tensors 149 and 139; into 16 bits 128 M
-// 129 and 127, 256 M 263 and 251, 596 M 595 and 570 (the 10,000 tensors 85 and 91).
-template <int AD, int GD, bool FIRST>
-constexpr Crowd kAccumulateCrowd =
-    AD != MXOPT_F32 ? (FIRST ? Crowd{5, 90, 128} : Crowd{4, 90, 128})
-                    : GD != MXOPT_F32 ? (FIRST ? Crowd{5, 75, 16} : Crowd{4, 75, 16}) : (FIRST ? Crowd{2, 75, 16} : kNoLimit);
+// float32 128 M 189 and 172, 256 M 379 and 335.  Later passes: into float32, the 10,000 tensors, of 16 bits 150 and 140, of 32 191 and
+// 172; of 16 bits in groups of 8 (two a unit) 128 M 236 and 208; into 16 bits 256 M 263 and 254, 596 M 598 and 573 (the 10,000 tensors
+// 85 and 91).
+template <int AD, int GD, int KIND>
+constexpr Crowd kAccumulateCrowd = KIND == kElsewhere ? kNoLimit
+                                   : KIND == kInPlaceWide ? Crowd{2, 90, 128}
+                                   : AD != MXOPT_F32 ? (KIND == kFirstPass ? Crowd{5, 90, 128} : Crowd{4, 90, 128})
+                                   : KIND == kInPlace ? Crowd{4, 75, 16}
+                                   : GD != MXOPT_F32 ? Crowd{5, 75, 16} : Crowd{2, 75, 16};
+
+template <int AD, int GD, int KIND>
+static void launch_accumulate_kind(const Launch& L, const DevPrep& prep) {
+  if (L.nontemporal) MXOPT_LAUNCH_CROWD((accumulate_kernel<AD, GD, true, KIND>), (kAccumulateCrowd<AD, GD, KIND>), L, prep);
+  else MXOPT_LAUNCH((accumulate_kernel<AD, GD, false, KIND>), L, prep);
+}
 
 template <int AD, int GD>
 static void launch_accumulate(const Launch& L, const DevPrep& prep, int first) {
-  if constexpr (AD == MXOPT_F32) {
-    if (!first && L.ntiles != 0 && L.tiles_per_cu >= (GD == MXOPT_F32 ? 2u : 32u)) {
-      hipLaunchKernelGGL(accumulate_tile_kernel<GD>, dim3(L.ntiles), dim3(kTileThreads), kOnePerCu, L.stream, L.tensors,
-                         L.chunks, L.one, L.nchunks, L.tiles, prep);
+  if (first) { launch_accumulate_kind<AD, GD, kFirstPass>(L, prep); return; }
+  if (!L.in_place) { launch_accumulate_kind<AD, GD, kElsewhere>(L, prep); return; }
+  if constexpr (AD == MXOPT_F32 && GD == MXOPT_F32) {
+    if (L.ntiles != 0 && L.tiles_per_cu >= 32u) {
+      hipLaunchKernelGGL(accumulate_tile_kernel, dim3(L.ntiles), dim3(kTileThreads), kOnePerCu, L.stream, L.tensors, L.chunks,
+                         L.one, L.nchunks, L.tiles, prep);
       return;
     }
   }
-  if (L.nontemporal) {
-    if (first) MXOPT_LAUNCH_CROWD((accumulate_kernel<AD, GD, true, true>), (kAccumulateCrowd<AD, GD, true>), L, prep);
-    else MXOPT_LAUNCH_CROWD((accumulate_kernel<AD, GD, true, false>), (kAccumulateCrowd<AD, GD, false>), L, prep);
-  } else {
-    if (first) MXOPT_LAUNCH((accumulate_kernel<AD, GD, false, true>), L, prep);
-    else MXOPT_LAUNCH((accumulate_kernel<AD, GD, false, false>), L, prep);
+  if constexpr (AD == MXOPT_F32 && GD != MXOPT_F32) {
+    if (L.nontemporal && crowd_lds(L, kAccumulateCrowd<AD, GD, kInPlaceWide>) != 0) {
+      launch_accumulate_kind<AD, GD, kInPlaceWide>(L, prep);
+      return;
+    }
   }
+  launch_accumulate_kind<AD, GD, kInPlace>(L, prep);
 }
 
 // ------------------------------------------------------------------------------------

@@ -4,7 +4,8 @@
 // row it moves in between.  A chunk's workgroup writes 8 or 16 KB of one stream, then of the next, while its three or more
 // neighbours on the compute unit are in other phases.  A tile's workgroup is alone on its compute unit, loads its streams one
 // after the other and stores them one after the other, 64 or 128 KB each.  In memory of one region (where a plain allocation
-// lies) that is 5.3 - 5.5 TB/s by chunks and 5.8 - 6.1 by tiles; in memory of two regions, 6.1, there is no difference.
+// lies) a long list of several streams reaches 5.8 - 6.1 TB/s by tiles, 5.5 - 5.8 by chunks with few workgroups per compute unit, 5.3 -
+// 5.5 with many; in memory of two regions all of them 6.1.
 // Bare streams, 4 read and 3 written, float32, 596 M elements: 256 lanes x 16 elements 3,150 us, 1,024 x 16 in the same
 // order 3,160, stream by stream 2,850; 512 x 32 3,050; 1,024 x 8 3,190.  Two 16-bit streams and two float32 ones: 2,490 by chunks,
 // 1,024 x 16 2,350, 1,024 x 32 2,140.

@@ -36,7 +36,10 @@ struct GradientOf {
   }
 };
 
-template <int PD, int GD, int OD, int G2, class Math, bool NT>
+// NTP: the parameters' stores stream too, which pays off only where the line was read (p_out == p in every tensor of the
+// launch).  A branch on the two pointers here had the compiler merge both stores into plain ones: plain SGD of 596 M bf16 elements
+// 674 us, 592 now, of 128 M 146 and 130; bf16 AdamW of 256 M 998 and 951 (with two workgroups per compute unit).
+template <int PD, int GD, int OD, int G2, class Math, bool NT, bool NTP>
 __device__ __forceinline__ void update_chunk(const ChunkView& cv, uint32_t tid, const Math& math, const PrepRegs& pr) {
   using Gradient = GradientOf<GD, G2>;
   constexpr bool kHasG2 = Gradient::kHasG2, kSum16 = Gradient::kSum16;
@@ -102,8 +105,7 @@ __device__ __forceinline__ void update_chunk(const ChunkView& cv, uint32_t tid, 
 #pragma unroll
     for (int j = 0; j < U; ++j) {
       const uint64_t off = start + (uint64_t)(j * kThreads + tid) * E;
-      if (PO == P) store_group<OD, E, NT>(PO, off, p[j]);  // streaming only where the line was read
-      else store_group<OD, E, false>(PO, off, p[j]);
+      store_group<OD, E, NTP>(PO, off, p[j]);
       if (Math::kM) store_group<MXOPT_F32, E, NT>(M, off, m[j]);
       if (use_v) store_group<MXOPT_F32, E, NT>(V, off, v[j]);
     }

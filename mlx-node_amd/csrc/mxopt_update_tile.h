@@ -7,10 +7,10 @@
 
 namespace mxopt {
 
-// See mxopt_tiles.h for what a tile gains.  Microseconds by chunks and by tiles, plain memory of one region: AdamW of 596 M
-// float32 elements 3,140 and 2,833, bf16 with float32 moments 2,453 and 2,224, of 1.72 G 7,010 and 6,315, with a float32 buffer
-// and a bf16 micro-batch folded in 8,460 and 7,750; SGD with momentum of 1.72 G float32 6,460 and 5,650; RMSprop of 596 M 2,183
-// and 1,958; plain SGD of 596 M bf16 651 and 585.  What did not help: the parameters stored row by row as they are computed
+// See mxopt_tiles.h for what a tile gains.  Microseconds by chunks as they were before (parameters' stores plain, as many
+// workgroups as fit) and by tiles, plain memory of one region: AdamW of 596 M float32 elements 3,140 and 2,833, bf16 with float32
+// moments 2,453 and 2,224, of 1.72 G 7,010 and 6,315, with a float32 buffer and a bf16 micro-batch folded in 8,460 and 7,750; SGD
+// with momentum of 1.72 G float32 6,460 and 5,650; RMSprop of 596 M 2,183 and 1,958; plain SGD of 596 M bf16 651 and 585.  What did not help: the parameters stored row by row as they are computed
 // (2 % slower: reads and writes mix again), a barrier between the streams' stores, workgroups that stay and walk the tiles
 // (4 % slower), tiles that begin at a multiple of their size in memory (nothing on a whole parameter list).
 //
@@ -32,7 +32,7 @@ __global__ __launch_bounds__(kTileThreads) void update_tile_kernel(const DevTens
   const TileView tv = this_tile(T, one, nchunks, tiles);
   if (!tv.whole) {
     chunks_of_tile(T, C, one, tv.tile, [&](const ChunkView& cv, uint32_t lane) {
-      update_chunk<PD, GD, PD, G2, Math, NT>(cv, lane, math, pr);
+      update_chunk<PD, GD, PD, G2, Math, NT, NT>(cv, lane, math, pr);
     });
     return;
   }
@@ -99,17 +99,17 @@ __global__ __launch_bounds__(kTileThreads) void update_tile_kernel(const DevTens
     ChunkView head = locate(T, C, one, tv.tile.entry);
     head.fast = false;
     head.len = 0;
-    update_chunk<PD, GD, PD, G2, Math, NT>(head, tid, math, pr);
+    update_chunk<PD, GD, PD, G2, Math, NT, NT>(head, tid, math, pr);
   }
 }
 
-// Where tiles begin to pay, in whole tiles per compute unit.  Microseconds by chunks and by tiles: float32 AdamW of 16 M
-// elements (2 tiles) 86 and 86, 24 M 130 and 124 (in memory of two regions 117 and 123), 48 M 251 and 240; SGD 8 M 33 and 34,
-// 16 M 65 and 60, 32 M 123 and 112; bf16 AdamW 64 M (8 tiles) 250
-// and 255, 96 M 369 and 372; plain bf16 SGD 64 M 71 and 76, 96 M (12 tiles) 111 and 108.  Below, the ramp of few large
-// workgroups costs more than their order gains.
+// Where tiles begin to pay, in whole tiles per compute unit.  Microseconds by chunks (streaming stores, two workgroups per compute
+// unit) and by tiles, memory of one region: float32 AdamW of 128 M elements (16 tiles) 622 and 631, 192 M (24) 948 and 936, 596 M 3,017 and
+// 2,874; SGD 128 M 438 and 443, 192 M 659 and 654, 596 M 2,146 and 1,988; bf16 AdamW 256 M (32) 951 and 997, 1.72 G 6,515 and
+// 6,301; plain bf16 SGD 256 M 264 and 271, 596 M (71) 592 and 578; a float32 buffer and a bf16 micro-batch folded into AdamW, 596 M
+// 2,754 and 2,688.  In memory of two regions the chunks stay ahead by 2 %.
 template <int PD, int GD, int G2, class Math>
-constexpr uint32_t kUpdateTilesPerCu = (PD == MXOPT_F32 && GD == MXOPT_F32 && G2 <= MXOPT_F32) ? (Math::kM ? 6 : 3) : Math::kM ? 16 : 12;
+constexpr uint32_t kUpdateTilesPerCu = (PD == MXOPT_F32 && GD == MXOPT_F32 && G2 <= MXOPT_F32) ? 24 : Math::kV ? 48 : 64;
 
 template <int PD, int GD, int G2, class Math>
 static bool launch_update_tiles(const Launch& L, const Math& math, const DevPrep& prep) {

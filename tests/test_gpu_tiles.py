@@ -174,7 +174,7 @@ def test_single_tensor(mx, ctx, n, shift):
 def test_rule_takes_tiles_for_long_lists_only(mx, ctx):
     """The default rule on both sides of its line gives the results of either route."""
     import torch
-    for n in (TILE * ctx.get_option("num_cus") * 3 - 5, TILE * ctx.get_option("num_cus") * 3 + 5):
+    for n in (TILE * ctx.get_option("num_cus") * 24 - 5, TILE * ctx.get_option("num_cus") * 24 + 5):
         gen = torch.Generator(device="cuda")
         gen.manual_seed(5)
         p = torch.empty(n, device="cuda").normal_(0.0, 0.5, generator=gen)
