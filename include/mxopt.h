@@ -30,7 +30,9 @@
  * HIP graphs: the kernel entry points (mxopt_adam ... mxopt_norm_with_pending_list) only launch
  * kernels -- no allocation, copy or memset -- once the first reduction call on a context has
  * allocated its per-workgroup partials buffer, so a step may be recorded into a graph after
- * one eager warm-up call.  mxopt_table_build, mxopt_table_set_step_scalars, mxopt_table_retarget
+ * one eager warm-up call.  A recorded reduction uses that buffer, which every reduction of the context shares: replays
+ * are ordered with the context's own work and with each other like calls on one stream (two reductions that overlap give
+ * wrong norms; later ones are right again).  mxopt_table_build, mxopt_table_set_step_scalars, mxopt_table_retarget
  * and mxopt_table_set_pending copy from host memory and stay outside a capture.
  */
 #ifndef MXOPT_H
@@ -437,9 +439,10 @@ int mxopt_sgd_plain_with_pending_list_each(mxopt_ctx* ctx, const mxopt_table* t,
 /* ---- global norm ------------------------------------------------------------------ */
 
 /* Sum of squares of the gradients (after prep's pre_mul / clamp_pre) over the whole
- * table: wavefront shuffle -> LDS -> one float64 partial per workgroup -> one
- * single-workgroup second pass; no atomics, run-to-run deterministic; the same pass yields the gradient-validity flag.  `which` = 0 reads
- * tensor.g, 1 reads tensor.g_out (the accumulation buffer).  If max_norm >= 0 the second
+ * table: wavefront shuffle -> LDS -> one float64 partial per workgroup -> a fold of the partials in a
+ * fixed order, by the workgroup that finishes last (up to 64 workgroups; it knows by an atomic count of arrivals) or by a
+ * second single-workgroup kernel (more, and under stream capture); run-to-run deterministic; the same pass yields the
+ * gradient-validity flag.  `which` = 0 reads tensor.g, 1 reads tensor.g_out (the accumulation buffer).  If max_norm >= 0 the second
  * pass also derives `scale` per `clip_mode`; otherwise scale = 1.  Writes *d_result
  * (device memory).  Replaces the square/sum/add chain of GradientUtils::clip_grad_norm
  * (optimizers/mod.rs:76-96), compute_gradient_norm (:43-55) and the per-tensor reductions

@@ -118,25 +118,41 @@ uint32_t persistent_grid(const mxopt_ctx* ctx, uint32_t nchunks) {
 
 static int ensure_partials(mxopt_ctx* ctx, size_t need) {
   if (need <= ctx->partial_cap) return MXOPT_OK;
-  constexpr size_t kFront = 256;  // the counter of arrivals, on lines of its own
   const size_t cap = std::max<size_t>(need, 4096);
-  char* base = nullptr;
-  HIP_TRY(ctx, hipMalloc((void**)&base, kFront + cap * sizeof(double)));
-  launch_clear_arrivals(ctx->stream, (uint32_t*)base);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) {
-    (void)hipFree(base);
-    return hip_fail(ctx, e, "clear_arrivals_kernel");
-  }
+  double* ps = nullptr;
+  HIP_TRY(ctx, hipMalloc((void**)&ps, cap * sizeof(double)));
   // Earlier launches may still be reading the old buffer.
-  if (ctx->d_arrived) {
+  if (ctx->d_partial_sum) {
     (void)hipStreamSynchronize(ctx->stream);
-    (void)hipFree(ctx->d_arrived);
+    (void)hipFree(ctx->d_partial_sum);
   }
-  ctx->d_arrived = (uint32_t*)base;
-  ctx->d_partial_sum = (double*)(base + kFront);
+  ctx->d_partial_sum = ps;
   ctx->partial_cap = cap;
   return MXOPT_OK;
+}
+
+// Whether the workgroups of the next call can count their arrivals.  Not while the stream is captured: a replay has no
+// number of its own in the count, may run beside other work of the context, and keeps pointers (a second kernel costs a
+// graph nothing, see finish_partial).  The counter's memory is the context's until its end; wherever its value is not
+// known, at first and behind a call that failed among its launches, a kernel on the stream sets it to zero.
+static bool can_count_arrivals(mxopt_ctx* ctx) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return false;
+  }
+  if (ctx->arrivals_known) return true;
+  constexpr size_t kLines = 256;  // lines that nothing else lies on
+  if (!ctx->d_arrived && hipMalloc((void**)&ctx->d_arrived, kLines) != hipSuccess) {
+    (void)hipGetLastError();
+    ctx->d_arrived = nullptr;
+    return false;
+  }
+  launch_clear_arrivals(ctx->stream, ctx->d_arrived);
+  if (hipGetLastError() != hipSuccess) return false;
+  ctx->arrivals = 0;
+  ctx->arrivals_known = true;
+  return true;
 }
 
 int check_launch(mxopt_ctx* ctx, const char* what) {
@@ -198,8 +214,9 @@ int begin_norm(mxopt_ctx* ctx, size_t npartials, double max_norm, int clip_mode,
   const int rc = ensure_partials(ctx, std::max<size_t>(npartials, 1));
   if (rc) return rc;
   fold->partials = ctx->d_partial_sum;
+  fold->count = can_count_arrivals(ctx) && npartials <= kMaxFolded ? (uint32_t)npartials : 0u;
   fold->arrived = ctx->d_arrived;
-  fold->count = npartials <= kMaxFolded ? (uint32_t)npartials : 0u;
+  fold->last_arrival = ctx->arrivals + fold->count - 1u;
   fold->has_max = max_norm >= 0.0;
   fold->clip_mode = clip_mode;
   fold->max_norm = max_norm;
@@ -208,16 +225,16 @@ int begin_norm(mxopt_ctx* ctx, size_t npartials, double max_norm, int clip_mode,
   return MXOPT_OK;
 }
 
-// The end of a call whose launches carried `fold`: `launched` workgroups.  A call that failed behind its first launch: those
-// workgroups have been counted, and the next call counts from zero.
+// The end of a call whose launches carried `fold`: `launched` workgroups, every one of which arrives exactly once.
 static int end_norm(mxopt_ctx* ctx, const NormFold& fold, size_t launched, int rc) {
-  if (rc == MXOPT_OK && fold.count != 0 && launched != fold.count)
-    rc = fail(ctx, MXOPT_ERR_FAILURE, "norm: workgroups launched and counted differ");
-  if (rc != MXOPT_OK) {
-    if (fold.count != 0 && launched != 0) launch_clear_arrivals(ctx->stream, fold.arrived);
+  if (fold.count != 0) {
+    if (rc == MXOPT_OK && launched != fold.count)
+      rc = fail(ctx, MXOPT_ERR_FAILURE, "norm: workgroups launched and counted differ");
+    ctx->arrivals += fold.count;
+    if (rc != MXOPT_OK) ctx->arrivals_known = false;  // a launch that reported an error may have happened or not
     return rc;
   }
-  if (fold.count != 0) return MXOPT_OK;
+  if (rc != MXOPT_OK) return rc;
   launch_norm_finish(ctx->stream, fold, (uint32_t)launched);
   return check_launch(ctx, "norm_finish_kernel");
 }
@@ -413,9 +430,10 @@ void mxopt_destroy(mxopt_ctx* ctx) {
     (void)hipStreamSynchronize(ctx->stream);
     (void)hipFree(ctx->d_norm_scratch);
   }
-  if (ctx->d_arrived) {
+  if (ctx->d_partial_sum || ctx->d_arrived) {
     (void)hipStreamSynchronize(ctx->stream);
-    (void)hipFree(ctx->d_arrived);
+    if (ctx->d_partial_sum) (void)hipFree(ctx->d_partial_sum);
+    if (ctx->d_arrived) (void)hipFree(ctx->d_arrived);
   }
   if (ctx->h_norm) (void)hipHostFree(ctx->h_norm);
   delete ctx;

@@ -105,7 +105,9 @@ struct mxopt_ctx {
   int pipelined_norm = 2;         // plain 16-bit norms: the software-pipelined kernel
   double* d_partial_sum = nullptr;            // one float64 partial per workgroup of a reduction
   size_t partial_cap = 0;
-  uint32_t* d_arrived = nullptr;              // NormFold::arrived, in front of the partial sums in their allocation
+  uint32_t* d_arrived = nullptr;              // NormFold::arrived, an allocation of its own
+  uint32_t arrivals = 0;                      // its value behind everything enqueued so far (modulo 2^32)
+  bool arrivals_known = false;                // ... which only counts where this is set
   double* d_static_partials = nullptr;        // this device's copy of the library's fixed partial-sum array
   mxopt_norm_result* d_norm_scratch = nullptr;  // result slot of the gradient utilities
   mxopt_norm_result* h_norm = nullptr;          // pinned: the norm that a gradient utility hands back

@@ -43,8 +43,9 @@ struct Launch {
 constexpr uint32_t kMaxFolded = 64;  // see finish_partial
 struct NormFold {
   const double* partials = nullptr;
-  uint32_t* arrived = nullptr;  // workgroups that have stored theirs; 0 between calls
+  uint32_t* arrived = nullptr;  // workgroups that have stored theirs, of all calls so far
   uint32_t count = 0;
+  uint32_t last_arrival = 0;    // what the last of the call's workgroups finds in *arrived
   int has_max = 0, clip_mode = 0;
   double max_norm = 0.0;
   mxopt_norm_result* out = nullptr;

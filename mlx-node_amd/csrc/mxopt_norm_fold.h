@@ -71,7 +71,8 @@ __device__ __forceinline__ void write_outcome(double sumsq, const NormFold& fold
 }
 
 // The lanes' float64 sums become the workgroup's partial sum; the workgroup that stores the last one of the call folds them
-// all, where they are at most kMaxFolded.  It saves a launch, not device time.  Global norm, microseconds a call with a second
+// all, where they are at most kMaxFolded.  The count is never reset: every call knows which arrival is its last one, so that
+// calls that should have been ordered and were not leave nothing behind for the next.  It saves a launch, not device time.  Global norm, microseconds a call with a second
 // kernel and with the fold, called from a loop: 1,000 elements (1 partial sum) 7.4 and 4.4, 60 chunks 8.0 and 6.0; replayed from a
 // graph 12 chunks 4.5 and 4.5, 60 4.6 and 4.9.  With 1,024 partial sums and their arrivals counted in two stages the
 // device takes 5.5 and 5.9, in one stage (an arrival every 12 ns at one counter) 16.
@@ -88,16 +89,13 @@ __device__ __forceinline__ void finish_partial(double acc_sum, double* __restric
     // would also write the die's whole L2 back.)
     __hip_atomic_store(partial_sum + blockIdx.x, acc_sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    last = __hip_atomic_fetch_add(fold.arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == fold.count - 1u;
+    last = __hip_atomic_fetch_add(fold.arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == fold.last_arrival;
   }
   __syncthreads();
   if (!last) return;
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   const double s = sum_of_partials<kThreads, true>(fold.partials, fold.count);
-  if (threadIdx.x == 0) {
-    write_outcome(s, fold);
-    __hip_atomic_store(fold.arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next call
-  }
+  if (threadIdx.x == 0) write_outcome(s, fold);
 }
 
 }  // namespace mxopt

@@ -177,3 +177,52 @@ def test_engine_call_that_waits_is_refused_under_capture(kind):
     del engines, captured, plain
     for ctx in ctxs:
         ctx.close()
+
+
+def _norm_is(ctx, res, want, what):
+    r = ctx.read_norm_result(res)
+    assert r.sumsq == want and r.nonfinite == 0, (what, r.sumsq, want)
+
+
+@pytest.mark.parametrize("chunks", [1, 3, 64])
+@pytest.mark.parametrize("warm", [True, False])
+def test_short_norms_eager_and_replayed_share_a_context(chunks, warm):
+    """Eager norms of up to 64 workgroups count arrivals; captured ones leave the count alone, whatever is captured, replayed,
+    dropped without a replay or refused in between, and also where the first norm of the context is a captured one (warm
+    False, a relaxed capture).  Elements are powers of two, so the sums are exact in any order."""
+    import torch
+    import mxopt as mx
+    n = (chunks - 1) * 4096 + 5
+    stream = torch.cuda.Stream()
+    ctx = mx.Context(stream=stream)
+    a, b = torch.full((n,), 2.0 ** -6, device="cuda"), torch.full((9,), 2.0 ** -3, dtype=torch.bfloat16, device="cuda")
+    table, one = ctx.table([mx.TensorSpec(g=a)]), ctx.table([mx.TensorSpec(g=b)])
+    bad = ctx.table([mx.TensorSpec(g=a), mx.TensorSpec(g=b)])     # its second group has no kernel
+    bad.set_pending([[a.clone(), torch.zeros(9, device="cuda")]])
+    eager, replayed, dropped = ctx.norm_result(), ctx.norm_result(), ctx.norm_result()
+    torch.cuda.synchronize()
+    if warm:
+        ctx.global_norm(table, eager, max_norm=1.0)
+        ctx.synchronize()
+    graph, other = torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream, capture_error_mode="relaxed"):
+        ctx.global_norm(table, replayed, max_norm=1.0)
+    with torch.cuda.graph(other, stream=stream, capture_error_mode="relaxed"):
+        ctx.global_norm(one, dropped, max_norm=1.0)
+    torch.cuda.synchronize()
+    for k in range(4):
+        ctx.global_norm(table, eager, max_norm=1.0)
+        _norm_is(ctx, eager, n * 2.0 ** -12 * 4.0 ** k, ("eager", k))
+        with torch.cuda.stream(stream):
+            graph.replay()
+        _norm_is(ctx, replayed, n * 2.0 ** -12 * 4.0 ** k, ("replayed", k))
+        with pytest.raises(mx.MxoptError):
+            ctx.norm_with_pending_list(bad, eager, max_norm=1.0)
+        ctx.global_norm(one, eager, max_norm=1.0)
+        _norm_is(ctx, eager, 9 * 2.0 ** -6, ("eager, another table", k))
+        ctx.synchronize()
+        a.mul_(2.0)
+        torch.cuda.synchronize()
+    for t in (table, one, bad):
+        t.close()
+    ctx.close()
