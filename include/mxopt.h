@@ -32,7 +32,7 @@
  * allocated its per-workgroup partials buffer, so a step may be recorded into a graph after
  * one eager warm-up call.  A recorded reduction uses that buffer, which every reduction of the context shares: replays
  * are ordered with the context's own work and with each other like calls on one stream (two reductions that overlap give
- * wrong norms; later ones are right again).  mxopt_table_build, mxopt_table_set_step_scalars, mxopt_table_retarget
+ * wrong norms; later ones are right again), and none follows the context's destruction.  mxopt_table_build, mxopt_table_set_step_scalars, mxopt_table_retarget
  * and mxopt_table_set_pending copy from host memory and stay outside a capture.
  */
 #ifndef MXOPT_H

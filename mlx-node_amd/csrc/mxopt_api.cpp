@@ -116,16 +116,14 @@ uint32_t persistent_grid(const mxopt_ctx* ctx, uint32_t nchunks) {
   return (uint32_t)std::min<uint64_t>(nchunks, std::max<uint64_t>(cap, 1));
 }
 
+// A buffer that has become too small is kept until the context's end: a recorded graph may hold its address.  Each is at
+// least twice as large as the one before, so that together they are less than twice the last.
 static int ensure_partials(mxopt_ctx* ctx, size_t need) {
   if (need <= ctx->partial_cap) return MXOPT_OK;
-  const size_t cap = std::max<size_t>(need, 4096);
+  const size_t cap = std::max<size_t>({need, 2 * ctx->partial_cap, 4096});
   double* ps = nullptr;
   HIP_TRY(ctx, hipMalloc((void**)&ps, cap * sizeof(double)));
-  // Earlier launches may still be reading the old buffer.
-  if (ctx->d_partial_sum) {
-    (void)hipStreamSynchronize(ctx->stream);
-    (void)hipFree(ctx->d_partial_sum);
-  }
+  if (ctx->d_partial_sum) ctx->old_partial_sums.push_back(ctx->d_partial_sum);
   ctx->d_partial_sum = ps;
   ctx->partial_cap = cap;
   return MXOPT_OK;
@@ -433,6 +431,7 @@ void mxopt_destroy(mxopt_ctx* ctx) {
   if (ctx->d_partial_sum || ctx->d_arrived) {
     (void)hipStreamSynchronize(ctx->stream);
     if (ctx->d_partial_sum) (void)hipFree(ctx->d_partial_sum);
+    for (double* ps : ctx->old_partial_sums) (void)hipFree(ps);
     if (ctx->d_arrived) (void)hipFree(ctx->d_arrived);
   }
   if (ctx->h_norm) (void)hipHostFree(ctx->h_norm);

@@ -105,6 +105,7 @@ struct mxopt_ctx {
   int pipelined_norm = 2;         // plain 16-bit norms: the software-pipelined kernel
   double* d_partial_sum = nullptr;            // one float64 partial per workgroup of a reduction
   size_t partial_cap = 0;
+  std::vector<double*> old_partial_sums;      // smaller ones, which recorded graphs may still write to
   uint32_t* d_arrived = nullptr;              // NormFold::arrived, an allocation of its own
   uint32_t arrivals = 0;                      // its value behind everything enqueued so far (modulo 2^32)
   bool arrivals_known = false;                // ... which only counts where this is set

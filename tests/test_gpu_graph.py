@@ -226,3 +226,44 @@ def test_short_norms_eager_and_replayed_share_a_context(chunks, warm):
     for t in (table, one, bad):
         t.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("chunks", [3, 100])
+def test_replay_of_a_norm_recorded_before_the_partial_sums_grew(chunks):
+    """A graph holds the address of the buffer that its reduction was recorded with.  A later reduction of the same context
+    that needs a larger one leaves that buffer alone: memory handed out in between keeps its values, and every replay gives
+    the norm of the gradients as they are."""
+    import torch
+    import mxopt as mx
+    n = (chunks - 1) * 4096 + 5
+    stream = torch.cuda.Stream()
+    ctx = mx.Context(stream=stream)
+    ctx.set_option("grid_blocks_per_cu", 64)
+    a = torch.full((n,), 2.0 ** -6, device="cuda")
+    table = ctx.table([mx.TensorSpec(g=a)])
+    replayed, eager = ctx.norm_result(), ctx.norm_result()
+    torch.cuda.synchronize()
+    ctx.global_norm(table, eager)
+    ctx.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        ctx.global_norm(table, replayed)
+    torch.cuda.synchronize()
+    for k, rows in enumerate((5000, 12000)):          # one workgroup per row: past 4,096, then past twice that
+        long = torch.full((rows * 4096,), 2.0 ** -9, device="cuda")
+        t = ctx.table([mx.TensorSpec(g=long)])
+        torch.cuda.synchronize()
+        ctx.global_norm(t, eager)
+        _norm_is(ctx, eager, rows * 4096 * 2.0 ** -18, ("eager", rows))
+        others = [torch.full((4096,), 3.0, dtype=torch.float64, device="cuda") for _ in range(64)]
+        torch.cuda.synchronize()
+        for j in range(3):
+            with torch.cuda.stream(stream):
+                graph.replay()
+            _norm_is(ctx, replayed, n * 2.0 ** -12 * 4.0 ** (3 * k + j), ("replayed", rows, j))
+            a.mul_(2.0)
+            torch.cuda.synchronize()
+        assert all(bool((o == 3.0).all()) for o in others)
+        t.close()
+    table.close()
+    ctx.close()
