@@ -82,7 +82,10 @@ int mxopt_synchronize(mxopt_ctx* ctx);
  * or 4 = a kernel that takes that many chunks per trip, for tables whose chunks are under 90 % full on
  * average, i.e. many small tensors; 1 = that kernel, two chunks per trip, for every table),
  * "tiles" (kernels that take 32,768 consecutive elements of a tensor per workgroup: 0 = never, 1 (default) = where a
- * launch is long enough for them to pay, 2 = wherever they can; same results). */
+ * launch is long enough for them to pay, 2 = wherever they can; same results; "persistent" = 1 or "nontemporal" = 0 switch
+ * them off whatever it says).  To be read only: "num_cus", and of the latest launch over tensors "last_launch_lanes" (of
+ * each workgroup: 1,024 by tiles, else 256), "last_launch_workgroups", "last_launch_lds" (bytes of LDS that a workgroup
+ * reserves, so that fewer of them share a compute unit; 0 = as many as fit). */
 int mxopt_set_option(mxopt_ctx* ctx, const char* name, int64_t value);
 int mxopt_get_option(const mxopt_ctx* ctx, const char* name, int64_t* value);
 

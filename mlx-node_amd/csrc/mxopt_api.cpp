@@ -187,6 +187,7 @@ Launch make_launch(const mxopt_ctx* ctx, const mxopt_table* t, const Group& g, b
   L.partial_chunks = g.elems * 10 < (uint64_t)g.nchunks * kChunkElems * 9;
   L.elems = g.elems;
   L.num_cus = (uint32_t)ctx->num_cus;
+  L.note = &ctx->last_launch;
   return L;
 }
 
@@ -380,6 +381,7 @@ Launch make_single_launch(const mxopt_ctx* ctx, const mxopt_tensor& t, bool pers
   L.partial_chunks = L.one.n * 10 < (uint64_t)L.nchunks * kChunkElems * 9;
   L.elems = L.one.n;
   L.num_cus = (uint32_t)ctx->num_cus;
+  L.note = &ctx->last_launch;
   return L;
 }
 
@@ -483,6 +485,9 @@ int mxopt_get_option(const mxopt_ctx* ctx, const char* name, int64_t* value) {
   else if (n == "persistent_accumulate") *value = ctx->persistent_accumulate;
   else if (n == "pipelined_norm") *value = ctx->pipelined_norm;
   else if (n == "num_cus") *value = ctx->num_cus;
+  else if (n == "last_launch_lanes") *value = ctx->last_launch.lanes;
+  else if (n == "last_launch_workgroups") *value = ctx->last_launch.workgroups;
+  else if (n == "last_launch_lds") *value = ctx->last_launch.lds;
   else return MXOPT_ERR_INVALID_ARG;
   return MXOPT_OK;
 }

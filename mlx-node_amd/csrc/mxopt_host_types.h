@@ -79,6 +79,12 @@ struct StreamScales {
 };
 
 // Tensors of one dtype combination: a contiguous run of chunk entries, one launch.
+// The shape of a launch, for mxopt_get_option.
+struct LaunchNote {
+  uint32_t lanes = 0, workgroups = 0;  // lanes of each workgroup
+  uint32_t lds = 0;                    // bytes of dynamic LDS
+};
+
 struct Group {
   int pd, gd, pod, god;
   uint32_t chunk_begin, nchunks;
@@ -112,6 +118,7 @@ struct mxopt_ctx {
   double* d_static_partials = nullptr;        // this device's copy of the library's fixed partial-sum array
   mxopt_norm_result* d_norm_scratch = nullptr;  // result slot of the gradient utilities
   mxopt_norm_result* h_norm = nullptr;          // pinned: the norm that a gradient utility hands back
+  mutable mxopt::LaunchNote last_launch;        // of the latest launch over tensors
   mxopt_hbm_pool* state_pool = nullptr;         // where the host layer takes moments and accumulation buffers from
   struct CachedTable {                          // tables built by the host layer, most recent last
     std::vector<mxopt_tensor> key;

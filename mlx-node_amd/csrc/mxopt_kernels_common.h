@@ -232,11 +232,16 @@ inline uint32_t crowd_lds(const Launch& L, Crowd crowd) {
   return ((163840u / (uint32_t)crowd.per_cu) / 1280u - 1u) * 1280u;
 }
 
-#define MXOPT_LAUNCH_CROWD(kernel, crowd, L, ...)                                                                        \
-  hipLaunchKernelGGL(kernel, dim3((L).grid), dim3(kThreads), crowd_lds(L, crowd), (L).stream, (L).tensors, (L).chunks, \
-                     (L).one, (L).nchunks, __VA_ARGS__)
-#define MXOPT_LAUNCH(kernel, L, ...)                                                                          \
-  hipLaunchKernelGGL(kernel, dim3((L).grid), dim3(kThreads), 0, (L).stream, (L).tensors, (L).chunks, (L).one, \
-                     (L).nchunks, __VA_ARGS__)
+// What a launch was, for mxopt_get_option; hands the LDS on.
+inline uint32_t note_launch(const Launch& L, uint32_t lanes, uint32_t workgroups, uint32_t lds) {
+  if (L.note != nullptr) *L.note = LaunchNote{lanes, workgroups, lds};
+  return lds;
+}
+
+#define MXOPT_LAUNCH_LDS(kernel, lds, L, ...)                                                                            \
+  hipLaunchKernelGGL(kernel, dim3((L).grid), dim3(kThreads), note_launch(L, kThreads, (L).grid, lds), (L).stream,      \
+                     (L).tensors, (L).chunks, (L).one, (L).nchunks, __VA_ARGS__)
+#define MXOPT_LAUNCH_CROWD(kernel, crowd, L, ...) MXOPT_LAUNCH_LDS(kernel, crowd_lds(L, crowd), L, __VA_ARGS__)
+#define MXOPT_LAUNCH(kernel, L, ...) MXOPT_LAUNCH_LDS(kernel, 0, L, __VA_ARGS__)
 
 }  // namespace mxopt

@@ -31,6 +31,7 @@ struct Launch {
   bool partial_chunks = false;       // the chunks are under 90 % full on average (many small tensors)
   uint64_t elems = 0;                // elements of the launch
   uint32_t num_cus = 1;
+  LaunchNote* note = nullptr;        // where the launch is written down
   // Deferred accumulation (the *_list launchers): stream j of table row r is pending[j * ntensors + r].
   const void* const* pending = nullptr;
   uint32_t ntensors = 0;

@@ -205,12 +205,10 @@ __global__ __launch_bounds__(kThreads) void update_list_kernel(const DevTensor* 
   }
 }
 
-#define MXOPT_LAUNCH_LIST(kernel, L, ...)                                                                     \
-  hipLaunchKernelGGL(kernel, dim3((L).grid), dim3(kThreads), 0, (L).stream, (L).tensors, (L).chunks, (L).one, \
-                     (L).nchunks, (L).ntensors, (L).pending, (L).npending, __VA_ARGS__)
-#define MXOPT_LAUNCH_UPDATE_LIST(kernel, crowd, L, ...)                                                                   \
-  hipLaunchKernelGGL(kernel, dim3((L).grid), dim3(kThreads), crowd_lds(L, crowd), (L).stream, (L).tensors, (L).chunks,  \
-                     (L).one, (L).nchunks, (L).ntensors, (L).pending, (L).npending, (L).scales, __VA_ARGS__)
+#define MXOPT_LAUNCH_LIST(kernel, L, ...) \
+  MXOPT_LAUNCH(kernel, L, (L).ntensors, (L).pending, (L).npending, __VA_ARGS__)
+#define MXOPT_LAUNCH_UPDATE_LIST(kernel, crowd, L, ...) \
+  MXOPT_LAUNCH_CROWD(kernel, crowd, L, (L).ntensors, (L).pending, (L).npending, (L).scales, __VA_ARGS__)
 
 constexpr int kFewPending = 3;  // up to four micro-batches take the instance with fewer registers
 

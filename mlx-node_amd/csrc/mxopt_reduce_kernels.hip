@@ -351,8 +351,9 @@ static void launch_accumulate(const Launch& L, const DevPrep& prep, int first) {
   if (!L.in_place) { launch_accumulate_kind<AD, GD, kElsewhere>(L, prep); return; }
   if constexpr (AD == MXOPT_F32 && GD == MXOPT_F32) {
     if (L.ntiles != 0 && L.tiles_per_cu >= 32u) {
-      hipLaunchKernelGGL(accumulate_tile_kernel, dim3(L.ntiles), dim3(kTileThreads), kOnePerCu, L.stream, L.tensors, L.chunks,
-                         L.one, L.nchunks, L.tiles, prep);
+      hipLaunchKernelGGL(accumulate_tile_kernel, dim3(L.ntiles), dim3(kTileThreads),
+                         note_launch(L, kTileThreads, L.ntiles, kOnePerCu), L.stream, L.tensors, L.chunks, L.one, L.nchunks,
+                         L.tiles, prep);
       return;
     }
   }

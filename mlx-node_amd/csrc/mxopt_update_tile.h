@@ -117,8 +117,9 @@ static bool launch_update_tiles(const Launch& L, const Math& math, const DevPrep
   constexpr int kG2Words = G2 < 0 ? 0 : Elem<(G2 < 0 ? MXOPT_F32 : G2)>::kBytes;
   constexpr int kWords = Elem<PD>::kBytes + Elem<GD>::kBytes + kG2Words + (Math::kM ? 4 : 0) + (Math::kV ? 4 : 0);
   constexpr int U = kWords <= 12 ? 8 : 4;
-  hipLaunchKernelGGL((update_tile_kernel<PD, GD, G2, Math, U>), dim3(L.ntiles), dim3(kTileThreads), kOnePerCu, L.stream,
-                     L.tensors, L.chunks, L.one, L.nchunks, L.tiles, math, prep);
+  hipLaunchKernelGGL((update_tile_kernel<PD, GD, G2, Math, U>), dim3(L.ntiles), dim3(kTileThreads),
+                     note_launch(L, kTileThreads, L.ntiles, kOnePerCu), L.stream, L.tensors, L.chunks, L.one, L.nchunks,
+                     L.tiles, math, prep);
   return true;
 }
 

@@ -171,6 +171,40 @@ def test_single_tensor(mx, ctx, n, shift):
     assert torch.equal(bits(torch, outs[0]), bits(torch, outs[1])) and not torch.equal(outs[0], base)
 
 
+def test_launches_say_which_route_they_took(mx, ctx):
+    """last_launch_*: tiles where the option asks for them and there are any, chunks where it forbids them, where parameters go
+    to another buffer and where another option overrides it."""
+    import torch
+    n = 2 * TILE + 5
+    p, g, out = (torch.zeros(n, device="cuda") for _ in range(3))
+    rows = {"in place": [mx.TensorSpec(p=p, p_out=p, g=g)], "out of place": [mx.TensorSpec(p=p, p_out=out, g=g)]}
+    sums = ctx.table([mx.TensorSpec(g_out=out, g=g)])
+
+    def lanes(option, value, call):
+        before = ctx.get_option(option)
+        ctx.set_option("tiles", 2)
+        ctx.set_option(option, value)
+        try:
+            call()
+        finally:
+            ctx.set_option(option, before)
+            ctx.set_option("tiles", 1)
+        got = [ctx.get_option("last_launch_" + k) for k in ("lanes", "workgroups", "lds")]
+        assert got[:2] in ([1024, 3], [256, 17]) and (got[2] > 0) == (got[0] == 1024), got
+        return got[0]
+
+    for where, spec in rows.items():
+        table = ctx.table(spec)
+        update = lambda: ctx.sgd_plain(table, 0.3)
+        assert lanes("tiles", 2, update) == (1024 if where == "in place" else 256)
+        assert lanes("tiles", 1, update) == 256 and lanes("tiles", 0, update) == 256
+        assert lanes("persistent", 1, update) == 256 and lanes("nontemporal", 0, update) == 256
+    add = lambda: ctx.accumulate(sums, first=False)
+    assert lanes("tiles", 2, add) == 1024 and lanes("tiles", 0, add) == 256 and lanes("nontemporal", 0, add) == 256
+    with pytest.raises(mx.MxoptError):
+        ctx.set_option("last_launch_lanes", 1)
+
+
 def test_rule_takes_tiles_for_long_lists_only(mx, ctx):
     """The default rule on both sides of its line gives the results of either route."""
     import torch
