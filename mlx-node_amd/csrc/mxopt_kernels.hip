@@ -109,9 +109,11 @@ __global__ __launch_bounds__(kThreads) void transform_kernel(const DevTensor* __
 // Microseconds with as many workgroups as the registers allow (4 or 5) and with two: bf16 AdamW, 10,000 tensors of 64 - 65,536
 // elements 405 and 367, one of 24 M 93 and 95, 48 M 185 and 181, 96 M 395 and 369; float32, the 10,000 518 and 488; float32 SGD 378 and
 // 356.  10,000 tensors of 100 - 3,000 (chunks 27 %
-// full) 52 and 86.  16-bit parameters without the first moment gain nothing (SGD, 32 M: 79 and 86).
+// full) 52 and 86.  Log-uniform lists, per mille full, 16-bit and float32 AdamW, float32 RMSprop: 620 375 and 389, 479 and 450, 328 and
+// 363; 681 386 and 381, 491 and 454, 338 and 354; 802 323 and 312, 418 and 377, 286 and 289; 876 368 and 349, 477 and 427, 324 and 318.
+// 16-bit parameters without the first moment gain nothing (SGD, 32 M: 79 and 86).
 template <int PD, int GD, class Math>
-constexpr Crowd kUpdateCrowd = Math::kM || (Math::kV && PD == MXOPT_F32 && GD == MXOPT_F32) ? Crowd{2, 75, 32} : kNoLimit;
+constexpr Crowd kUpdateCrowd = Math::kM || (Math::kV && PD == MXOPT_F32 && GD == MXOPT_F32) ? Crowd{2, 750, 32} : kNoLimit;
 
 template <int PD, int GD, int OD, int G2, class Math>
 static void launch_update_t(const Launch& L, const Math& math, const DevPrep& prep) {
@@ -252,10 +254,14 @@ bool launch_sgd_plain(int pd, int gd, int od, const Launch& L, float lr_p, float
 // 68, 256 M 277 and 247, 1.72 G 1,852 and 1,596 (10,000 tensors whose chunks are 82 % full 107 and 122); 16-bit into 16-bit 64 M 49
 // and 47, 256 M 182 and 168, 596 M 419 and 374; float32 64 M 93 and 89, 256 M 360 and 351.  Added into a float32 buffer 256 M 435
 // and 426, 596 M 1,005 and 954; into a 16-bit one 128 M 131 and 128, 596 M 589 and 553.
+// Where the lists' last chunks begin to spoil it (log-uniform lists; per mille full): 16-bit into 16-bit 933 184 and 194, 974 209 and
+// 223, 996 317 and 323, the 0.6B list (999) 414 and 371; into float32 933 131 and 137, 961 166 and 168, 984 205 and 203, 996 260 and
+// 250; float32 877 141 and 142, 933 178 and 169; added, 16-bit 933 250 and 263, 952 307 and 312, 974 303 and 298, into float32 933 455
+// and 438.
 template <int GD, int OD, bool ADD>
 constexpr Crowd kTransformCrowd =
-    ADD ? (OD == MXOPT_F32 ? (GD == MXOPT_F32 ? kNoLimit : Crowd{2, 90, 256}) : Crowd{4, 90, 128})
-        : (OD != MXOPT_F32 ? Crowd{6, 90, 16} : GD != MXOPT_F32 ? Crowd{4, 90, 16} : Crowd{3, 90, 32});
+    ADD ? (OD == MXOPT_F32 ? (GD == MXOPT_F32 ? kNoLimit : Crowd{2, 900, 256}) : Crowd{4, 970, 128})
+        : (OD != MXOPT_F32 ? Crowd{6, 998, 16} : GD != MXOPT_F32 ? Crowd{4, 970, 16} : Crowd{3, 900, 32});
 
 template <int GD, int OD>
 static void launch_transform_t(const Launch& L, const DevPrep& prep, int add) {

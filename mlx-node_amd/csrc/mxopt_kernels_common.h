@@ -218,7 +218,7 @@ __device__ __forceinline__ float norm_value(const PrepRegs& pr, float x, bool cl
 // reading to writing less often.  Too few leave it waiting; each launcher says what it measured.
 struct Crowd {
   int per_cu;         // workgroups (of kThreads) per compute unit
-  int fill;           // only where the chunks are at least this full on average, in per cent (short chunks need company), and
+  int fill;           // only where the chunks are at least this full on average, per mille (short chunks need company), and
   int chunks_per_cu;  // only where the launch has at least this many for each compute unit
 };
 constexpr Crowd kNoLimit{0, 0, 0};
@@ -227,7 +227,7 @@ constexpr Crowd kNoLimit{0, 0, 0};
 // (1,280 bytes), one unit less for what a kernel declares itself.
 inline uint32_t crowd_lds(const Launch& L, Crowd crowd) {
   if (crowd.per_cu == 0 || (uint64_t)L.nchunks < (uint64_t)crowd.chunks_per_cu * L.num_cus ||
-      L.elems * 100u < (uint64_t)L.nchunks * kChunk * (uint32_t)crowd.fill)
+      L.elems * 1000u < (uint64_t)L.nchunks * kChunk * (uint32_t)crowd.fill)
     return 0;
   return ((163840u / (uint32_t)crowd.per_cu) / 1280u - 1u) * 1280u;
 }

@@ -212,10 +212,11 @@ __global__ __launch_bounds__(kThreads) void update_list_kernel(const DevTensor* 
 
 constexpr int kFewPending = 3;  // up to four micro-batches take the instance with fewer registers
 
-// Plain SGD over four bf16 micro-batches of 596 M elements: 1,203 us without a limit, 1,137 with it.  AdamW gains 3 % in memory of one
+// Plain SGD over four bf16 micro-batches of 596 M elements: 1,203 us without a limit, 1,137 with it; log-uniform lists 933 per mille
+// full 504 and 544, 952 614 and 649, 974 609 and 595, 984 774 and 725.  AdamW gains 3 % in memory of one
 // region and loses as much in memory of two.
 template <int PD, int GD, int XD, class Math>
-constexpr Crowd kListCrowd = XD == MXOPT_F32 || GD == MXOPT_F32 || PD == MXOPT_F32 || Math::kV ? kNoLimit : Crowd{5, 90, 64};
+constexpr Crowd kListCrowd = XD == MXOPT_F32 || GD == MXOPT_F32 || PD == MXOPT_F32 || Math::kV ? kNoLimit : Crowd{5, 970, 64};
 
 template <int PD, int GD, int XD, class Math>
 static void launch_update_list_t(const Launch& L, const Math& math, const DevPrep& prep) {

@@ -331,18 +331,29 @@ __global__ __launch_bounds__(kTileThreads) void accumulate_tile_kernel(const Dev
 // 1,908 and 1,598; into 16 bits 128 M 92 and 87, 596 M 421 and 372 (32 M 27 and 28; 10,000 tensors of 64 - 65,536 74 and 80);
 // float32 128 M 189 and 172, 256 M 379 and 335.  Later passes: into float32, the 10,000 tensors, of 16 bits 150 and 140, of 32 191 and
 // 172; of 16 bits in groups of 8 (two a unit) 128 M 236 and 208; into 16 bits 256 M 263 and 254, 596 M 598 and 573 (the 10,000 tensors
-// 85 and 91).
+// 85 and 91).  First pass of float32 over log-uniform lists, per mille full: 802 124 and 144, 877 143 and 150, 933 184 and 181, 952 252
+// and 242.
 template <int AD, int GD, int KIND>
 constexpr Crowd kAccumulateCrowd = KIND == kElsewhere ? kNoLimit
-                                   : KIND == kInPlaceWide ? Crowd{2, 90, 128}
-                                   : AD != MXOPT_F32 ? (KIND == kFirstPass ? Crowd{5, 90, 128} : Crowd{4, 90, 128})
-                                   : KIND == kInPlace ? Crowd{4, 75, 16}
-                                   : GD != MXOPT_F32 ? Crowd{5, 75, 16} : Crowd{2, 75, 16};
+                                   : KIND == kInPlaceWide ? Crowd{2, 900, 128}
+                                   : AD != MXOPT_F32 ? (KIND == kFirstPass ? Crowd{5, 900, 128} : Crowd{4, 900, 128})
+                                   : KIND == kInPlace ? Crowd{4, 600, 16}
+                                   : GD != MXOPT_F32 ? Crowd{5, 750, 16} : Crowd{2, 920, 16};
+// Later passes into float32 over shorter chunks.  Log-uniform lists, per mille full, without a limit, with 4 and with 6 (float32: 7) a
+// unit: of 16 bits 285 132, 186 and 146, 438 158, 162 and 151, 620 172, 156 and 164, 681 174, 155 and 168, 802 141, 127 and 138; of
+// float32 285 163, 191 and 157, 438 189, 179 and 183, 620 200, 181 and 200, 681 205, 185 and 204.
+template <int GD>
+constexpr Crowd kShortChunksCrowd = GD != MXOPT_F32 ? Crowd{6, 400, 16} : Crowd{7, 0, 16};
 
 template <int AD, int GD, int KIND>
 static void launch_accumulate_kind(const Launch& L, const DevPrep& prep) {
-  if (L.nontemporal) MXOPT_LAUNCH_CROWD((accumulate_kernel<AD, GD, true, KIND>), (kAccumulateCrowd<AD, GD, KIND>), L, prep);
-  else MXOPT_LAUNCH((accumulate_kernel<AD, GD, false, KIND>), L, prep);
+  if (!L.nontemporal) {
+    MXOPT_LAUNCH((accumulate_kernel<AD, GD, false, KIND>), L, prep);
+    return;
+  }
+  uint32_t lds = crowd_lds(L, kAccumulateCrowd<AD, GD, KIND>);
+  if (lds == 0 && AD == MXOPT_F32 && KIND == kInPlace) lds = crowd_lds(L, kShortChunksCrowd<GD>);
+  MXOPT_LAUNCH_LDS((accumulate_kernel<AD, GD, true, KIND>), lds, L, prep);
 }
 
 template <int AD, int GD>
@@ -496,9 +507,9 @@ static void launch_sumsq_t(const Launch& L, const DevPrep& prep, int first, doub
     if (ps == nullptr) { launch_accumulate<AD, GD>(L, prep, first); return; }
   }
   // The norm of a sum that is not stored, microseconds without a limit and with it: float32 and a 16-bit gradient 96 M elements 99
-  // and 97, 256 M 253 and 239, 1.72 G 1,604 and 1,464 (64 M 68 and 69); 16-bit both 256 M 174 and 167, 596 M 377 and 361.  One
-  // stream and two float32 ones gain nothing.
-  constexpr Crowd kCrowd = MODE != 3 || GD == MXOPT_F32 ? kNoLimit : AD == MXOPT_F32 ? Crowd{2, 90, 96} : Crowd{4, 90, 256};
+  // and 97, 256 M 253 and 239, 1.72 G 1,604 and 1,464 (64 M 68 and 69); 16-bit both 256 M 174 and 167, 596 M 377 and 361 (log-uniform
+  // lists 952 per mille full 204 and 208, 974 192 and 192, 984 236 and 234).  One stream and two float32 ones gain nothing.
+  constexpr Crowd kCrowd = MODE != 3 || GD == MXOPT_F32 ? kNoLimit : AD == MXOPT_F32 ? Crowd{2, 900, 96} : Crowd{4, 970, 256};
   if (L.nontemporal) MXOPT_LAUNCH_CROWD((sumsq_kernel<MODE, AD, GD, true>), kCrowd, L, prep, first, ps, fold);
   else MXOPT_LAUNCH((sumsq_kernel<MODE, AD, GD, false>), L, prep, first, ps, fold);
 }

@@ -281,3 +281,62 @@ def test_accumulation(mx, ctx, ad, gd, layout):
             ctx.set_option("tiles", 1)
     for p, q, o in zip(views(other[0], layout, 0), views(other[1], layout, 0), vo):
         assert torch.equal(bits(torch, p.clone()), bits(torch, q.clone())) and torch.equal(bits(torch, p.clone()), bits(torch, o.clone()))
+
+
+def reserved(per_cu):
+    """Bytes of LDS a workgroup reserves so that this many share a compute unit (0: as many as fit)."""
+    return 0 if per_cu is None else (163840 // per_cu // 1280 - 1) * 1280
+
+
+# gradient, output / accumulator, workgroups per compute unit below and above the line, the line in per mille of a full chunk
+LINES = {
+    "transform": [("bfloat16", "bfloat16", None, 6, 998), ("bfloat16", "float32", None, 4, 970)],
+    "first": [("bfloat16", "float32", None, 5, 750), ("float32", "float32", None, 2, 920)],
+    "later": [("float16", "float32", 6, 4, 600), ("float16", "float32", None, 6, 400), ("float32", "float32", 7, 4, 600)],
+}
+
+
+@pytest.mark.parametrize("kind,gd,od,below,above,line",
+                         [(k,) + row for k, rows in LINES.items() for row in rows])
+@pytest.mark.parametrize("side", [-1, 1])
+def test_fewer_workgroups_share_a_unit_where_chunks_are_full_enough(mx, ctx, kind, gd, od, below, above, line, side):
+    """Lists of 16 chunks per compute unit, just emptier and just fuller than a rule's line: the launch says which side it
+    is on, and the results are torch's on both."""
+    import torch
+    chunks = 8 if line > 900 else 3 if line > 700 else 2 if line > 500 else 1
+    count = -(-16 * ctx.get_option("num_cus") // chunks)
+    n = chunks * 4096 * line // 1000 + side * 8                       # elements of each tensor, in `chunks` chunks
+    assert (n + 4095) // 4096 == chunks
+    step = -(-n // 64) * 64
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(9)
+    g = torch.empty(count * step, device="cuda").normal_(0.0, 1e-2, generator=gen).to(getattr(torch, gd))
+    out = torch.empty(count * step, device="cuda").normal_(0.0, 1e-2, generator=gen).to(getattr(torch, od))
+    before = out.clone()
+    table = ctx.table([mx.TensorSpec(g=g[i * step:i * step + n], g_out=out[i * step:i * step + n]) for i in range(count)])
+    if kind == "transform":
+        ctx.grad_transform(table, mx.make_prep(pre_mul=0.5))
+        want = (g.float() * 0.5).to(out.dtype)
+    else:
+        ctx.accumulate(table, first=kind == "first")
+        want = g.to(out.dtype) if kind == "first" else (before.float() + g.float()).to(out.dtype)
+    assert ctx.get_option("last_launch_lds") == reserved(above if side > 0 else below)
+    inside = torch.zeros(count * step, dtype=torch.bool, device="cuda")
+    inside.view(count, step)[:, :n] = True
+    assert torch.equal(bits(torch, out), bits(torch, torch.where(inside, want, before)))
+
+
+@pytest.mark.parametrize("gd", ["bfloat16", "float16"])
+@pytest.mark.parametrize("extra,per_cu", [(-1, 4), (3, 2)])
+def test_accumulation_of_16_bit_gradients_into_a_long_float32_buffer(mx, ctx, gd, extra, per_cu):
+    """On both sides of 128 chunks per compute unit, where the pass goes over to groups of 8 and two workgroups a unit; the
+    buffers start one element behind a 16-byte boundary and end in the middle of a group."""
+    import torch
+    n = 128 * ctx.get_option("num_cus") * 4096 - 4096 * (extra < 0) + extra
+    g = torch.empty(n + 8, device="cuda").normal_(0.0, 1e-2).to(getattr(torch, gd))
+    acc = torch.empty(n + 4, device="cuda").normal_(0.0, 1e-2)
+    want = acc.clone()
+    want[1:1 + n] += g[1:1 + n].float()
+    ctx.accumulate(ctx.table([mx.TensorSpec(g=g[1:1 + n], g_out=acc[1:1 + n])]), first=False)
+    assert ctx.get_option("last_launch_lds") == reserved(per_cu)
+    assert torch.equal(bits(torch, acc), bits(torch, want))
