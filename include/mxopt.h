@@ -85,7 +85,8 @@ int mxopt_synchronize(mxopt_ctx* ctx);
  * launch is long enough for them to pay, 2 = wherever they can; same results; "persistent" = 1 or "nontemporal" = 0 switch
  * them off whatever it says).  To be read only: "num_cus", and of the latest launch over tensors "last_launch_lanes" (of
  * each workgroup: 1,024 by tiles, else 256), "last_launch_workgroups", "last_launch_lds" (bytes of LDS that a workgroup
- * reserves, so that fewer of them share a compute unit; 0 = as many as fit). */
+ * reserves, so that fewer of them share a compute unit; 0 = as many as fit), "last_launch_streams_parameters"
+ * (an update: the stores of the parameters carry the streaming hint). */
 int mxopt_set_option(mxopt_ctx* ctx, const char* name, int64_t value);
 int mxopt_get_option(const mxopt_ctx* ctx, const char* name, int64_t* value);
 

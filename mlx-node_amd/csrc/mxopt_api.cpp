@@ -186,6 +186,7 @@ Launch make_launch(const mxopt_ctx* ctx, const mxopt_table* t, const Group& g, b
   L.pipelined_norm = ctx->pipelined_norm;
   L.partial_chunks = g.elems * 10 < (uint64_t)g.nchunks * kChunkElems * 9;
   L.elems = g.elems;
+  L.spread = t->spread;
   L.num_cus = (uint32_t)ctx->num_cus;
   L.note = &ctx->last_launch;
   return L;
@@ -195,9 +196,11 @@ Launch make_launch(const mxopt_ctx* ctx, const mxopt_table* t, const Group& g, b
 // elements lie in whole ones: a mixed tile occupies a compute unit for a few short chunks.  Microseconds by tiles and by chunks (two
 // workgroups per compute unit): 10,000 tensors of 64 - 65,536 elements, 35 % of them in whole tiles, bf16 AdamW 391 and 367,
 // float32 511 and 488, SGD 366 and 356; 2,000 of 1,000 - 200,000, 69 %, float32 AdamW 375 and 391, SGD 272 and 292.
+// Not in memory of several regions, where the chunks are ahead: float32 AdamW of 596 M 2,647 and 2,584, SGD 1,892 and 1,858, bf16
+// AdamW of 1.72 G 5,985 and 5,941, plain SGD 1,682 and 1,642.
 static void offer_tiles(const mxopt_ctx* ctx, Launch& L, const DevTile* tiles, uint32_t ntiles, uint32_t whole, uint64_t elems) {
   if (ctx->tiles == 0 || ctx->persistent || !ctx->nontemporal || ntiles == 0) return;
-  if (ctx->tiles == 1 && (uint64_t)whole * kTileElems * 3u < elems * 2u) return;
+  if (ctx->tiles == 1 && (L.spread || (uint64_t)whole * kTileElems * 3u < elems * 2u)) return;
   L.tiles = tiles;
   L.ntiles = ntiles;
   L.tiles_per_cu = ctx->tiles == 1 ? whole / (uint32_t)ctx->num_cus : 0xffffffffu;
@@ -352,6 +355,7 @@ void fill_dev_tensor(const mxopt_tensor& s, DevTensor& d) {
 }
 
 static void note_places(mxopt_table* t) {
+  t->spread = in_spread_memory(t->host.data(), t->host.size());
   t->in_place = t->sums_in_place = true;
   for (const mxopt_tensor& r : t->host) {
     if (r.n == 0) continue;
@@ -370,6 +374,7 @@ uint64_t chunks_of(const DevTensor& d) {
 Launch make_single_launch(const mxopt_ctx* ctx, const mxopt_tensor& t, bool persistent) {
   Launch L;
   fill_dev_tensor(t, L.one);
+  L.spread = in_spread_memory(&t, 1);
   L.nchunks = (uint32_t)chunks_of(L.one);
   L.grid = persistent ? persistent_grid(ctx, L.nchunks) : L.nchunks;
   L.stream = ctx->stream;
@@ -488,6 +493,7 @@ int mxopt_get_option(const mxopt_ctx* ctx, const char* name, int64_t* value) {
   else if (n == "last_launch_lanes") *value = ctx->last_launch.lanes;
   else if (n == "last_launch_workgroups") *value = ctx->last_launch.workgroups;
   else if (n == "last_launch_lds") *value = ctx->last_launch.lds;
+  else if (n == "last_launch_streams_parameters") *value = ctx->last_launch.streams_parameters;
   else return MXOPT_ERR_INVALID_ARG;
   return MXOPT_OK;
 }

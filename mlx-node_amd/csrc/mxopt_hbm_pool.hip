@@ -282,6 +282,23 @@ mxopt_hbm_pool* pool_of(const void* ptr) {
 
 }  // namespace
 
+bool mxopt::in_spread_memory(const mxopt_tensor* rows, size_t n) {
+  std::lock_guard<std::mutex> all(g_pools_mu);
+  if (g_pools.empty()) return false;
+  auto alternates = [](const void* ptr) {
+    for (const mxopt_hbm_pool* p : g_pools)
+      if (ptr && (const char*)ptr >= p->base && (const char*)ptr < p->base + p->one_region_begin) return true;
+    return false;
+  };
+  uint64_t spread = 0, total = 0;
+  for (size_t i = 0; i < n; ++i) {
+    const mxopt_tensor& r = rows[i];
+    total += r.n;
+    if (alternates(r.p_out) || alternates(r.m) || alternates(r.v) || alternates(r.g_out)) spread += r.n;
+  }
+  return spread * 2 > total;
+}
+
 extern "C" {
 
 int mxopt_probe_stream(mxopt_ctx* ctx, int kind, void* a, void* b, void* c, void* d, uint64_t n_elems) {

@@ -83,6 +83,7 @@ struct StreamScales {
 struct LaunchNote {
   uint32_t lanes = 0, workgroups = 0;  // lanes of each workgroup
   uint32_t lds = 0;                    // bytes of dynamic LDS
+  uint32_t streams_parameters = 0;     // updates: the parameters' stores stream
 };
 
 struct Group {
@@ -137,6 +138,7 @@ struct mxopt_table {
   mxopt::DevChunk* d_chunks = nullptr;
   mxopt::DevTile* d_tiles = nullptr;          // behind the chunks, in their allocation
   bool in_place = false;                      // p_out == p in every tensor
+  bool spread = false;                        // in_spread_memory of the rows
   bool sums_in_place = false;                 // p is NULL or g_out in every tensor: accumulation reads what it writes
   uint64_t total_elems = 0;
   uint64_t num_chunks = 0;

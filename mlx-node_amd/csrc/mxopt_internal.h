@@ -68,6 +68,9 @@ int accumulate_norm_only(mxopt_ctx* ctx, const mxopt_table* t, const mxopt_grad_
 int norm_with_pending_list(mxopt_ctx* ctx, const mxopt_table* t, const mxopt_grad_prep* prep, double max_norm, int clip_mode,
                            mxopt_norm_result* d_result, mxopt_norm_result* host_out);
 void fill_dev_tensor(const mxopt_tensor& s, DevTensor& d);
+// Whether most of what kernels write for these rows lies in an arena that alternates between memory regions (a matter of
+// speed alone: results are the same wherever buffers lie).
+bool in_spread_memory(const mxopt_tensor* rows, size_t n);
 uint64_t chunks_of(const DevTensor& d);  // chunk-table entries (= workgroups of work) of one tensor
 // A launch over the single tensor `t` (descriptor passed in the kernel arguments).
 Launch make_single_launch(const mxopt_ctx* ctx, const mxopt_tensor& t, bool persistent);

@@ -111,9 +111,31 @@ __global__ __launch_bounds__(kThreads) void transform_kernel(const DevTensor* __
 // 356.  10,000 tensors of 100 - 3,000 (chunks 27 %
 // full) 52 and 86.  Log-uniform lists, per mille full, 16-bit and float32 AdamW, float32 RMSprop: 620 375 and 389, 479 and 450, 328 and
 // 363; 681 386 and 381, 491 and 454, 338 and 354; 802 323 and 312, 418 and 377, 286 and 289; 876 368 and 349, 477 and 427, 324 and 318.
+// In memory of several regions: 78 M at 802 per mille (93 chunks a unit) bf16 AdamW 280 and 315, RMSprop 253 and 288, the 10,000
+// 339 and 356, 306 and 329; 267 M at 933 (273 a unit) 965 and 936, 885 and 857; float32 AdamW and SGD, the 10,000 428 and 417, 309 and
+// 299; a micro-batch folded in 96 M 432 and 420.
 // 16-bit parameters without the first moment gain nothing (SGD, 32 M: 79 and 86).
-template <int PD, int GD, class Math>
-constexpr Crowd kUpdateCrowd = Math::kM || (Math::kV && PD == MXOPT_F32 && GD == MXOPT_F32) ? Crowd{2, 750, 32} : kNoLimit;
+template <int PD, int GD, int G2, class Math>
+constexpr Crowd update_crowd() {
+  constexpr bool kF32 = PD == MXOPT_F32 && GD == MXOPT_F32;
+  if (!Math::kM && !(Math::kV && kF32)) return kNoLimit;
+  return Crowd{2, 750, 32, 750, Math::kSquare && !(Math::kM && kF32) && G2 < 0 ? 200 : 32};
+}
+template <int PD, int GD, int G2, class Math>
+constexpr Crowd kUpdateCrowd = update_crowd<PD, GD, G2, Math>();
+
+// Whether the stores of parameters that are updated in place stream.  In memory of several regions they do not as long as
+// the parameters stay in the 256 MB memory-side cache for whoever reads them next.  Microseconds plain and streaming, the
+// same list again and again: bf16 AdamW 48 M 166 and 175, 90 M 307 and 333, 128 M 440 and 476, 160 M 602 and 598; SGD 90 M 191 and
+// 211; float32 AdamW 48 M 205 and 221, 72 M 321 and 331, 80 M 375 and 366, RMSprop 72 M 222 and 234; several lists in turn: bf16 AdamW
+// 96 M 365 and 357, float32 64 M 315 and 314.  Plain SGD and a folded-in micro-batch gain nothing (64 M 65 and 66, 96 M 105 and
+// 99; 48 M 216 and 217).
+template <int PD, int G2, class Math>
+static bool stream_parameters(const Launch& L) {
+  if (!L.in_place) return false;
+  if (!Math::kV || G2 >= 0 || !L.spread) return true;
+  return L.elems * Elem<PD>::kBytes >= (300ull << 20);
+}
 
 template <int PD, int GD, int OD, int G2, class Math>
 static void launch_update_t(const Launch& L, const Math& math, const DevPrep& prep) {
@@ -123,12 +145,13 @@ static void launch_update_t(const Launch& L, const Math& math, const DevPrep& pr
   }
   if constexpr (OD == PD) {
     if (launch_update_tiles<PD, GD, G2>(L, math, prep)) return;
-    if (L.in_place) {
-      MXOPT_LAUNCH_CROWD((update_kernel<PD, GD, OD, G2, Math, true, true>), (kUpdateCrowd<PD, GD, Math>), L, math, prep);
+    if (stream_parameters<PD, G2, Math>(L)) {
+      MXOPT_LAUNCH_CROWD((update_kernel<PD, GD, OD, G2, Math, true, true>), (kUpdateCrowd<PD, GD, G2, Math>), L, math, prep);
+      if (L.note != nullptr) L.note->streams_parameters = 1;
       return;
     }
   }
-  MXOPT_LAUNCH_CROWD((update_kernel<PD, GD, OD, G2, Math, true, false>), (kUpdateCrowd<PD, GD, Math>), L, math, prep);
+  MXOPT_LAUNCH_CROWD((update_kernel<PD, GD, OD, G2, Math, true, false>), (kUpdateCrowd<PD, GD, G2, Math>), L, math, prep);
 }
 
 template <int PD, int GD, class Math>
@@ -257,11 +280,12 @@ bool launch_sgd_plain(int pd, int gd, int od, const Launch& L, float lr_p, float
 // Where the lists' last chunks begin to spoil it (log-uniform lists; per mille full): 16-bit into 16-bit 933 184 and 194, 974 209 and
 // 223, 996 317 and 323, the 0.6B list (999) 414 and 371; into float32 933 131 and 137, 961 166 and 168, 984 205 and 203, 996 260 and
 // 250; float32 877 141 and 142, 933 178 and 169; added, 16-bit 933 250 and 263, 952 307 and 312, 974 303 and 298, into float32 933 455
-// and 438.
+// and 438.  In memory of several regions: 16-bit into float32 974 156 and 164, 984 190 and 198, 996 242 and 241, 998 208 and 205; float32
+// 933 160 and 165, 952 223 and 223, 974 209 and 206; 16-bit added into float32 256 M 419 and 424, 596 M 935 and 947.
 template <int GD, int OD, bool ADD>
 constexpr Crowd kTransformCrowd =
-    ADD ? (OD == MXOPT_F32 ? (GD == MXOPT_F32 ? kNoLimit : Crowd{2, 900, 256}) : Crowd{4, 970, 128})
-        : (OD != MXOPT_F32 ? Crowd{6, 998, 16} : GD != MXOPT_F32 ? Crowd{4, 970, 16} : Crowd{3, 900, 32});
+    ADD ? (OD == MXOPT_F32 ? (GD == MXOPT_F32 ? kNoLimit : Crowd{2, 900, 256, kNever, 0}) : Crowd{4, 970, 128})
+        : (OD != MXOPT_F32 ? Crowd{6, 998, 16} : GD != MXOPT_F32 ? Crowd{4, 970, 16, 995, 16} : Crowd{3, 900, 32, 950, 32});
 
 template <int GD, int OD>
 static void launch_transform_t(const Launch& L, const DevPrep& prep, int add) {

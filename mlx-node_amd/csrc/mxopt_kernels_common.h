@@ -220,21 +220,27 @@ struct Crowd {
   int per_cu;         // workgroups (of kThreads) per compute unit
   int fill;           // only where the chunks are at least this full on average, per mille (short chunks need company), and
   int chunks_per_cu;  // only where the launch has at least this many for each compute unit
+  // The same in memory that alternates between regions, where there is less to gain.
+  int spread_fill, spread_chunks_per_cu;
+  constexpr Crowd(int n, int f, int c, int sf, int sc) : per_cu(n), fill(f), chunks_per_cu(c), spread_fill(sf), spread_chunks_per_cu(sc) {}
+  constexpr Crowd(int n, int f, int c) : Crowd(n, f, c, f, c) {}
 };
 constexpr Crowd kNoLimit{0, 0, 0};
+constexpr int kNever = 1001;  // per mille
 
 // Dynamic LDS that leaves room for crowd.per_cu workgroups: an equal part of a compute unit's 160 KB in units of its allocation
 // (1,280 bytes), one unit less for what a kernel declares itself.
 inline uint32_t crowd_lds(const Launch& L, Crowd crowd) {
-  if (crowd.per_cu == 0 || (uint64_t)L.nchunks < (uint64_t)crowd.chunks_per_cu * L.num_cus ||
-      L.elems * 1000u < (uint64_t)L.nchunks * kChunk * (uint32_t)crowd.fill)
+  const int fill = L.spread ? crowd.spread_fill : crowd.fill, chunks = L.spread ? crowd.spread_chunks_per_cu : crowd.chunks_per_cu;
+  if (crowd.per_cu == 0 || (uint64_t)L.nchunks < (uint64_t)chunks * L.num_cus ||
+      L.elems * 1000u < (uint64_t)L.nchunks * kChunk * (uint32_t)fill)
     return 0;
   return ((163840u / (uint32_t)crowd.per_cu) / 1280u - 1u) * 1280u;
 }
 
 // What a launch was, for mxopt_get_option; hands the LDS on.
 inline uint32_t note_launch(const Launch& L, uint32_t lanes, uint32_t workgroups, uint32_t lds) {
-  if (L.note != nullptr) *L.note = LaunchNote{lanes, workgroups, lds};
+  if (L.note != nullptr) *L.note = LaunchNote{lanes, workgroups, lds, 0u};
   return lds;
 }
 

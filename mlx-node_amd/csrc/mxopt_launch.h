@@ -25,6 +25,7 @@ struct Launch {
   uint32_t ntiles = 0;
   uint32_t tiles_per_cu = 0;
   bool in_place = false;             // what is written has been read: p_out == p (updates), the sum's own buffer (accumulation)
+  bool spread = false;               // most of what is written lies in memory that alternates between regions
   hipStream_t stream = nullptr;
   int nontemporal = 1;               // non-zero: streaming-hint loads and stores
   int pipelined_norm = 2;            // plain 16-bit norms take the software-pipelined kernel

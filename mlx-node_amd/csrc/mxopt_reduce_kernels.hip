@@ -332,13 +332,14 @@ __global__ __launch_bounds__(kTileThreads) void accumulate_tile_kernel(const Dev
 // float32 128 M 189 and 172, 256 M 379 and 335.  Later passes: into float32, the 10,000 tensors, of 16 bits 150 and 140, of 32 191 and
 // 172; of 16 bits in groups of 8 (two a unit) 128 M 236 and 208; into 16 bits 256 M 263 and 254, 596 M 598 and 573 (the 10,000 tensors
 // 85 and 91).  First pass of float32 over log-uniform lists, per mille full: 802 124 and 144, 877 143 and 150, 933 184 and 181, 952 252
-// and 242.
+// and 242; in memory of several regions 802 107 and 138, 933 161 and 175, 974 212 and 219, 998 273 and 279, 256 M full 343 and 333, 596 M
+// 753 and 756.
 template <int AD, int GD, int KIND>
 constexpr Crowd kAccumulateCrowd = KIND == kElsewhere ? kNoLimit
                                    : KIND == kInPlaceWide ? Crowd{2, 900, 128}
-                                   : AD != MXOPT_F32 ? (KIND == kFirstPass ? Crowd{5, 900, 128} : Crowd{4, 900, 128})
+                                   : AD != MXOPT_F32 ? (KIND == kFirstPass ? Crowd{5, 900, 128, 970, 128} : Crowd{4, 900, 128})
                                    : KIND == kInPlace ? Crowd{4, 600, 16}
-                                   : GD != MXOPT_F32 ? Crowd{5, 750, 16} : Crowd{2, 920, 16};
+                                   : GD != MXOPT_F32 ? Crowd{5, 750, 16} : Crowd{2, 920, 16, kNever, 0};
 // Later passes into float32 over shorter chunks.  Log-uniform lists, per mille full, without a limit, with 4 and with 6 (float32: 7) a
 // unit: of 16 bits 285 132, 186 and 146, 438 158, 162 and 151, 620 172, 156 and 164, 681 174, 155 and 168, 802 141, 127 and 138; of
 // float32 285 163, 191 and 157, 438 189, 179 and 183, 620 200, 181 and 200, 681 205, 185 and 204.

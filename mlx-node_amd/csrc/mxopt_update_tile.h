@@ -120,6 +120,7 @@ static bool launch_update_tiles(const Launch& L, const Math& math, const DevPrep
   hipLaunchKernelGGL((update_tile_kernel<PD, GD, G2, Math, U>), dim3(L.ntiles), dim3(kTileThreads),
                      note_launch(L, kTileThreads, L.ntiles, kOnePerCu), L.stream, L.tensors, L.chunks, L.one, L.nchunks,
                      L.tiles, math, prep);
+  if (L.note != nullptr) L.note->streams_parameters = 1;
   return true;
 }
 

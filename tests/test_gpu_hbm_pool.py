@@ -134,6 +134,65 @@ def test_results_do_not_depend_on_the_arena(mx, ctx, pool):
     assert pool.info().used_bytes == 0        # torch handed its segments back through the free hook
 
 
+def test_rules_for_memory_of_several_regions(mx, ctx, pool):
+    """The same updates on buffers that alternate between regions and on plain ones: limits on workgroups, tiles and streaming
+    stores follow the place (also where a table is retargeted to the other place), results do not."""
+    import torch
+    if pool.info().interleaved_bytes == 0:
+        pytest.skip("the free memory lies in one region")
+    cus = ctx.get_option("num_cus")
+    n = 32768 * 24 * cus + 5                                  # float32: tiles begin here, in memory of one region
+    mem = pool.torch_pool()
+
+    def made(inside, dtype, count, std):
+        if inside:
+            with torch.cuda.use_mem_pool(mem):
+                x = torch.empty(count, dtype=dtype, device="cuda")
+            assert pool.owns(x.data_ptr())
+        else:
+            x = torch.empty(count, dtype=dtype, device="cuda")
+        gen = torch.Generator(device="cuda")
+        gen.manual_seed(int(std * 1e6))
+        return x.normal_(0.0, std, generator=gen)
+
+    def took():
+        return tuple(ctx.get_option("last_launch_" + k) for k in ("lanes", "lds", "streams_parameters"))
+
+    two = (163840 // 2 // 1280 - 1) * 1280
+    places = {}
+    for inside in (True, False):
+        p, g, v = (made(inside, torch.float32, n, s) for s in (0.5, 1e-3, 1e-4))
+        table = ctx.table([mx.TensorSpec(p=p, p_out=p, g=g, v=v)])
+        ctx.sgd(table, mx.sgd_hp(0.1, 0.9, 0.01))
+        shape = took()
+        small = 64 * 4096 * cus                                # 64 chunks per compute unit
+        q, h, m, w = made(inside, torch.bfloat16, small, 0.5), made(inside, torch.bfloat16, small, 1e-3), *(
+            made(inside, torch.float32, small, s).square_() for s in (2e-3, 3e-3))
+        other = ctx.table([mx.TensorSpec(p=q, p_out=q, g=h, m=m, v=w)])
+        ctx.adam(other, mx.adam_hp(1e-2, 0.9, 0.999, 1e-8, 0.01))
+        shape += took()
+        places[inside] = (p, v, q, m, w, shape, other, h)
+    (inside, plain) = places[True], places[False]
+    assert plain[5][:3] == (1024, plain[5][1], 1) and inside[5][:3] == (256, two, 1)
+    assert plain[5][3:] == (256, two, 1) and inside[5][3:] == (256, 0, 0)
+    for a, b in zip(inside[:5], plain[:5]):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    # a table follows its buffers, and one tensor's call follows its own
+    table = plain[6]
+    table.retarget([mx.TensorSpec(p=inside[2], p_out=inside[2], g=inside[7], m=inside[3], v=inside[4])])
+    ctx.adam(table, mx.adam_hp(1e-2, 0.9, 0.999, 1e-8, 0.01))
+    assert took() == (256, 0, 0)
+    opt = mx.AdamW(1e-2, ctx=ctx)
+    for x, y, want in ((inside[2], inside[7], (256, 0, 0)), (plain[2], plain[7], (256, two, 1))):
+        opt.update_single("w", x, y, out=x)
+        assert took() == want
+    del places, inside, plain, p, g, v, q, h, m, w, a, b, x, y, table, other, opt, mem
+    import gc
+    gc.collect()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+
+
 def test_optimizer_state_comes_from_the_pool(mx, ctx, pool):
     rng = np.random.default_rng(12)
     n = 300_000
