@@ -128,13 +128,17 @@ constexpr Crowd kUpdateCrowd = update_crowd<PD, GD, G2, Math>();
 // the parameters stay in the 256 MB memory-side cache for whoever reads them next.  Microseconds plain and streaming, the
 // same list again and again: bf16 AdamW 48 M 166 and 175, 90 M 307 and 333, 128 M 440 and 476, 160 M 602 and 598; SGD 90 M 191 and
 // 211; float32 AdamW 48 M 205 and 221, 72 M 321 and 331, 80 M 375 and 366, RMSprop 72 M 222 and 234; several lists in turn: bf16 AdamW
-// 96 M 365 and 357, float32 64 M 315 and 314.  Plain SGD and a folded-in micro-batch gain nothing (64 M 65 and 66, 96 M 105 and
+// 96 M 365 and 357, float32 64 M 315 and 314.  In memory of one region streaming is ahead except for 16-bit parameters of up to 108 MB:
+// several lists in turn, mean over 8 - 50 M elements and three places, streaming takes 1.02 times as long for SGD, 1.01 for RMSprop, the
+// same for AdamW, on the same list 1.07, 1.05 and 1.04; 56 M AdamW 214 and 221, SGD 137 and 139, float32 SGD 18 M 73 and 65.
+// Plain SGD and a folded-in micro-batch gain nothing (64 M 65 and 66, 96 M 105 and
 // 99; 48 M 216 and 217).
 template <int PD, int G2, class Math>
 static bool stream_parameters(const Launch& L) {
   if (!L.in_place) return false;
-  if (!Math::kV || G2 >= 0 || !L.spread) return true;
-  return L.elems * Elem<PD>::kBytes >= (300ull << 20);
+  if (!Math::kV || G2 >= 0) return true;
+  const uint64_t bytes = L.elems * Elem<PD>::kBytes;
+  return L.spread ? bytes >= (300ull << 20) : PD == MXOPT_F32 || bytes >= (108ull << 20);
 }
 
 template <int PD, int GD, int OD, int G2, class Math>

@@ -340,3 +340,30 @@ def test_accumulation_of_16_bit_gradients_into_a_long_float32_buffer(mx, ctx, gd
     ctx.accumulate(ctx.table([mx.TensorSpec(g=g[1:1 + n], g_out=acc[1:1 + n])]), first=False)
     assert ctx.get_option("last_launch_lds") == reserved(per_cu)
     assert torch.equal(bits(torch, acc), bits(torch, want))
+
+
+@pytest.mark.parametrize("dtype,n,momentum,streams", [
+    ("bfloat16", (54 << 20) - 8, 0.9, 0), ("bfloat16", 54 << 20, 0.9, 1), ("float16", (54 << 20) - 8, 0.9, 0),
+    ("float32", 4099, 0.9, 1), ("bfloat16", 4099, None, 1)])
+def test_parameters_are_stored_streaming_or_not(mx, ctx, dtype, n, momentum, streams):
+    """16-bit parameters with moments stream from 108 MB, others always; with streaming switched off the results are the same."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(10)
+    base = torch.empty(n, device="cuda").normal_(0.0, 0.5, generator=gen).to(getattr(torch, dtype))
+    g = torch.empty(n, device="cuda").normal_(0.0, 1e-2, generator=gen).to(base.dtype)
+    outs = []
+    for hints in (1, 0):
+        p, v = base.clone(), torch.full((n,), 1e-3, device="cuda")
+        ctx.set_option("nontemporal", hints)
+        try:
+            if momentum is None:
+                ctx.sgd_plain(ctx.table([mx.TensorSpec(p=p, p_out=p, g=g)]), 0.3)
+            else:
+                ctx.sgd(ctx.table([mx.TensorSpec(p=p, p_out=p, g=g, v=v)]), mx.sgd_hp(0.1, momentum, 0.01))
+            assert ctx.get_option("last_launch_streams_parameters") == (streams if hints else 0)
+        finally:
+            ctx.set_option("nontemporal", 1)
+        outs.append((p, v))
+    assert torch.equal(bits(torch, outs[0][0]), bits(torch, outs[1][0])) and torch.equal(outs[0][1], outs[1][1])
+    assert not torch.equal(outs[0][0], base)
