@@ -7,12 +7,9 @@
 
 namespace mxopt {
 
-// See mxopt_tiles.h for what a tile gains.  Microseconds by chunks as they were before (parameters' stores plain, as many
-// workgroups as fit) and by tiles, plain memory of one region: AdamW of 596 M float32 elements 3,140 and 2,833, bf16 with float32
-// moments 2,453 and 2,224, of 1.72 G 7,010 and 6,315, with a float32 buffer and a bf16 micro-batch folded in 8,460 and 7,750; SGD
-// with momentum of 1.72 G float32 6,460 and 5,650; RMSprop of 596 M 2,183 and 1,958; plain SGD of 596 M bf16 651 and 585.  What did not help: the parameters stored row by row as they are computed
-// (2 % slower: reads and writes mix again), a barrier between the streams' stores, workgroups that stay and walk the tiles
-// (4 % slower), tiles that begin at a multiple of their size in memory (nothing on a whole parameter list).
+// See mxopt_tiles.h for what a tile gains, and update_tiles_per_cu for where.  What did not help: the parameters stored row by row
+// as they are computed (2 % slower: reads and writes mix again), a barrier between the streams' stores, workgroups that stay and
+// walk the tiles (4 % slower), tiles that begin at a multiple of their size in memory (nothing on a whole parameter list).
 //
 // U rows of 4,096 elements are in registers at once: 8 (the tile) while a row takes at most 12 of them a lane, else 4 in two
 // turns (8 would not fit the 128 that 1,024 lanes leave each).
@@ -103,17 +100,25 @@ __global__ __launch_bounds__(kTileThreads) void update_tile_kernel(const DevTens
   }
 }
 
-// Where tiles begin to pay, in whole tiles per compute unit.  Microseconds by chunks (streaming stores, two workgroups per compute
-// unit) and by tiles, memory of one region: float32 AdamW of 128 M elements (16 tiles) 622 and 631, 192 M (24) 948 and 936, 596 M 3,017 and
-// 2,874; SGD 128 M 438 and 443, 192 M 659 and 654, 596 M 2,146 and 1,988; bf16 AdamW 256 M (32) 951 and 997, 1.72 G 6,515 and
-// 6,301; plain bf16 SGD 256 M 264 and 271, 596 M (71) 592 and 578; a float32 buffer and a bf16 micro-batch folded into AdamW, 596 M
-// 2,754 and 2,688.  In memory of two regions the chunks stay ahead by 2 %.
+// Where tiles begin to pay in memory of one region, in whole tiles per compute unit.  Microseconds by chunks and by tiles, pairs
+// from several places in memory: float32 AdamW of 192 M elements (24 tiles) 946 and 942, 909 and 914, 596 M 2,850 and 2,828, 2,658 and
+// 2,691, 310 M in 4,000 tensors 1,451 and 1,428; SGD 192 M 642 and 647, 660 and 653, 1.5 G 5,544 and 5,239, 5,408 and 5,293, the 4,000 tensors
+// 1,077 and 1,052; plain SGD 192 M 398 and 399, the 4,000 648 and 609.  A float32 buffer and a bf16 micro-batch folded into bf16 AdamW 384 M
+// (48) 1,813 and 1,749, 1.72 G 7,885 and 7,729, 7,490 and 7,351, into plain SGD 512 M (64) 907 and 883; SGD and RMSprop of 16-bit
+// parameters 384 M 967 and 919, 958 and 908, 945 and 917, 950 and 909.  Never ahead: float32 RMSprop 192 M 644 and 668, 1.72 G
+// 5,554 and 5,661; bf16 AdamW 512 M 1,938 and 2,027, 1.72 G 6,316 and 6,328 (means of five); plain bf16 SGD 512 M 524 and 533, 1.72 G 1,713
+// and 1,730.
 template <int PD, int GD, int G2, class Math>
-constexpr uint32_t kUpdateTilesPerCu = (PD == MXOPT_F32 && GD == MXOPT_F32 && G2 <= MXOPT_F32) ? 24 : Math::kV ? 48 : 64;
+constexpr uint32_t update_tiles_per_cu() {
+  constexpr uint32_t kNoLength = 0xffffffffu - 1u;  // option "tiles" = 2 says 0xffffffff
+  if (PD == MXOPT_F32 && GD == MXOPT_F32 && G2 <= MXOPT_F32) return Math::kSquare && !Math::kM ? kNoLength : 24u;
+  if (G2 >= 0) return Math::kV ? 48u : 64u;
+  return Math::kV && !Math::kM ? 48u : kNoLength;
+}
 
 template <int PD, int GD, int G2, class Math>
 static bool launch_update_tiles(const Launch& L, const Math& math, const DevPrep& prep) {
-  if (L.ntiles == 0 || !L.in_place || L.tiles_per_cu < kUpdateTilesPerCu<PD, GD, G2, Math>) return false;
+  if (L.ntiles == 0 || !L.in_place || L.tiles_per_cu < update_tiles_per_cu<PD, GD, G2, Math>()) return false;
   constexpr int kG2Words = G2 < 0 ? 0 : Elem<(G2 < 0 ? MXOPT_F32 : G2)>::kBytes;
   constexpr int kWords = Elem<PD>::kBytes + Elem<GD>::kBytes + kG2Words + (Math::kM ? 4 : 0) + (Math::kV ? 4 : 0);
   constexpr int U = kWords <= 12 ? 8 : 4;

@@ -205,6 +205,39 @@ def test_launches_say_which_route_they_took(mx, ctx):
         ctx.set_option("last_launch_lanes", 1)
 
 
+@pytest.mark.parametrize("update,pd,gd,line", [
+    ("adam", "float32", "float32", 24), ("sgd_plain", "float32", "float32", 24), ("rmsprop", "float32", "float32", None),
+    ("adam", "bfloat16", "bfloat16", None), ("sgd", "bfloat16", "bfloat16", 48), ("rmsprop", "float16", "float16", 48),
+    ("sgd_plain", "bfloat16", "bfloat16", None), ("adam_with_pending", "bfloat16", "float32", 48),
+    ("sgd_plain_with_pending", "float16", "float32", 64), ("accumulate", "float32", "float32", 32)])
+def test_lists_on_both_sides_of_each_line(mx, ctx, update, pd, gd, line):
+    """Which kernel the default rule takes, in whole tiles per compute unit; None: chunks at every length."""
+    import torch
+    PD, GD, F = getattr(torch, pd), getattr(torch, gd), torch.float32
+    for tiles in (line - 1, line) if line else (100,):
+        n = TILE * ctx.get_option("num_cus") * tiles + 5
+        zeros = lambda dtype: torch.zeros(n, dtype=dtype, device="cuda")
+        p, g = zeros(PD), zeros(GD)
+        row = dict(g=g, g_out=p) if update == "accumulate" else dict(p=p, p_out=p, g=g)
+        if update.endswith("with_pending"):
+            row["g_out"] = zeros(PD)
+        if update.startswith("adam"):
+            row["m"] = zeros(F)
+        if update.startswith(("adam", "rmsprop")) or update == "sgd":
+            row["v"] = zeros(F)
+        table = ctx.table([mx.TensorSpec(**row)])
+        if update == "accumulate":
+            ctx.accumulate(table, first=False)
+        elif update.startswith("sgd_plain"):
+            getattr(ctx, update)(table, 0.3)
+        else:
+            hp = {"adam": mx.adam_hp(1e-2, 0.9, 0.999, 1e-8, 0.01), "sgd": mx.sgd_hp(0.1, 0.9, 0.01),
+                  "rmsprop": mx.rmsprop_hp(1e-2, 0.99, 1e-8, 0.0)}[update.split("_")[0]]
+            getattr(ctx, update)(table, hp, None)
+        assert ctx.get_option("last_launch_lanes") == (1024 if line and tiles >= line else 256)
+        table.close()
+
+
 def test_rule_takes_tiles_for_long_lists_only(mx, ctx):
     """The default rule on both sides of its line gives the results of either route."""
     import torch
