@@ -289,8 +289,8 @@ __global__ __launch_bounds__(kThreads) void accumulate_kernel(const DevTensor* _
   for (uint32_t c = blockIdx.x; c < nchunks; c += gridDim.x) Chunk::accumulate(locate(T, C, one, c), pr, threadIdx.x, FIRST);
 }
 
-// Later passes of float32 into float32 by tiles (mxopt_tiles.h): microseconds by chunks and by tiles 64 M elements 126 and 130, 256 M
-// 521 and 509, 596 M 1,205 and 1,145.
+// Later passes of float32 into float32 by tiles (mxopt_tiles.h), the sum in its own buffer: microseconds by chunks and by tiles, from
+// 32 whole tiles per compute unit, 256 M elements 521 and 510, 524 and 526, 596 M 1,197 and 1,178, 1.5 G 3,216 and 3,145; 64 M 126 and 130.
 __global__ __launch_bounds__(kTileThreads) void accumulate_tile_kernel(const DevTensor* __restrict__ T,
                                                                        const DevChunk* __restrict__ C, DevTensor one,
                                                                        uint32_t nchunks, const DevTile* __restrict__ tiles,
@@ -306,11 +306,10 @@ __global__ __launch_bounds__(kTileThreads) void accumulate_tile_kernel(const Dev
     return;
   }
   const uint64_t first = tv.t.head + (uint64_t)tv.tile.index * kChunk;
-  const void* A = tv.t.p != nullptr ? tv.t.p : tv.t.g_out;
   typename Piece<AD>::T a[U];
   typename Piece<GD>::T g[U];
   MXOPT_ROWS g[j] = load_piece<GD, true>(tv.t.g, first + j * kChunk, tid);
-  MXOPT_ROWS a[j] = load_piece<AD, true>(A, first + j * kChunk, tid);
+  MXOPT_ROWS a[j] = load_piece<AD, true>(tv.t.g_out, first + j * kChunk, tid);
   MXOPT_ROWS {
     pin(a[j]); pin(g[j]);
     float xa[4], xg[4];

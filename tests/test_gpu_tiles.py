@@ -64,10 +64,12 @@ def run_both(torch, mx, ctx, streams, layout, call):
         ctx.set_option("tiles", tiles)
         try:
             call(ctx.table(rows))
+            lanes = ctx.get_option("last_launch_lanes")
         finally:
             ctx.set_option("tiles", 1)
         results.append(own)
     torch.cuda.synchronize()
+    assert lanes == 1024 or "p" not in streams      # updates in place go by tiles where they are asked to
     for k in streams:
         a, b = bits(torch, results[0][k]), bits(torch, results[1][k])
         assert torch.equal(a, b), (k, int((a != b).sum()), int((a != b).nonzero()[0]))
@@ -292,14 +294,16 @@ def test_engines(mx, ctx, kind, defer, dtype):
 @pytest.mark.parametrize("layout", LAYOUTS)
 @pytest.mark.parametrize("ad,gd", list(itertools.product(["float32", "bfloat16", "float16"], repeat=2)))
 def test_accumulation(mx, ctx, ad, gd, layout):
-    """Later passes without the norm, in place and into another buffer; chunk by chunk they also give what torch gives (one
-    float32 addition, rounded to the buffer's type)."""
+    """Later passes without the norm give what torch gives (one float32 addition, rounded to the buffer's type), in place and
+    into another buffer, with tiles asked for and without.  Float32 into float32 in place is what tiles are taken for: chunks and
+    tiles over the same slabs there; the other passes go by chunks whatever the option says."""
     import torch
     gen = torch.Generator(device="cuda")
     gen.manual_seed(8)
     a, g = slab(torch, getattr(torch, ad), gen, 1e-2), slab(torch, getattr(torch, gd), gen, 1e-2)
     a[70000], g[70001] = float("inf"), -0.0
     run_both(torch, mx, ctx, dict(g_out=a, g=g), layout, lambda t: ctx.accumulate(t, first=False))
+    assert ctx.get_option("last_launch_lanes") == (1024 if ad == gd == "float32" else 256)
     out = a.clone()
     va, vg, vo = views(a, layout, 0), views(g, layout, 1), views(out, layout, 0)
     ctx.accumulate(ctx.table([mx.TensorSpec(g_out=o, g=x) for o, x in zip(vo, vg)]), first=False)
@@ -310,6 +314,7 @@ def test_accumulation(mx, ctx, ad, gd, layout):
         ctx.set_option("tiles", tiles)
         try:
             ctx.accumulate(ctx.table([mx.TensorSpec(p=x, g_out=o, g=y) for x, o, y in zip(va, views(dst, layout, 0), vg)]), first=False)
+            assert ctx.get_option("last_launch_lanes") == 256
         finally:
             ctx.set_option("tiles", 1)
     for p, q, o in zip(views(other[0], layout, 0), views(other[1], layout, 0), vo):
