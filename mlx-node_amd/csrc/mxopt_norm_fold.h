@@ -6,7 +6,9 @@ namespace mxopt {
 
 // Sum of n partial sums by the THREADS lanes of one workgroup, in an order that depends on n and THREADS alone; valid on thread
 // 0.  Bound by the latency of memory round trips, not by bytes (16,384 partials are 128 KB): every lane issues its next
-// kFoldLoads loads before it adds the first of them.  SHARED: other workgroups of the same launch have written them.
+// kFoldLoads loads before it adds the first of them.  Microseconds of the second pass with 8 loads and 256 lanes up to 2,048 partial
+// sums, and with 16 and 256 up to 4,096 (which adds 2,049 - 4,096 of them in another order): 100 1.7 and 1.9, 2,048 1.9 and 2.0, 2,049 2.3
+// and 2.0, 4,096 3.8 and 2.2, 8,192 4.4 and 3.9, 16,384 4.6 and 4.6.  SHARED: other workgroups of the same launch have written them.
 constexpr int kFoldLoads = 16;
 template <int THREADS, bool SHARED>
 __device__ __forceinline__ double sum_of_partials(const double* partials, uint32_t n) {

@@ -3,9 +3,10 @@
 // What bounds the passes that read and write is how often the memory has to turn round between the two, and how much of a
 // row it moves in between.  A chunk's workgroup writes 8 or 16 KB of one stream, then of the next, while its three or more
 // neighbours on the compute unit are in other phases.  A tile's workgroup is alone on its compute unit, loads its streams one
-// after the other and stores them one after the other, 64 or 128 KB each.  In memory of one region (where a plain allocation
-// lies) a long list of several streams reaches 5.8 - 6.1 TB/s by tiles, 5.5 - 5.8 by chunks with few workgroups per compute unit, 5.3 -
-// 5.5 with many; in memory of two regions all of them 6.1.
+// after the other and stores them one after the other: runs of 64 KB of a 16-bit stream and 128 KB of a float32 one where a lane's
+// registers hold the whole tile, half of that in two turns where they do not.  In memory of one region (where a plain allocation
+// lies) a long list of several streams reaches 5.8 - 6.1 TB/s by tiles, 5.6 - 6.1 by chunks with few workgroups per compute unit, 5.3 -
+// 5.6 with many; in memory of two regions 6.2 - 6.35 by tiles, 6.3 - 6.45 by chunks.
 // Bare streams, 4 read and 3 written, float32, 596 M elements: 256 lanes x 16 elements 3,150 us, 1,024 x 16 in the same
 // order 3,160, stream by stream 2,850; 512 x 32 3,050; 1,024 x 8 3,190.  Two 16-bit streams and two float32 ones: 2,490 by chunks,
 // 1,024 x 16 2,350, 1,024 x 32 2,140.

@@ -1,5 +1,5 @@
 // One chunk of the optimizer update, shared by the kernels that walk chunk by chunk (mxopt_kernels.hip) and tile by
-// tile (mxopt_tile_kernels.hip).
+// tile (mxopt_update_tile.h).
 #pragma once
 #include "mxopt_kernels_common.h"
 

@@ -142,7 +142,7 @@ def test_widening_transform(mx, ctx, n, dtype):
 @pytest.mark.parametrize("which", ["norm", "sum", "list"])
 def test_norm_folded_by_the_last_workgroup(mx, ctx, chunks, which):
     """Up to 64 partial sums are folded by the workgroup that stores the last one, more by a second kernel: the same call
-    again and again (the count of arrivals starts from zero each time), in two dtype groups, next to a call that fails
+    again and again (the count of arrivals goes on from call to call), in two dtype groups, next to a call that fails
     behind its first launch.  Elements are powers of two, so the sums are exact in any order."""
     import torch
     n = (chunks - 1) * CHUNK + 5
