@@ -131,13 +131,15 @@ constexpr Crowd kUpdateCrowd = update_crowd<PD, GD, G2, Math>();
 // 96 M 365 and 357, float32 64 M 315 and 314.  In memory of one region streaming is ahead except for 16-bit parameters of up to 108 MB:
 // several lists in turn, mean over 8 - 50 M elements and three places, streaming takes 1.02 times as long for SGD, 1.01 for RMSprop, the
 // same for AdamW, on the same list 1.07, 1.05 and 1.04; 56 M AdamW 214 and 221, SGD 137 and 139, float32 SGD 18 M 73 and 65.
-// Plain SGD and a folded-in micro-batch gain nothing (64 M 65 and 66, 96 M 105 and
-// 99; 48 M 216 and 217).
+// Launches of less than 24 MB of parameters stream, as they may be pieces of a longer list (22 calls over 31 M elements, plain 174.6,
+// streaming 171.7), and so do plain SGD and updates with a micro-batch folded in, which gain nothing by plain stores (96 M 105 and 99;
+// 48 M 216 and 217).
 template <int PD, int G2, class Math>
 static bool stream_parameters(const Launch& L) {
   if (!L.in_place) return false;
   if (!Math::kV || G2 >= 0) return true;
   const uint64_t bytes = L.elems * Elem<PD>::kBytes;
+  if (bytes < (24ull << 20)) return true;
   return L.spread ? bytes >= (300ull << 20) : PD == MXOPT_F32 || bytes >= (108ull << 20);
 }
 

@@ -105,15 +105,16 @@ __global__ __launch_bounds__(kTileThreads) void update_tile_kernel(const DevTens
 // 2,691, 310 M in 4,000 tensors 1,451 and 1,428; SGD 192 M 642 and 647, 660 and 653, 1.5 G 5,544 and 5,239, 5,408 and 5,293, the 4,000 tensors
 // 1,077 and 1,052; plain SGD 192 M 398 and 399, the 4,000 648 and 609.  A float32 buffer and a bf16 micro-batch folded into bf16 AdamW 384 M
 // (48) 1,813 and 1,749, 1.72 G 7,885 and 7,729, 7,490 and 7,351, into plain SGD 512 M (64) 907 and 883; SGD and RMSprop of 16-bit
-// parameters 384 M 967 and 919, 958 and 908, 945 and 917, 950 and 909.  Never ahead: float32 RMSprop 192 M 644 and 668, 1.72 G
-// 5,554 and 5,661; bf16 AdamW 512 M 1,938 and 2,027, 1.72 G 6,316 and 6,328 (means of five); plain bf16 SGD 512 M 524 and 533, 1.72 G 1,713
-// and 1,730.
+// parameters 384 M 967 and 919, 958 and 908, 945 and 917, 950 and 909.  bf16 AdamW 512 M 1,938 and 2,027, 1 G
+// (127) 4,046 and 4,029, 3,739 and 3,833, 1.72 G (205) 6,316 and 6,328 (means of five), behind its norm with several lists in turn
+// 7,028 and 6,868; plain bf16 SGD 512 M 524 and 533, 596 M (71) 587 and 585, behind its norm 815 and 801.  Never ahead: float32 RMSprop
+// 192 M 644 and 668, 1.72 G 5,554 and 5,661.
 template <int PD, int GD, int G2, class Math>
 constexpr uint32_t update_tiles_per_cu() {
   constexpr uint32_t kNoLength = 0xffffffffu - 1u;  // option "tiles" = 2 says 0xffffffff
   if (PD == MXOPT_F32 && GD == MXOPT_F32 && G2 <= MXOPT_F32) return Math::kSquare && !Math::kM ? kNoLength : 24u;
-  if (G2 >= 0) return Math::kV ? 48u : 64u;
-  return Math::kV && !Math::kM ? 48u : kNoLength;
+  if (!Math::kV) return 64u;
+  return Math::kM && G2 < 0 ? 192u : 48u;
 }
 
 template <int PD, int GD, int G2, class Math>

@@ -209,8 +209,8 @@ def test_launches_say_which_route_they_took(mx, ctx):
 
 @pytest.mark.parametrize("update,pd,gd,line", [
     ("adam", "float32", "float32", 24), ("sgd_plain", "float32", "float32", 24), ("rmsprop", "float32", "float32", None),
-    ("adam", "bfloat16", "bfloat16", None), ("sgd", "bfloat16", "bfloat16", 48), ("rmsprop", "float16", "float16", 48),
-    ("sgd_plain", "bfloat16", "bfloat16", None), ("adam_with_pending", "bfloat16", "float32", 48),
+    ("adam", "bfloat16", "bfloat16", 192), ("sgd", "bfloat16", "bfloat16", 48), ("rmsprop", "float16", "float16", 48),
+    ("sgd_plain", "bfloat16", "bfloat16", 64), ("adam_with_pending", "bfloat16", "float32", 48),
     ("sgd_plain_with_pending", "float16", "float32", 64), ("accumulate", "float32", "float32", 32)])
 def test_lists_on_both_sides_of_each_line(mx, ctx, update, pd, gd, line):
     """Which kernel the default rule takes, in whole tiles per compute unit; None: chunks at every length."""
@@ -381,10 +381,11 @@ def test_accumulation_of_16_bit_gradients_into_a_long_float32_buffer(mx, ctx, gd
 
 
 @pytest.mark.parametrize("dtype,n,momentum,streams", [
+    ("bfloat16", (12 << 20) - 8, 0.9, 1), ("bfloat16", 12 << 20, 0.9, 0),
     ("bfloat16", (54 << 20) - 8, 0.9, 0), ("bfloat16", 54 << 20, 0.9, 1), ("float16", (54 << 20) - 8, 0.9, 0),
     ("float32", 4099, 0.9, 1), ("bfloat16", 4099, None, 1)])
 def test_parameters_are_stored_streaming_or_not(mx, ctx, dtype, n, momentum, streams):
-    """16-bit parameters with moments stream from 108 MB, others always; with streaming switched off the results are the same."""
+    """16-bit parameters with moments of 24 - 108 MB are stored plain, others stream; with streaming switched off the results are the same."""
     import torch
     gen = torch.Generator(device="cuda")
     gen.manual_seed(10)
