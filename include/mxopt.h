@@ -76,17 +76,19 @@ int mxopt_synchronize(mxopt_ctx* ctx);
  * "persistent" (0: one workgroup per chunk for the update kernels), "persistent_accumulate" (1: the
  * persistent grid also for accumulation passes after the first that take no norm), "nontemporal" /
  * "nontemporal_reduce" (both 1 by default: streaming-hint memory instructions in the read-write / read-only
- * kernels -- on every load that fetches whole 32-byte sectors, and on stores to lines the kernel has read;
- * 0 = plain loads and stores; the list kernels of deferred accumulation always stream),
+ * kernels -- on every load that fetches whole 32-byte sectors, and on stores to lines the kernel has read, but for
+ * parameters that the memory-side cache keeps; 0 = plain loads and stores; the list kernels of deferred accumulation
+ * always stream),
  * "pipelined_norm" (the plain norm of a 16-bit stream: 0 = the general reduction kernel always; 2 (default)
  * or 4 = a kernel that takes that many chunks per trip, for tables whose chunks are under 90 % full on
  * average, i.e. many small tensors; 1 = that kernel, two chunks per trip, for every table),
  * "tiles" (kernels that take 32,768 consecutive elements of a tensor per workgroup: 0 = never, 1 (default) = where a
- * launch is long enough for them to pay, 2 = wherever they can; same results; "persistent" = 1 or "nontemporal" = 0 switch
- * them off whatever it says).  To be read only: "num_cus", and of the latest launch over tensors "last_launch_lanes" (of
- * each workgroup: 1,024 by tiles, else 256), "last_launch_workgroups", "last_launch_lds" (bytes of LDS that a workgroup
- * reserves, so that fewer of them share a compute unit; 0 = as many as fit), "last_launch_streams_parameters"
- * (an update: the stores of the parameters carry the streaming hint). */
+ * launch is long enough for them to pay and its buffers do not alternate between memory regions, 2 = wherever they
+ * can; same results; "persistent" = 1 or "nontemporal" = 0 switch them off whatever it says).
+ * To be read only: "num_cus", and of the latest launch over tensors "last_launch_lanes" (of each workgroup: 1,024 by
+ * tiles, else 256), "last_launch_workgroups", "last_launch_lds" (bytes of LDS that a workgroup reserves, so that fewer of
+ * them share a compute unit; 0 = as many as fit), "last_launch_streams_parameters" (an update: the stores of the
+ * parameters carry the streaming hint). */
 int mxopt_set_option(mxopt_ctx* ctx, const char* name, int64_t value);
 int mxopt_get_option(const mxopt_ctx* ctx, const char* name, int64_t* value);
 

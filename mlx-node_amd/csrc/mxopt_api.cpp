@@ -195,7 +195,9 @@ Launch make_launch(const mxopt_ctx* ctx, const mxopt_table* t, const Group& g, b
 // Offers the tiled kernels a cut of `elems` elements into `ntiles` tiles, `whole` of them whole, where two thirds of the
 // elements lie in whole ones: a mixed tile occupies a compute unit for a few short chunks.  Microseconds by tiles and by chunks (two
 // workgroups per compute unit): 10,000 tensors of 64 - 65,536 elements, 35 % of them in whole tiles, bf16 AdamW 391 and 367,
-// float32 511 and 488, SGD 366 and 356; 2,000 of 1,000 - 200,000, 69 %, float32 AdamW 375 and 391, SGD 272 and 292.
+// float32 511 and 488, SGD 366 and 356; 2,000 of 1,000 - 200,000, 69 %, float32 AdamW 375 and 391, SGD 272 and 292; by chunks as they are now 10,000 of 8,000 - 120,000, 61 %, float32 AdamW 2,024 and
+// 2,080, SGD 1,381 and 1,276, plain SGD 811 and 865; 7,000 of 16,000 - 120,000, 66 %, 1,803 and 1,829, 1,229 and 1,244, 710 and 761, a
+// micro-batch folded in 1,645 and 1,572; 4,000 of 20,000 - 200,000, 78 %, 1,428 and 1,451, 1,052 and 1,077, 609 and 648, 1,379 and 1,377.
 // Not in memory of several regions, where the chunks are ahead: float32 AdamW of 596 M 2,647 and 2,584, SGD 1,892 and 1,858, bf16
 // AdamW of 1.72 G 5,985 and 5,941, plain SGD 1,682 and 1,642.
 static void offer_tiles(const mxopt_ctx* ctx, Launch& L, const DevTile* tiles, uint32_t ntiles, uint32_t whole, uint64_t elems) {

@@ -102,7 +102,9 @@ __device__ __forceinline__ void chunks_of_tile(const DevTensor* __restrict__ T, 
 #define MXOPT_ROWS _Pragma("unroll") for (int j = 0; j < U; ++j)
 
 // Dynamic LDS of every tiled launch, unused: more than half a compute unit's 160 KB, so that one workgroup has it to itself.
-// Plain SGD on 596 M bf16 elements: 586 us with it, 659 without (AdamW's registers have the same effect).
+// Plain SGD on 596 M bf16 elements: 586 us with it, 659 without (AdamW's registers have the same effect).  Kernels of another stream
+// find less room meanwhile: ten float32 AdamW updates of 256 M and matrix products of 8,192 on another stream, 12.4 and 8.0 ms alone,
+// take 20.4 ms together, 19.4 with the chunk kernel as it was without limits (13.4 alone); with products of 4,096 18.7 and 21.3.
 constexpr unsigned kOnePerCu = 84 * 1024;
 
 }  // namespace mxopt
