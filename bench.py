@@ -43,7 +43,7 @@ TRAFFIC_PROFILE = "profiles/hbm_traffic_pmc_cfg5_and_copy.txt"
 TRAFFIC_KERNEL_SOURCES = ["mxopt_kernels.hip", "mxopt_kernels_common.h", "mxopt_device.h", "mxopt_list_kernels.h",
                           "mxopt_list_kernels.hip", "mxopt_update_chunk.h", "mxopt_update_tile.h", "mxopt_tiles.h",
                           "mxopt_reduce_kernels.hip"]
-MEASURED_TRAFFIC_B_PER_ELEM = {("cfg5", 1): 25.88, ("cfg5-deferred", 1): 27.89}
+MEASURED_TRAFFIC_B_PER_ELEM = {("cfg5", 1): 25.91, ("cfg5-deferred", 1): 27.89}
 PROBE_PROFILE = "profiles/probe_streams_pool_and_plain.txt"
 OTHER_CONFIGS = ["cfg1", "cfg2", "cfg3-sgd", "cfg3-rmsprop", "cfg4", "cfg4-flat"]
 # steps each configuration states for itself
