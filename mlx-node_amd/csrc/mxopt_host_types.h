@@ -78,7 +78,6 @@ struct StreamScales {
   const float* s[MXOPT_MAX_PENDING + 1];
 };
 
-// Tensors of one dtype combination: a contiguous run of chunk entries, one launch.
 // The shape of a launch, for mxopt_get_option.
 struct LaunchNote {
   uint32_t lanes = 0, workgroups = 0;  // lanes of each workgroup
@@ -86,6 +85,7 @@ struct LaunchNote {
   uint32_t streams_parameters = 0;     // updates: the parameters' stores stream
 };
 
+// Tensors of one dtype combination: a contiguous run of chunk entries, one launch.
 struct Group {
   int pd, gd, pod, god;
   uint32_t chunk_begin, nchunks;
